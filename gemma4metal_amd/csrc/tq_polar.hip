@@ -511,133 +511,337 @@ struct P7EncParams {
   uint32_t* qjl;     // [.][4]
 };
 
-// One wave per vector: lane l holds y[2l], y[2l+1]; level k pairs come from
-// lanes 2j, 2j+1 of level k-1.  Grid-stride over vectors.
-__global__ __launch_bounds__(256) void polar7_encode_kernel(P7EncParams p) {
-#pragma clang fp contract(off)
-  __shared__ float cb[20];
-  __shared__ float2 cs[20];
-  __shared__ float xs[4][128];
-  __shared__ float rs[4][128];
-  if (threadIdx.x < 20) {
-    cb[threadIdx.x] = p.cb[threadIdx.x];
-    cs[threadIdx.x] = make_float2(p.cs[2 * threadIdx.x], p.cs[2 * threadIdx.x + 1]);
+constexpr int kEncThreads = 512;
+// Row strides in LDS, 16 bytes past a multiple of the 256-byte bank period:
+// a 16-lane phase of row reads covers every bank once.
+constexpr int kEncStr = 132;     // rows of 128 floats
+constexpr int kEncHalfStr = 68;  // rows of 64 floats
+
+// Columns 64 half .. +63 of a 128 x 128 matrix into registers, 4 float4 a
+// thread, and from there into LDS rows.
+__device__ __forceinline__ void load_half(const float* m, int half, float4 (&r)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = threadIdx.x + kEncThreads * i;
+    r[i] = reinterpret_cast<const float4*>(m)[(e >> 4) * 32 + 16 * half + (e & 15)];
   }
-  __syncthreads();
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + wave; row < p.n;
-       row += static_cast<int64_t>(gridDim.x) * 4) {
-    int64_t orow = row;
-    if (p.positions) {
+}
+__device__ __forceinline__ void store_half(float* ms, const float4 (&r)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int e = threadIdx.x + kEncThreads * i;
+    *reinterpret_cast<float4*>(ms + (e >> 4) * kEncHalfStr + 4 * (e & 15)) = r[i];
+  }
+}
+
+// Adds 64 terms, in order, product and sum rounded separately (the encoder's
+// definition), to the sums of TV vectors and TI matrix rows a thread:
+// acc[j][k] += sum_d xs[v0 + j][d] * ms[i0 + IG k][d].  Every 16-byte LDS read
+// of a row serves TV or TI sums, so the VALU binds (2 instructions a term).
+template <int TV, int TI>
+__device__ __forceinline__ void exact_dots(const float* xs, const float* ms, int v0, int i0, float (&acc)[TV][TI]) {
+#pragma clang fp contract(off)
+  constexpr int IG = 128 / TI;
+#pragma unroll 2
+  for (int d = 0; d < 64; d += 4) {
+    float4 x[TV], m[TI];
+#pragma unroll
+    for (int j = 0; j < TV; ++j) x[j] = *reinterpret_cast<const float4*>(xs + (v0 + j) * kEncStr + d);
+#pragma unroll
+    for (int k = 0; k < TI; ++k) m[k] = *reinterpret_cast<const float4*>(ms + (i0 + IG * k) * kEncHalfStr + d);
+#pragma unroll
+    for (int j = 0; j < TV; ++j)
+#pragma unroll
+      for (int k = 0; k < TI; ++k) {
+        float a = acc[j][k];
+        a = a + x[j].x * m[k].x;
+        a = a + x[j].y * m[k].y;
+        a = a + x[j].z * m[k].z;
+        a = a + x[j].w * m[k].w;
+        acc[j][k] = a;
+      }
+  }
+}
+
+// The index of angle j of level l (1 .. 7) goes into word p7_word(l, j) of the
+// vector at bit p7_bit(l, j) (the layout of tq_c_api.h).
+__device__ __forceinline__ constexpr int p7_word(int l, int j) {
+  return l == 1 ? j >> 3 : l == 2 ? 8 + (j >> 4) : l == 3 ? 10 : 11;
+}
+__device__ __forceinline__ constexpr int p7_bit(int l, int j) {
+  return l == 1 ? 4 * (j & 7) : l == 2 ? 2 * (j & 15) : l <= 4 ? 2 * j : l == 5 ? 16 + 2 * j : l == 6 ? 24 + 2 * j : 28;
+}
+
+// Bound of |sum in another order - exact sum| over |S_i| |r| (Cauchy-Schwarz
+// over the 128 terms): each of the two sums is off by at most 129 roundings
+// of 2^-24 per term.  Twice that, for the rounding of the norms.
+constexpr float kSketchSlack = 4.0f * 129.0f * 0x1p-24f;
+
+// V vectors per workgroup of eight waves, PPL level-1 pairs a lane.
+//  1. y = P x with the thread tile of exact_dots, P staged in two halves of 64
+//     columns (the loads of the second run under the first's sums); y goes
+//     over x.
+//  2. 64 / PPL lanes encode one vector: the levels inside a lane's 2 PPL
+//     values in registers, the upper ones across the lanes.  (A lane per pair
+//     evaluates every upper level on all 64 lanes: 448 angles a vector
+//     instead of 144 at PPL 8.)  Indices are ORed into the vector's words in
+//     LDS.
+//  3. The residual goes over y, S over P, and the sketch S r runs on the fp32
+//     matrix cores.  Only its signs are stored: a sum within the rounding
+//     bound of zero (about 3e-4 |r|: one bit in several thousand) is
+//     recomputed in the defined order, so the bits are those of the exact
+//     sums at an eighth of their VALU cost.
+// What bounds it: the VALU of step 1, 2 x 16,384 lane instructions a vector in
+// the only order the definition allows (54 us at 65,536 vectors), and of step
+// 2 (~26 us).  Half-staged matrices take 71 KB at V = 64, so two workgroups
+// share a CU and one's matrix-core and memory phases run under the other's
+// VALU phases.  A wave per vector with P and S rows read from L2 at a 1 KB
+// lane stride took 901 us there; V = 128 with whole matrices in LDS, one
+// workgroup a CU, 112 us; this form 105 us.
+template <int V, int TV, int TI, int PPL>
+__global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams p) {
+#pragma clang fp contract(off)
+  constexpr int LPV = 64 / PPL;  // lanes a vector
+  static_assert((V / TV) * (128 / TI) == kEncThreads && V % 16 == 0 && V * LPV <= kEncThreads, "thread tiles");
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  __shared__ __align__(16) float ms[128 * kEncHalfStr];  // a half of P, then of S
+  __shared__ __align__(16) float xs[V * kEncStr];        // x, then y, then the residual
+  __shared__ uint32_t words[V * kP7Words];
+  __shared__ float2 cs[20];
+  __shared__ float rn[V];        // |r|, or infinity where the bound does not hold
+  __shared__ float sn[128];      // |S_i|, likewise
+  __shared__ int64_t orow_s[V];  // output row, -1: none
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * V;
+  float4 mreg[4];
+  if (p.P) load_half(p.P, 0, mreg);
+  // uniform: scalar registers
+  float cb1[16], cb2[4];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) cb1[i] = p.cb[i];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cb2[i] = p.cb[16 + i];
+  if (tid < 20) cs[tid] = make_float2(p.cs[2 * tid], p.cs[2 * tid + 1]);
+  if (tid < V) {
+    const int64_t row = row0 + tid;
+    int64_t orow = row < p.n ? row : -1;
+    if (p.positions && row < p.n) {
       const int64_t bh = row / p.n_new;
       const int t = static_cast<int>(row - bh * p.n_new);
       const int64_t pos = static_cast<int64_t>(p.positions[bh / p.Hkv]) + t;
-      if (pos < 0 || pos >= p.cap) continue;  // wave-uniform
-      orow = bh * p.cap + pos;
+      orow = (pos < 0 || pos >= p.cap) ? -1 : bh * p.cap + pos;
     }
-    const float2 xv = reinterpret_cast<const float2*>(p.x + row * 128)[lane];
-    float y0 = xv.x, y1 = xv.y;
-    if (p.P) {
-      xs[wave][2 * lane] = xv.x;
-      xs[wave][2 * lane + 1] = xv.y;
-      wave_lds_sync();
-      const float* pa = p.P + (2 * lane) * 128;
-      const float* pb = pa + 128;
-      float acc0 = 0.0f, acc1 = 0.0f;
-      for (int d = 0; d < 128; d += 4) {
-        const float4 a4 = *reinterpret_cast<const float4*>(pa + d);
-        const float4 b4 = *reinterpret_cast<const float4*>(pb + d);
-        const float x0 = xs[wave][d], x1 = xs[wave][d + 1], x2 = xs[wave][d + 2], x3 = xs[wave][d + 3];
-        acc0 = acc0 + x0 * a4.x; acc0 = acc0 + x1 * a4.y; acc0 = acc0 + x2 * a4.z; acc0 = acc0 + x3 * a4.w;
-        acc1 = acc1 + x0 * b4.x; acc1 = acc1 + x1 * b4.y; acc1 = acc1 + x2 * b4.z; acc1 = acc1 + x3 * b4.w;
-      }
-      y0 = acc0;
-      y1 = acc1;
-    }
-    // ---- encode: level 1 (4-bit, wrapped to [0, 2pi)), levels 2..7 (2-bit)
-    int idx[7];
-    float r;
-    {
-      float th = atan2_det(y1, y0);
-      if (th < 0.0f) th = th + kTwoPi;
-      idx[0] = nearest_idx(th, cb, 16);
-      r = pair_radius(y0, y1);
-    }
-#pragma unroll
-    for (int lv = 1; lv < 7; ++lv) {
-      const float a = __shfl(r, (2 * lane) & 63, 64);
-      const float b = __shfl(r, (2 * lane + 1) & 63, 64);
-      idx[lv] = nearest_idx(atan2_det(b, a), cb + 16, 4);
-      r = pair_radius(a, b);
-    }
-    const float R = __shfl(r, 0, 64);
-    const __half R16 = __float2half_rn(R);
-    // ---- decode top-down (the stored bits): child = parent * cos|sin
-    float v = __half2float(R16);
-#pragma unroll
-    for (int lv = 6; lv >= 1; --lv) {
-      const float pv = __shfl(v, lane >> 1, 64);
-      const int pi = __shfl(idx[lv], lane >> 1, 64);
-      const float2 c = cs[16 + pi];
-      v = (lane & 1) ? pv * c.y : pv * c.x;
-    }
-    const float2 c1 = cs[idx[0]];
-    const float yh0 = v * c1.x, yh1 = v * c1.y;
-    const float r0 = y0 - yh0, r1 = y1 - yh1;
-    float nrm = r0 * r0;
-    const float q1 = r1 * r1;
-    nrm = nrm + q1;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) nrm = nrm + shfl_xor_f(nrm, off);
-    const __half rn16 = __float2half_rn(sqrtf(nrm));
-    // ---- QJL sketch: rows lane and lane + 64 of S r
-    rs[wave][2 * lane] = r0;
-    rs[wave][2 * lane + 1] = r1;
-    wave_lds_sync();
-    const float* sa = p.S + lane * 128;
-    const float* sb = sa + 64 * 128;
-    float ka = 0.0f, kb = 0.0f;
-    for (int d = 0; d < 128; d += 4) {
-      const float4 a4 = *reinterpret_cast<const float4*>(sa + d);
-      const float4 b4 = *reinterpret_cast<const float4*>(sb + d);
-      const float e0 = rs[wave][d], e1 = rs[wave][d + 1], e2 = rs[wave][d + 2], e3 = rs[wave][d + 3];
-      ka = ka + e0 * a4.x; ka = ka + e1 * a4.y; ka = ka + e2 * a4.z; ka = ka + e3 * a4.w;
-      kb = kb + e0 * b4.x; kb = kb + e1 * b4.y; kb = kb + e2 * b4.z; kb = kb + e3 * b4.w;
-    }
-    const uint64_t ba = __ballot(ka >= 0.0f);
-    const uint64_t bb = __ballot(kb >= 0.0f);
-    // ---- pack: lanes 0-7 level-1 words, 8-9 level-2, 10 level 3, 11 levels 4-7
-    uint32_t wa = 0, wb = 0, wc = 0, wd = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      wa |= (static_cast<uint32_t>(__shfl(idx[0], (8 * lane + i) & 63, 64)) & 0xFu) << (4 * i);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      wb |= (static_cast<uint32_t>(__shfl(idx[1], (16 * (lane - 8) + i) & 63, 64)) & 0x3u) << (2 * i);
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      wc |= (static_cast<uint32_t>(__builtin_amdgcn_readlane(idx[2], i)) & 0x3u) << (2 * i);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      wd |= (static_cast<uint32_t>(__builtin_amdgcn_readlane(idx[3], i)) & 0x3u) << (2 * i);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      wd |= (static_cast<uint32_t>(__builtin_amdgcn_readlane(idx[4], i)) & 0x3u) << (16 + 2 * i);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      wd |= (static_cast<uint32_t>(__builtin_amdgcn_readlane(idx[5], i)) & 0x3u) << (24 + 2 * i);
-    wd |= (static_cast<uint32_t>(__builtin_amdgcn_readlane(idx[6], 0)) & 0x3u) << 28;
-    const uint32_t w = lane < 8 ? wa : (lane < 10 ? wb : (lane == 10 ? wc : wd));
-    if (lane < kP7Words) p.angles[orow * kP7Words + lane] = w;
-    if (lane < 4) {
-      const uint64_t bits = lane < 2 ? ba : bb;
-      p.qjl[orow * 4 + lane] = static_cast<uint32_t>(bits >> (32 * (lane & 1)));
-    }
-    if (lane == 0)
-      p.norms[orow] = static_cast<uint32_t>(__half_as_ushort(R16)) |
-                      (static_cast<uint32_t>(__half_as_ushort(rn16)) << 16);
+    orow_s[tid] = orow;
   }
+  for (int i = tid; i < V * kP7Words; i += kEncThreads) words[i] = 0;
+#pragma unroll
+  for (int e = tid; e < V * 32; e += kEncThreads) {
+    const int64_t row = min(row0 + (e >> 5), p.n - 1);  // rows past the end: a copy, not stored
+    *reinterpret_cast<float4*>(xs + (e >> 5) * kEncStr + 4 * (e & 31)) =
+        reinterpret_cast<const float4*>(p.x + row * 128)[e & 31];
+  }
+  if (p.P) {
+    constexpr int IG = 128 / TI;
+    const int i0 = tid % IG, v0 = (tid / IG) * TV;
+    float acc[TV][TI];
+#pragma unroll
+    for (int j = 0; j < TV; ++j)
+#pragma unroll
+      for (int k = 0; k < TI; ++k) acc[j][k] = 0.0f;
+    store_half(ms, mreg);
+    load_half(p.P, 1, mreg);
+    __syncthreads();
+    exact_dots<TV, TI>(xs, ms, v0, i0, acc);
+    __syncthreads();  // every wave is done with the first half
+    store_half(ms, mreg);
+    __syncthreads();
+    exact_dots<TV, TI>(xs + 64, ms, v0, i0, acc);
+    __syncthreads();  // every wave is done with x and P
+#pragma unroll
+    for (int j = 0; j < TV; ++j)
+#pragma unroll
+      for (int k = 0; k < TI; ++k) xs[(v0 + j) * kEncStr + i0 + IG * k] = acc[j][k];
+  }
+  load_half(p.S, 0, mreg);
+  __syncthreads();
+
+  // ---- encode: lane b of a vector has pairs PPL b .. PPL b + PPL - 1
+  if (tid < V * LPV) {
+    constexpr int LIN = __builtin_ctz(2 * PPL);  // levels inside a lane
+    const int b = tid % LPV, v = tid / LPV;
+    uint32_t* wv = words + v * kP7Words;
+    float y[2 * PPL], r[2 * PPL];
+#pragma unroll
+    for (int j = 0; j < 2 * PPL; j += 4) {
+      const float4 t = *reinterpret_cast<const float4*>(xs + v * kEncStr + 2 * PPL * b + j);
+      y[j] = t.x; y[j + 1] = t.y; y[j + 2] = t.z; y[j + 3] = t.w;
+    }
+#pragma unroll
+    for (int j = 0; j < 2 * PPL; ++j) r[j] = y[j];
+    int ki[LIN][PPL];
+#pragma unroll
+    for (int l = 1; l <= LIN; ++l) {
+      const int cnt = (2 * PPL) >> l;
+      uint32_t w = 0;
+#pragma unroll
+      for (int j = 0; j < cnt; ++j) {
+        float th = atan2_det(r[2 * j + 1], r[2 * j]);
+        if (l == 1 && th < 0.0f) th = th + kTwoPi;
+        ki[l - 1][j] = l == 1 ? nearest_idx(th, cb1, 16) : nearest_idx(th, cb2, 4);
+        r[j] = pair_radius(r[2 * j], r[2 * j + 1]);
+        w |= static_cast<uint32_t>(ki[l - 1][j]) << ((l == 1 ? 4 : 2) * j);
+      }
+      // a lane's indices of one level are adjacent bits of one word
+      atomicOr(&wv[p7_word(l, cnt * b)], w << p7_bit(l, cnt * b));
+    }
+    // upper levels: every lane below a pair computes it
+    float rad = r[0];
+    int ku[7 - LIN];
+#pragma unroll
+    for (int l = LIN + 1; l <= 7; ++l) {
+      const int sh = l - LIN - 1;
+      const float other = __shfl_xor(rad, 1 << sh, 64);
+      const bool second = (b >> sh) & 1;
+      const float a = second ? other : rad, c = second ? rad : other;
+      ku[sh] = nearest_idx(atan2_det(c, a), cb2, 4);
+      rad = pair_radius(a, c);
+      const int j = b >> (sh + 1);
+      if ((b & ((2 << sh) - 1)) == 0) atomicOr(&wv[p7_word(l, j)], static_cast<uint32_t>(ku[sh]) << p7_bit(l, j));
+    }
+    const __half R16 = __float2half_rn(rad);
+    // ---- decode top-down (the stored bits): child = parent * cos|sin
+    r[0] = __half2float(R16);
+#pragma unroll
+    for (int l = 7; l > LIN; --l) {
+      const float2 c = cs[16 + ku[l - LIN - 1]];
+      r[0] = ((b >> (l - LIN - 1)) & 1) ? r[0] * c.y : r[0] * c.x;
+    }
+#pragma unroll
+    for (int l = LIN; l >= 1; --l) {
+      const int cnt = (2 * PPL) >> l;
+#pragma unroll
+      for (int j = cnt - 1; j >= 0; --j) {
+        const float2 c = cs[(l == 1 ? 0 : 16) + ki[l - 1][j]];
+        const float t = r[j];
+        r[2 * j] = t * c.x;
+        r[2 * j + 1] = t * c.y;
+      }
+    }
+    float nr[PPL];
+#pragma unroll
+    for (int j = 0; j < PPL; ++j) {
+      y[2 * j] = y[2 * j] - r[2 * j];
+      y[2 * j + 1] = y[2 * j + 1] - r[2 * j + 1];
+      const float q0 = y[2 * j] * y[2 * j], q1 = y[2 * j + 1] * y[2 * j + 1];
+      nr[j] = q0 + q1;
+    }
+    // |r|^2 as a balanced tree over the 64 pairs
+#pragma unroll
+    for (int st = 1; st < PPL; st *= 2)
+#pragma unroll
+      for (int j = 0; j < PPL; j += 2 * st) nr[j] = nr[j] + nr[j + st];
+    float nrm = nr[0];
+#pragma unroll
+    for (int l = 1; l < LPV; l *= 2) nrm = nrm + __shfl_xor(nrm, l, 64);
+    const float rnorm = sqrtf(nrm);
+    const __half rn16 = __float2half_rn(rnorm);
+#pragma unroll
+    for (int j = 0; j < 2 * PPL; j += 4)
+      *reinterpret_cast<float4*>(xs + v * kEncStr + 2 * PPL * b + j) = make_float4(y[j], y[j + 1], y[j + 2], y[j + 3]);
+    if (b == 0) {
+      // the relative bound needs squares that neither vanish nor overflow
+      rn[v] = (nrm > 1e-25f && nrm < 1e30f) ? rnorm : INFINITY;
+      const int64_t orow = orow_s[v];
+      if (orow >= 0)
+        p.norms[orow] = static_cast<uint32_t>(__half_as_ushort(R16)) |
+                        (static_cast<uint32_t>(__half_as_ushort(rn16)) << 16);
+    }
+  }
+  store_half(ms, mreg);  // P is no longer read (barrier before the encoding)
+  load_half(p.S, 1, mreg);
+  __syncthreads();
+  for (int i = tid; i < V * kP7Words; i += kEncThreads) {
+    const int64_t orow = orow_s[i / kP7Words];
+    if (orow >= 0) p.angles[orow * kP7Words + i % kP7Words] = words[i];
+  }
+
+  // ---- sketch: 16 S rows x 16 vectors a tile, k = a lane group's four dims
+  // (one 16-byte read of a row feeds four products)
+  constexpr int SETS = V / 16, TILES = SETS < 8 ? SETS : 8;  // 8 row tiles x SETS over 8 waves
+  static_assert(SETS == 1 || SETS == 2 || SETS == 4 || SETS == 8, "V");
+  const int m = lane & 15, c = lane >> 4;
+  const int v = 16 * (wave % SETS) + m, tile0 = (wave / SETS) * TILES;
+  const float* rrow = xs + v * kEncStr;
+  f4 acc[TILES];
+#pragma unroll
+  for (int tl = 0; tl < TILES; ++tl) acc[tl] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  float s2 = 0.0f;  // |S_i|^2: four lanes a row
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+#pragma unroll
+    for (int j = 0; j < 16; j += 4) {
+      const float4 a = *reinterpret_cast<const float4*>(ms + (tid >> 2) * kEncHalfStr + 16 * (tid & 3) + j);
+      s2 += a.x * a.x; s2 += a.y * a.y; s2 += a.z * a.z; s2 += a.w * a.w;
+    }
+#pragma unroll
+    for (int d = 0; d < 64; d += 16) {
+      const f4 bv = *reinterpret_cast<const f4*>(rrow + 64 * half + d + 4 * c);
+#pragma unroll
+      for (int tl = 0; tl < TILES; ++tl) {
+        const f4 av = *reinterpret_cast<const f4*>(ms + (16 * (tile0 + tl) + m) * kEncHalfStr + d + 4 * c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[tl] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], bv[e], acc[tl], 0, 0, 0);
+      }
+    }
+    if (half == 0) {
+      __syncthreads();
+      store_half(ms, mreg);
+    } else {
+      s2 += __shfl_xor(s2, 1, 64);
+      s2 += __shfl_xor(s2, 2, 64);
+      if ((tid & 3) == 0) sn[tid >> 2] = (s2 > 1e-25f && s2 < 1e30f) ? sqrtf(s2) : INFINITY;
+    }
+    __syncthreads();
+  }
+  const float rv = rn[v];
+  const int64_t orow = orow_s[v];
+  uint16_t* qj = reinterpret_cast<uint16_t*>(p.qjl);
+#pragma unroll
+  for (int tl = 0; tl < TILES; ++tl) {
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = 16 * (tile0 + tl) + 4 * c + i;
+      float dot = acc[tl][i];
+      if (!(fabsf(dot) > kSketchSlack * sn[row] * rv)) {  // NaN too
+        const float* srow = p.S + row * 128;
+        dot = 0.0f;
+#pragma unroll 8
+        for (int d = 0; d < 128; ++d) dot = dot + rrow[d] * srow[d];
+      }
+      bits |= (dot >= 0.0f ? 1u : 0u) << i;
+    }
+    bits <<= 4 * c;
+    bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), 16, 64));
+    bits |= static_cast<uint32_t>(__shfl_xor(static_cast<int>(bits), 32, 64));
+    if (c == 0 && orow >= 0) qj[orow * 8 + tile0 + tl] = static_cast<uint16_t>(bits);
+  }
+}
+
+// Vectors per workgroup: 64, or 16 for small inputs (four times the
+// workgroups, a quarter of a lane's chain of angles).  Whole calls, 16 against
+// 64 vectors: 17.6 / 31.0 us at 16 rows, 32.9 / 38.3 at 8,192, 44.6 / 38.8 at
+// 12,288, 181.7 / 104.7 at 65,536.
+int launch_p7_encode(const P7EncParams& p, hipStream_t s) {
+  constexpr int64_t kWide = 10240;
+  if (p.n > kWide) {
+    polar7_encode_kernel<64, 2, 8, 8><<<static_cast<unsigned>((p.n + 63) / 64), kEncThreads, 0, s>>>(p);
+  } else {
+    polar7_encode_kernel<16, 1, 4, 2><<<static_cast<unsigned>((p.n + 15) / 16), kEncThreads, 0, s>>>(p);
+  }
+  TQ_CHECK_LAUNCH("polar7_encode_kernel");
+  return TQ_OK;
 }
 
 // y = x P^T for rows of 128 (the query rotation q' = P q); fp32, any order.
@@ -1906,10 +2110,7 @@ int tq_polar7_encode(const float* x, const float* precondition, const float* ske
   p.x = x; p.P = precondition; p.S = sketch; p.cb = codebooks; p.cs = cs_tables;
   p.n = n_vectors;
   p.angles = angles; p.norms = norms; p.qjl = qjl;
-  const int64_t grid = std::min<int64_t>((n_vectors + 3) / 4, 8192);
-  polar7_encode_kernel<<<static_cast<unsigned>(grid), 256, 0, static_cast<hipStream_t>(stream)>>>(p);
-  TQ_CHECK_LAUNCH("polar7_encode_kernel");
-  return TQ_OK;
+  return launch_p7_encode(p, static_cast<hipStream_t>(stream));
 }
 
 int tq_polar7_kv_append(const float* k_new, const float* precondition, const float* sketch,
@@ -1927,10 +2128,7 @@ int tq_polar7_kv_append(const float* k_new, const float* precondition, const flo
   p.n = static_cast<int64_t>(batch) * num_kv_heads * n_new;
   p.positions = positions; p.n_new = n_new; p.cap = kv_capacity; p.Hkv = num_kv_heads;
   p.angles = angles; p.norms = norms; p.qjl = qjl;
-  const int64_t grid = std::min<int64_t>((p.n + 3) / 4, 8192);
-  polar7_encode_kernel<<<static_cast<unsigned>(grid), 256, 0, static_cast<hipStream_t>(stream)>>>(p);
-  TQ_CHECK_LAUNCH("polar7_encode_kernel");
-  return TQ_OK;
+  return launch_p7_encode(p, static_cast<hipStream_t>(stream));
 }
 
 int tq_polar7_prepare_query(const float* q, const float* precondition, const float* sketch,

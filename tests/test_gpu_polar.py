@@ -165,6 +165,25 @@ def test_polar7_encode_bit_exact(pq, n, rot):
         assert mism.size == 0, f"{name}: rows {mism[:8]} differ ({mism.size} rows)"
 
 
+@pytest.mark.parametrize("n,rot", [(16, True), (17, False), (10240 - 8, True), (10240 - 7 + 64, True), (10240 + 129, False)])
+def test_polar7_encode_tiles_and_scales(pq, n, rot):
+    """Row counts at the edges of the 16- and 64-vector workgroups, rows of
+    very small and very large norm (the sketch's sign bound does not hold
+    there), and a sketch with zero rows and exact cancellations."""
+    rng, x, P, S = p7_inputs(300 + n, n, rot)
+    x[: n // 4] *= np.array([1e-30, 1e-14, 1e14, 1.0], f32)[np.arange(n // 4) % 4][:, None]
+    S[3] = 0.0
+    S[5] = np.sign(S[5])
+    S[77] *= f32(1e-20)
+    ang, norms, qjl = PQ.polar7_encode(x, P, S)
+    codec = pq.Polar7Codec(dev(P) if rot else None, dev(S))
+    ga, gn, gq = (host(t) for t in codec.encode(dev(x)))
+    nrm16 = norms.view(np.uint16).astype(np.uint32)
+    for name, g, w in (("angles", ga, ang), ("norms", gn, nrm16[:, 0] | (nrm16[:, 1] << 16)), ("qjl", gq, qjl)):
+        mism = np.flatnonzero((g != w).reshape(g.shape[0], -1).any(axis=1))
+        assert mism.size == 0, f"{name}: rows {mism[:8]} differ ({mism.size} rows)"
+
+
 def test_polar7_kv_append_positions(pq):
     rng, x, P, S = p7_inputs(5, 0)
     B, Hkv, T, cap = 3, 2, 4, 10
