@@ -136,11 +136,224 @@ struct Enc16Params {
   uint32_t* p1;                 // packed outputs
   uint8_t *p2, *p3, *p4;
   uint16_t* radii;
+  bool wide_idx;   // unpacked outputs aligned for whole-block stores
 };
 
-// One workgroup per `rows` vectors: the tile is rotated in LDS (y = x P^T,
-// y_i accumulated d = 0..D-1 with separately rounded products and sums),
-// then one thread encodes each 16-value block.
+constexpr int kEncThreads = 512;
+// Values up to which a workgroup takes 16 (D 64: 32) vectors, more above it.
+// Whole calls, few against many vectors: D 256, 4,096 vectors 43 / 51 us, 5,120
+// 61 / 51; D 128, 8,192 vectors 28 / 28, 10,240 34 / 28, 32,768 68 / 47.
+constexpr int64_t kEnc16Small = 1 << 20;
+// LDS row strides of the encoders are 16 bytes past a multiple of the 256-byte
+// bank period (rows of 64 k floats, padded by 4): a 16-lane phase of row
+// reads covers every bank once.
+constexpr int kEncColStr = 64 + 4;  // 64 columns of a matrix
+
+// Rows r0 .. r0 + ROWS - 1, columns c0 .. c0 + 63 of a matrix with rows of DIM
+// floats (the 16-byte global loads here need the 4-byte alignment of a float
+// only): into registers, ROWS / 32 float4 a thread, and from there into LDS.
+template <int ROWS, int DIM>
+__device__ __forceinline__ void load_cols(const float* m, int r0, int c0, float4 (&r)[ROWS / 32]) {
+#pragma unroll
+  for (int i = 0; i < ROWS / 32; ++i) {
+    const int e = threadIdx.x + kEncThreads * i;
+    r[i] = *reinterpret_cast<const float4*>(m + (r0 + (e >> 4)) * DIM + c0 + 4 * (e & 15));
+  }
+}
+template <int N>
+__device__ __forceinline__ void store_cols(float* ms, const float4 (&r)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int e = threadIdx.x + kEncThreads * i;
+    *reinterpret_cast<float4*>(ms + (e >> 4) * kEncColStr + 4 * (e & 15)) = r[i];
+  }
+}
+
+// Adds 64 terms, in order, product and sum rounded separately (the encoders'
+// definition), to the sums of TV vectors and TI matrix rows a thread:
+// acc[j][k] += sum_d xs[v0 + j][d] * ms[i0 + ig k][d].  Every 16-byte LDS read
+// of a row serves TV or TI sums, so the VALU binds (2 instructions a term).
+template <int XSTR, int TV, int TI>
+__device__ __forceinline__ void exact_dots(const float* xs, const float* ms, int v0, int i0, int ig,
+                                           float (&acc)[TV][TI]) {
+#pragma clang fp contract(off)
+#pragma unroll 2
+  for (int d = 0; d < 64; d += 4) {
+    float4 x[TV], m[TI];
+#pragma unroll
+    for (int j = 0; j < TV; ++j) x[j] = *reinterpret_cast<const float4*>(xs + (v0 + j) * XSTR + d);
+#pragma unroll
+    for (int k = 0; k < TI; ++k) m[k] = *reinterpret_cast<const float4*>(ms + (i0 + ig * k) * kEncColStr + d);
+#pragma unroll
+    for (int j = 0; j < TV; ++j)
+#pragma unroll
+      for (int k = 0; k < TI; ++k) {
+        float a = acc[j][k];
+        a = a + x[j].x * m[k].x;
+        a = a + x[j].y * m[k].y;
+        a = a + x[j].z * m[k].z;
+        a = a + x[j].w * m[k].w;
+        acc[j][k] = a;
+      }
+  }
+}
+
+// nearest_idx over an LDS codebook padded with infinities to a multiple of
+// four entries (an infinity is never nearest), four entries a read.
+__device__ __forceinline__ int nearest_idx4(float th, const float* cb, int n) {
+#pragma clang fp contract(off)
+  float best = 1e10f;
+  int idx = 0;
+  for (int c = 0; c < n; c += 4) {
+    const float4 e = *reinterpret_cast<const float4*>(cb + c);
+    const float d[4] = {fabsf(th - e.x), fabsf(th - e.y), fabsf(th - e.z), fabsf(th - e.w)};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (d[i] < best) {
+        best = d[i];
+        idx = c + i;
+      }
+  }
+  return idx;
+}
+
+// The codebooks in LDS, [4][256], padded for nearest_idx4.
+template <int NT>
+__device__ __forceinline__ void fill_codebooks(float* cbs, const Enc16Params& p) {
+#pragma unroll
+  for (int l = 0; l < 4; ++l)
+    for (int c = threadIdx.x; c < ((p.ncb[l] + 3) & ~3); c += NT)
+      cbs[256 * l + c] = c < p.ncb[l] ? p.cb[p.cb_off[l] + c] : INFINITY;
+}
+
+// Encodes one 16-value block (global block gb) and stores its indices and radius.
+template <bool kPacked>
+__device__ __forceinline__ void encode_block16(const Enc16Params& p, const float* cbs, const float* y, int64_t gb) {
+#pragma clang fp contract(off)
+  float r[16];
+#pragma unroll
+  for (int j = 0; j < 16; j += 4) {
+    const float4 t = *reinterpret_cast<const float4*>(y + j);
+    r[j] = t.x; r[j + 1] = t.y; r[j + 2] = t.z; r[j + 3] = t.w;
+  }
+  int k1[8], k2[4], k3[2], k4;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float a = r[2 * j], b = r[2 * j + 1];
+    float th = atan2_det(b, a);
+    if (th < 0.0f) th = th + kTwoPi;
+    k1[j] = nearest_idx4(th, cbs, p.ncb[0]);
+    r[j] = pair_radius(a, b);
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float a = r[2 * j], b = r[2 * j + 1];
+    k2[j] = nearest_idx4(atan2_det(b, a), cbs + 256, p.ncb[1]);
+    r[j] = pair_radius(a, b);
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float a = r[2 * j], b = r[2 * j + 1];
+    k3[j] = nearest_idx4(atan2_det(b, a), cbs + 512, p.ncb[2]);
+    r[j] = pair_radius(a, b);
+  }
+  k4 = nearest_idx4(atan2_det(r[1], r[0]), cbs + 768, p.ncb[3]);
+  const float rad = pair_radius(r[0], r[1]);
+  if constexpr (kPacked) {
+    uint32_t w1 = 0, w2 = 0, w3 = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w1 |= (static_cast<uint32_t>(k1[j]) & 0xFu) << (4 * j);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w2 |= (static_cast<uint32_t>(k2[j]) & 0x3u) << (2 * j);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) w3 |= (static_cast<uint32_t>(k3[j]) & 0x3u) << (2 * j);
+    p.p1[gb] = w1;
+    p.p2[gb] = static_cast<uint8_t>(w2);
+    p.p3[gb] = static_cast<uint8_t>(w3);
+    p.p4[gb] = static_cast<uint8_t>(k4 & 0x3);
+  } else if (p.wide_idx) {
+    uint2 a;
+    a.x = k1[0] | (k1[1] << 8) | (k1[2] << 16) | (k1[3] << 24);
+    a.y = k1[4] | (k1[5] << 8) | (k1[6] << 16) | (k1[7] << 24);
+    reinterpret_cast<uint2*>(p.i1)[gb] = a;
+    reinterpret_cast<uint32_t*>(p.i2)[gb] = k2[0] | (k2[1] << 8) | (k2[2] << 16) | (k2[3] << 24);
+    reinterpret_cast<uint16_t*>(p.i3)[gb] = static_cast<uint16_t>(k3[0] | (k3[1] << 8));
+    p.i4[gb] = static_cast<uint8_t>(k4);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p.i1[gb * 8 + j] = static_cast<uint8_t>(k1[j]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) p.i2[gb * 4 + j] = static_cast<uint8_t>(k2[j]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) p.i3[gb * 2 + j] = static_cast<uint8_t>(k3[j]);
+    p.i4[gb] = static_cast<uint8_t>(k4);
+  }
+  p.radii[gb] = __half_as_ushort(__float2half_rn(rad));
+}
+
+// D 64 / 128 / 256: V vectors per workgroup of eight waves.  The rotation
+// stages P in tiles of up to 128 rows x 64 columns (the next tile's loads run
+// under the sums), a thread sums TV vectors x TI rows, and y goes over x once
+// every tile is done; then a thread encodes a 16-value block.
+// What bounds it: the rotation's VALU (2 D^2 lane instructions a vector in the
+// defined order; 27 us for 32,768 vectors of 128) and the angles (~15 of ~130
+// instructions a block).  One thread per output with P rows read from L2 at a
+// 4 D-byte lane stride took 246 us there.
+template <int D, int V, int TV, int TI, bool kPacked>
+__global__ __launch_bounds__(kEncThreads) void polar_encode16_tile_kernel(Enc16Params p) {
+#pragma clang fp contract(off)
+  constexpr int ROWS = D < 128 ? D : 128, NR = D / ROWS, NC = D / 64, IG = ROWS / TI, XSTR = D + 4;
+  static_assert((V / TV) * IG == kEncThreads && V * D / 16 <= kEncThreads, "thread tiles");
+  __shared__ __align__(16) float cbs[1024];
+  __shared__ __align__(16) float ms[ROWS * kEncColStr];
+  __shared__ __align__(16) float xs[V * XSTR];
+  const int tid = threadIdx.x;
+  const int64_t row0 = static_cast<int64_t>(blockIdx.x) * V;
+  const int rows = static_cast<int>(min(static_cast<int64_t>(V), p.n - row0));
+  float4 mreg[ROWS / 32];
+  if (p.P) load_cols<ROWS, D>(p.P, 0, 0, mreg);
+  fill_codebooks<kEncThreads>(cbs, p);
+#pragma unroll
+  for (int e = tid; e < V * D / 4; e += kEncThreads) {
+    const int r = e / (D / 4), c = 4 * (e % (D / 4));
+    // rows past the end: a copy, not stored
+    *reinterpret_cast<float4*>(xs + r * XSTR + c) =
+        *reinterpret_cast<const float4*>(p.x + (row0 + min(r, rows - 1)) * D + c);
+  }
+  if (p.P) {
+    const int i0 = tid % IG, v0 = (tid / IG) * TV;
+    float acc[NR][TV][TI];
+#pragma unroll
+    for (int t = 0; t < NR * NC; ++t) {
+      const int rt = t / NC, ct = t % NC;
+      if (t) __syncthreads();  // every wave is done with the previous tile
+      store_cols(ms, mreg);
+      if (t + 1 < NR * NC) load_cols<ROWS, D>(p.P, (t + 1) / NC * ROWS, (t + 1) % NC * 64, mreg);
+      __syncthreads();
+      if (ct == 0) {
+#pragma unroll
+        for (int j = 0; j < TV; ++j)
+#pragma unroll
+          for (int k = 0; k < TI; ++k) acc[rt][j][k] = 0.0f;
+      }
+      exact_dots<XSTR>(xs + 64 * ct, ms, v0, i0, IG, acc[rt]);
+    }
+    __syncthreads();  // every wave is done with x
+#pragma unroll
+    for (int rt = 0; rt < NR; ++rt)
+#pragma unroll
+      for (int j = 0; j < TV; ++j)
+#pragma unroll
+        for (int k = 0; k < TI; ++k) xs[(v0 + j) * XSTR + ROWS * rt + i0 + IG * k] = acc[rt][j][k];
+  }
+  __syncthreads();
+  constexpr int NB = D / 16;
+  if (tid < rows * NB) encode_block16<kPacked>(p, cbs, xs + (tid / NB) * XSTR + 16 * (tid % NB), row0 * NB + tid);
+}
+
+// Any other D: one workgroup per `rows` vectors, the tile rotated in LDS
+// (y = x P^T, y_i accumulated d = 0..D-1 with separately rounded products and
+// sums), then one thread encodes each 16-value block.
 template <bool kPacked>
 __global__ __launch_bounds__(256) void polar_encode16_kernel(Enc16Params p) {
 #pragma clang fp contract(off)
@@ -151,10 +364,7 @@ __global__ __launch_bounds__(256) void polar_encode16_kernel(Enc16Params p) {
   float* ys = xs + R * D;  // [R][D]
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
   const int rows = static_cast<int>(min(static_cast<int64_t>(R), p.n - row0));
-  for (int i = threadIdx.x; i < 1024; i += 256) {
-    const int l = i >> 8, c = i & 255;
-    cbs[i] = c < p.ncb[l] ? p.cb[p.cb_off[l] + c] : 0.0f;
-  }
+  fill_codebooks<256>(cbs, p);
   for (int i = threadIdx.x; i < rows * D; i += 256) xs[i] = p.x[row0 * D + i];
   __syncthreads();
   const float* y = xs;
@@ -171,57 +381,8 @@ __global__ __launch_bounds__(256) void polar_encode16_kernel(Enc16Params p) {
     y = ys;
   }
   const int nb = D / 16;
-  for (int blk = threadIdx.x; blk < rows * nb; blk += 256) {
-    float r[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) r[j] = y[blk * 16 + j];
-    int k1[8], k2[4], k3[2], k4;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float a = r[2 * j], b = r[2 * j + 1];
-      float th = atan2_det(b, a);
-      if (th < 0.0f) th = th + kTwoPi;
-      k1[j] = nearest_idx(th, cbs, p.ncb[0]);
-      r[j] = pair_radius(a, b);
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float a = r[2 * j], b = r[2 * j + 1];
-      k2[j] = nearest_idx(atan2_det(b, a), cbs + 256, p.ncb[1]);
-      r[j] = pair_radius(a, b);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const float a = r[2 * j], b = r[2 * j + 1];
-      k3[j] = nearest_idx(atan2_det(b, a), cbs + 512, p.ncb[2]);
-      r[j] = pair_radius(a, b);
-    }
-    k4 = nearest_idx(atan2_det(r[1], r[0]), cbs + 768, p.ncb[3]);
-    const float rad = pair_radius(r[0], r[1]);
-    const int64_t gb = row0 * nb + blk;
-    if constexpr (kPacked) {
-      uint32_t w1 = 0, w2 = 0, w3 = 0;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) w1 |= (static_cast<uint32_t>(k1[j]) & 0xFu) << (4 * j);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w2 |= (static_cast<uint32_t>(k2[j]) & 0x3u) << (2 * j);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) w3 |= (static_cast<uint32_t>(k3[j]) & 0x3u) << (2 * j);
-      p.p1[gb] = w1;
-      p.p2[gb] = static_cast<uint8_t>(w2);
-      p.p3[gb] = static_cast<uint8_t>(w3);
-      p.p4[gb] = static_cast<uint8_t>(k4 & 0x3);
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p.i1[gb * 8 + j] = static_cast<uint8_t>(k1[j]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) p.i2[gb * 4 + j] = static_cast<uint8_t>(k2[j]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) p.i3[gb * 2 + j] = static_cast<uint8_t>(k3[j]);
-      p.i4[gb] = static_cast<uint8_t>(k4);
-    }
-    p.radii[gb] = __half_as_ushort(__float2half_rn(rad));
-  }
+  for (int blk = threadIdx.x; blk < rows * nb; blk += 256)
+    encode_block16<kPacked>(p, cbs, y + blk * 16, row0 * nb + blk);
 }
 
 struct Keys16 {
@@ -511,58 +672,6 @@ struct P7EncParams {
   uint32_t* qjl;     // [.][4]
 };
 
-constexpr int kEncThreads = 512;
-// Row strides in LDS, 16 bytes past a multiple of the 256-byte bank period:
-// a 16-lane phase of row reads covers every bank once.
-constexpr int kEncStr = 132;     // rows of 128 floats
-constexpr int kEncHalfStr = 68;  // rows of 64 floats
-
-// Columns 64 half .. +63 of a 128 x 128 matrix into registers, 4 float4 a
-// thread, and from there into LDS rows.
-__device__ __forceinline__ void load_half(const float* m, int half, float4 (&r)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int e = threadIdx.x + kEncThreads * i;
-    r[i] = reinterpret_cast<const float4*>(m)[(e >> 4) * 32 + 16 * half + (e & 15)];
-  }
-}
-__device__ __forceinline__ void store_half(float* ms, const float4 (&r)[4]) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int e = threadIdx.x + kEncThreads * i;
-    *reinterpret_cast<float4*>(ms + (e >> 4) * kEncHalfStr + 4 * (e & 15)) = r[i];
-  }
-}
-
-// Adds 64 terms, in order, product and sum rounded separately (the encoder's
-// definition), to the sums of TV vectors and TI matrix rows a thread:
-// acc[j][k] += sum_d xs[v0 + j][d] * ms[i0 + IG k][d].  Every 16-byte LDS read
-// of a row serves TV or TI sums, so the VALU binds (2 instructions a term).
-template <int TV, int TI>
-__device__ __forceinline__ void exact_dots(const float* xs, const float* ms, int v0, int i0, float (&acc)[TV][TI]) {
-#pragma clang fp contract(off)
-  constexpr int IG = 128 / TI;
-#pragma unroll 2
-  for (int d = 0; d < 64; d += 4) {
-    float4 x[TV], m[TI];
-#pragma unroll
-    for (int j = 0; j < TV; ++j) x[j] = *reinterpret_cast<const float4*>(xs + (v0 + j) * kEncStr + d);
-#pragma unroll
-    for (int k = 0; k < TI; ++k) m[k] = *reinterpret_cast<const float4*>(ms + (i0 + IG * k) * kEncHalfStr + d);
-#pragma unroll
-    for (int j = 0; j < TV; ++j)
-#pragma unroll
-      for (int k = 0; k < TI; ++k) {
-        float a = acc[j][k];
-        a = a + x[j].x * m[k].x;
-        a = a + x[j].y * m[k].y;
-        a = a + x[j].z * m[k].z;
-        a = a + x[j].w * m[k].w;
-        acc[j][k] = a;
-      }
-  }
-}
-
 // The index of angle j of level l (1 .. 7) goes into word p7_word(l, j) of the
 // vector at bit p7_bit(l, j) (the layout of tq_c_api.h).
 __device__ __forceinline__ constexpr int p7_word(int l, int j) {
@@ -603,8 +712,9 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
 #pragma clang fp contract(off)
   constexpr int LPV = 64 / PPL;  // lanes a vector
   static_assert((V / TV) * (128 / TI) == kEncThreads && V % 16 == 0 && V * LPV <= kEncThreads, "thread tiles");
+  constexpr int kEncStr = 128 + 4;
   typedef float f4 __attribute__((ext_vector_type(4)));
-  __shared__ __align__(16) float ms[128 * kEncHalfStr];  // a half of P, then of S
+  __shared__ __align__(16) float ms[128 * kEncColStr];  // a half of P, then of S
   __shared__ __align__(16) float xs[V * kEncStr];        // x, then y, then the residual
   __shared__ uint32_t words[V * kP7Words];
   __shared__ float2 cs[20];
@@ -615,7 +725,7 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * V;
   float4 mreg[4];
-  if (p.P) load_half(p.P, 0, mreg);
+  if (p.P) load_cols<128, 128>(p.P, 0, 0, mreg);
   // uniform: scalar registers
   float cb1[16], cb2[4];
 #pragma unroll
@@ -649,21 +759,21 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
     for (int j = 0; j < TV; ++j)
 #pragma unroll
       for (int k = 0; k < TI; ++k) acc[j][k] = 0.0f;
-    store_half(ms, mreg);
-    load_half(p.P, 1, mreg);
+    store_cols(ms, mreg);
+    load_cols<128, 128>(p.P, 0, 64, mreg);
     __syncthreads();
-    exact_dots<TV, TI>(xs, ms, v0, i0, acc);
+    exact_dots<kEncStr>(xs, ms, v0, i0, IG, acc);
     __syncthreads();  // every wave is done with the first half
-    store_half(ms, mreg);
+    store_cols(ms, mreg);
     __syncthreads();
-    exact_dots<TV, TI>(xs + 64, ms, v0, i0, acc);
+    exact_dots<kEncStr>(xs + 64, ms, v0, i0, IG, acc);
     __syncthreads();  // every wave is done with x and P
 #pragma unroll
     for (int j = 0; j < TV; ++j)
 #pragma unroll
       for (int k = 0; k < TI; ++k) xs[(v0 + j) * kEncStr + i0 + IG * k] = acc[j][k];
   }
-  load_half(p.S, 0, mreg);
+  load_cols<128, 128>(p.S, 0, 0, mreg);
   __syncthreads();
 
   // ---- encode: lane b of a vector has pairs PPL b .. PPL b + PPL - 1
@@ -758,8 +868,8 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
                         (static_cast<uint32_t>(__half_as_ushort(rn16)) << 16);
     }
   }
-  store_half(ms, mreg);  // P is no longer read (barrier before the encoding)
-  load_half(p.S, 1, mreg);
+  store_cols(ms, mreg);  // P is no longer read (barrier before the encoding)
+  load_cols<128, 128>(p.S, 0, 64, mreg);
   __syncthreads();
   for (int i = tid; i < V * kP7Words; i += kEncThreads) {
     const int64_t orow = orow_s[i / kP7Words];
@@ -781,7 +891,7 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
   for (int half = 0; half < 2; ++half) {
 #pragma unroll
     for (int j = 0; j < 16; j += 4) {
-      const float4 a = *reinterpret_cast<const float4*>(ms + (tid >> 2) * kEncHalfStr + 16 * (tid & 3) + j);
+      const float4 a = *reinterpret_cast<const float4*>(ms + (tid >> 2) * kEncColStr + 16 * (tid & 3) + j);
       s2 += a.x * a.x; s2 += a.y * a.y; s2 += a.z * a.z; s2 += a.w * a.w;
     }
 #pragma unroll
@@ -789,14 +899,14 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
       const f4 bv = *reinterpret_cast<const f4*>(rrow + 64 * half + d + 4 * c);
 #pragma unroll
       for (int tl = 0; tl < TILES; ++tl) {
-        const f4 av = *reinterpret_cast<const f4*>(ms + (16 * (tile0 + tl) + m) * kEncHalfStr + d + 4 * c);
+        const f4 av = *reinterpret_cast<const f4*>(ms + (16 * (tile0 + tl) + m) * kEncColStr + d + 4 * c);
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[tl] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[e], bv[e], acc[tl], 0, 0, 0);
       }
     }
     if (half == 0) {
       __syncthreads();
-      store_half(ms, mreg);
+      store_cols(ms, mreg);
     } else {
       s2 += __shfl_xor(s2, 1, 64);
       s2 += __shfl_xor(s2, 2, 64);
@@ -836,7 +946,7 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
 int launch_p7_encode(const P7EncParams& p, hipStream_t s) {
   constexpr int64_t kWide = 10240;
   if (p.n > kWide) {
-    polar7_encode_kernel<64, 2, 8, 8><<<static_cast<unsigned>((p.n + 63) / 64), kEncThreads, 0, s>>>(p);
+    polar7_encode_kernel<64, 4, 4, 8><<<static_cast<unsigned>((p.n + 63) / 64), kEncThreads, 0, s>>>(p);
   } else {
     polar7_encode_kernel<16, 1, 4, 2><<<static_cast<unsigned>((p.n + 15) / 16), kEncThreads, 0, s>>>(p);
   }
@@ -1763,6 +1873,36 @@ using namespace tq;
 
 namespace {
 
+// 512 blocks per workgroup, or 16 vectors for small inputs (more workgroups).
+template <int D, int V, int TV, int TI, bool kPacked>
+int launch_encode16_tile(const Enc16Params& p, hipStream_t s, const char* fn) {
+  const int64_t grid = (p.n + V - 1) / V;
+  TQ_CHECK_ARG(grid <= (int64_t{1} << 31) - 1, "%s: too many vectors", fn);
+  polar_encode16_tile_kernel<D, V, TV, TI, kPacked><<<static_cast<unsigned>(grid), kEncThreads, 0, s>>>(p);
+  TQ_CHECK_LAUNCH("polar_encode16_tile_kernel");
+  return TQ_OK;
+}
+
+template <bool kPacked>
+int launch_encode16(const Enc16Params& p, hipStream_t s, const char* fn) {
+  const bool small = p.n * p.D <= kEnc16Small;
+  switch (p.D) {
+    case 64: return small ? launch_encode16_tile<64, 32, 1, 4, kPacked>(p, s, fn)
+                          : launch_encode16_tile<64, 128, 4, 4, kPacked>(p, s, fn);
+    case 128: return small ? launch_encode16_tile<128, 16, 1, 4, kPacked>(p, s, fn)
+                           : launch_encode16_tile<128, 64, 4, 4, kPacked>(p, s, fn);
+    case 256: return small ? launch_encode16_tile<256, 16, 1, 4, kPacked>(p, s, fn)
+                           : launch_encode16_tile<256, 32, 2, 4, kPacked>(p, s, fn);
+    default: break;
+  }
+  const int64_t grid = (p.n + p.rows - 1) / p.rows;
+  TQ_CHECK_ARG(grid <= (int64_t{1} << 31) - 1, "%s: too many vectors", fn);
+  const size_t shm = sizeof(float) * (1024 + 2 * static_cast<size_t>(p.rows) * p.D);
+  polar_encode16_kernel<kPacked><<<static_cast<unsigned>(grid), 256, shm, s>>>(p);
+  TQ_CHECK_LAUNCH("polar_encode16_kernel");
+  return TQ_OK;
+}
+
 int encode16_common(const float* x, const float* P, const float* codebooks, const int* n_codebook,
                     int64_t n, int D, int block_size, bool packed, uint8_t* i1, uint8_t* i2,
                     uint8_t* i3, uint8_t* i4, uint32_t* p1, uint8_t* p2, uint8_t* p3, uint8_t* p4,
@@ -1788,14 +1928,10 @@ int encode16_common(const float* x, const float* P, const float* codebooks, cons
   p.i1 = i1; p.i2 = i2; p.i3 = i3; p.i4 = i4;
   p.p1 = p1; p.p2 = p2; p.p3 = p3; p.p4 = p4;
   p.radii = radii;
-  const int64_t grid = (n + p.rows - 1) / p.rows;
-  TQ_CHECK_ARG(grid <= (int64_t{1} << 31) - 1, "%s: too many vectors", fn);
-  const size_t shm = sizeof(float) * (1024 + 2 * static_cast<size_t>(p.rows) * D);
+  p.wide_idx = reinterpret_cast<uintptr_t>(i1) % 8 == 0 && reinterpret_cast<uintptr_t>(i2) % 4 == 0 &&
+               reinterpret_cast<uintptr_t>(i3) % 2 == 0;
   hipStream_t hs = static_cast<hipStream_t>(stream);
-  if (packed) polar_encode16_kernel<true><<<static_cast<unsigned>(grid), 256, shm, hs>>>(p);
-  else polar_encode16_kernel<false><<<static_cast<unsigned>(grid), 256, shm, hs>>>(p);
-  TQ_CHECK_LAUNCH("polar_encode16_kernel");
-  return TQ_OK;
+  return packed ? launch_encode16<true>(p, hs, fn) : launch_encode16<false>(p, hs, fn);
 }
 
 int decode16_common(const Keys16& k, const float* P, const float* codebooks, const float* cs_tables,

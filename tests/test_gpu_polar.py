@@ -73,6 +73,38 @@ def test_polar_quantize_bit_exact(pq, D, packed, rot):
         assert mism.size == 0, f"output {i}: {mism.size} mismatches, first at {mism[:5]}"
 
 
+@pytest.mark.parametrize("D,n", [(64, 33), (64, 16384 + 130), (128, 1), (128, 17), (128, 8192), (128, 8192 + 65),
+                                 (256, 31), (256, 4096 + 33), (48, 100), (512, 9)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_polar_quantize_tiles(pq, D, n, packed):
+    """Row counts at the edges of the rotation tiles (up to 1,048,576 values:
+    16 or 32 vectors a workgroup, 512 blocks above), dims without a tile
+    kernel, and unpacked index arrays at odd addresses."""
+    import ctypes
+    from gemma4metal_amd._lib import call
+    rng = np.random.default_rng(D + n)
+    x, P = rng.standard_normal((n, D)).astype(f32), ortho(rng, D)
+    cbs = rand_codebooks(rng, packed)
+    ref = PQ.polar_quantize(x, P, cbs)
+    dcb, dx, dP = [dev(c) for c in cbs], dev(x), dev(P)
+    if packed:
+        got = [host(t) for t in pq.polar_quantize_packed(dx, dP, *dcb)]
+        want = list(PQ.pack_ref(ref[:4])) + [ref[4]]
+    else:
+        nb = n * D // 16
+        raw = [torch.zeros(nb * k + 1, dtype=torch.uint8, device="cuda") for k in (8, 4, 2, 1)]
+        rad = torch.empty(nb, dtype=torch.float16, device="cuda")
+        sizes = (ctypes.c_int * 4)(*[c.size for c in cbs])
+        call("tq_polar_quantize", dx.data_ptr(), dP.data_ptr(), torch.cat(dcb).data_ptr(),
+             ctypes.cast(sizes, ctypes.c_void_p), n, D, 16, *[t.data_ptr() + 1 for t in raw], rad.data_ptr(),
+             torch.cuda.current_stream().cuda_stream)
+        got, want = [host(t)[1:] for t in raw] + [host(rad)], list(ref)
+        for g, w in zip((host(t) for t in pq.polar_quantize(dx, dP, *dcb)), ref):
+            assert np.array_equal(g, w)
+    for i, (g, w) in enumerate(zip(got, want)):
+        assert np.array_equal(g.reshape(-1), w.reshape(-1)), f"output {i}"
+
+
 # ------------------------------------------------------------ decode ---------
 
 @pytest.mark.parametrize("D", [64, 128])
