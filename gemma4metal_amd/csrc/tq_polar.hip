@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "tq_sdpa_common.h"
 
@@ -530,123 +531,275 @@ struct Attn16 {
   float qscale;         // multiplies q (scale, or scale*log2e for attention)
 };
 
-// scores of key t of kv head kvh for G heads (q pre-scaled in LDS, [G][D])
-template <int D, int G, bool kPacked>
-__device__ __forceinline__ void score16(const Attn16& a, const float2* cst, const float* qs,
-                                        int64_t keyrow, float s[G]) {
-  constexpr int NB = D / 16;
+// Keys of the scores and attention: 64 / LPK keys per wave at a time, LPK =
+// D / 16 lanes a key, one 16-value block a lane.  The blocks of consecutive
+// keys are consecutive, so a wave's index loads are contiguous (8, 4, 2, 1 and
+// 2 bytes a lane; a key per lane read them at a D / 2-byte lane stride, 17
+// loads a block, and the address unit bound the kernel), and a lane's slice of
+// every query stays in registers.
+struct Block16 {
+  uint2 w1;            // level 1: a byte an index (packed: x holds the nibbles)
+  uint32_t w2, w3, w4;
+  uint16_t rad;
+};
+
+// Index layouts: unpacked at any address, unpacked and aligned for one load a
+// level of a block, packed.
+constexpr int kIdxBytes = 0, kIdxWide = 1, kIdxPacked = 2;
+
+// Block gb0 + i: gb0 is uniform, so every array is addressed as a scalar base
+// and one 32-bit lane offset (64-bit lane addresses of 16 loads in flight
+// spilled).
+template <int kIdx>
+__device__ __forceinline__ Block16 load_block16(const Attn16& a, int64_t gb0, uint32_t i) {
+  Block16 o;
+  o.rad = (a.k.radii + gb0)[i];
+  if constexpr (kIdx == kIdxPacked) {
+    o.w1 = make_uint2((a.k.p1 + gb0)[i], 0);
+    o.w2 = (a.k.p2 + gb0)[i];
+    o.w3 = (a.k.p3 + gb0)[i];
+    o.w4 = (a.k.p4 + gb0)[i];
+  } else if constexpr (kIdx == kIdxWide) {
+    o.w1 = reinterpret_cast<const uint2*>(a.k.i1 + gb0 * 8)[i];
+    o.w2 = reinterpret_cast<const uint32_t*>(a.k.i2 + gb0 * 4)[i];
+    o.w3 = reinterpret_cast<const uint16_t*>(a.k.i3 + gb0 * 2)[i];
+    o.w4 = (a.k.i4 + gb0)[i];
+  } else {
+    const auto bytes = [](const uint8_t* s, uint32_t at, int n) {
+      uint32_t w = 0;
 #pragma unroll
-  for (int g = 0; g < G; ++g) s[g] = 0.0f;
-  for (int blk = 0; blk < NB; ++blk) {
-    const int64_t gb = keyrow * NB + blk;
-    int k1[8], k2[4], k3[2], k4;
-    load_block_idx<kPacked>(a.k, gb, k1, k2, k3, k4);
-    const float rad = __half2float(__ushort_as_half(a.k.radii[gb]));
+      for (int j = 0; j < n; ++j) w |= static_cast<uint32_t>(s[at + j]) << (8 * j);
+      return w;
+    };
+    o.w1 = make_uint2(bytes(a.k.i1 + gb0 * 8, 8 * i, 4), bytes(a.k.i1 + gb0 * 8, 8 * i + 4, 4));
+    o.w2 = bytes(a.k.i2 + gb0 * 4, 4 * i, 4);
+    o.w3 = bytes(a.k.i3 + gb0 * 2, 2 * i, 2);
+    o.w4 = (a.k.i4 + gb0)[i];
+  }
+  return o;
+}
+
+// Dot products of one block with G query slices.  The tree is folded bottom
+// up (31 operations a head) or, from four heads on, decoded top down once (30)
+// and multiplied out (16 a head).
+template <int G, int kIdx>
+__device__ __forceinline__ void block_dots(const float2* cst, const Block16& o, const float (&q)[G][16], float (&s)[G]) {
+  constexpr bool kPacked = kIdx == kIdxPacked;
+  int k1[8], k2[4], k3[2];
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    k1[j] = kPacked ? (o.w1.x >> (4 * j)) & 0xF : ((j < 4 ? o.w1.x : o.w1.y) >> (8 * (j & 3))) & 0xFF;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) k2[j] = kPacked ? (o.w2 >> (2 * j)) & 0x3 : (o.w2 >> (8 * j)) & 0xFF;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) k3[j] = kPacked ? (o.w3 >> (2 * j)) & 0x3 : (o.w3 >> (8 * j)) & 0xFF;
+  const int k4 = kPacked ? o.w4 & 0x3 : o.w4;
+  const float rad = __half2float(__ushort_as_half(o.rad));
+  if constexpr (G >= 4) {
     float v[16];
     decode_block16(cst, rad, k1, k2, k3, k4, v);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const float4* q4 = reinterpret_cast<const float4*>(qs + g * D + blk * 16);
+      s[g] = q[g][0] * v[0];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float4 qv = q4[j];
-        s[g] = fmaf(qv.x, v[4 * j], s[g]);
-        s[g] = fmaf(qv.y, v[4 * j + 1], s[g]);
-        s[g] = fmaf(qv.z, v[4 * j + 2], s[g]);
-        s[g] = fmaf(qv.w, v[4 * j + 3], s[g]);
-      }
+      for (int j = 1; j < 16; ++j) s[g] = fmaf(q[g][j], v[j], s[g]);
+    }
+  } else {
+    float2 c1[8], c2[4], c3[2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c1[j] = cst[k1[j]];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c2[j] = cst[256 + k2[j]];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) c3[j] = cst[512 + k3[j]];
+    const float2 c4 = cst[768 + k4];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float t[8], u[4];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[j] = fmaf(q[g][2 * j + 1], c1[j].y, q[g][2 * j] * c1[j].x);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = fmaf(t[2 * j + 1], c2[j].y, t[2 * j] * c2[j].x);
+      const float w0 = fmaf(u[1], c3[0].y, u[0] * c3[0].x), w1 = fmaf(u[3], c3[1].y, u[2] * c3[1].x);
+      s[g] = rad * fmaf(w1, c4.y, w0 * c4.x);
     }
   }
 }
 
-// tq_score_shared (lib/turboquant.metal:424-499) + GQA: one key per thread,
-// 1024 keys per workgroup, grid (key blocks, kv heads * head subgroups).
-template <int D, int G, bool kPacked>
+// A lane's slice of the G queries, scaled.
+template <int D, int G>
+__device__ __forceinline__ void load_q_slices(const Attn16& a, int h0, int blk, float (&q)[G][16]) {
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) q[g][j] = a.qscale * a.q[static_cast<int64_t>(h0 + g) * D + 16 * blk + j];
+}
+
+// tq_score_shared (lib/turboquant.metal:424-499) + GQA: kScoreKeys keys per
+// workgroup of four waves, 64 keys (LPK batches) per wave at a time, grid
+// (key blocks, kv heads * head subgroups).
+constexpr int kScoreKeys = 512;
+
+template <int D, int G, int kIdx>
 __global__ __launch_bounds__(256) void polar16_score_kernel(Attn16 a, int n, int gqa, int n_sub) {
+  constexpr int LPK = D / 16, KPB = 64 / LPK;  // lanes a key, keys a batch
   __shared__ float2 cst[1024];
-  __shared__ __align__(16) float qs[G * D];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int hy = blockIdx.y, kvh = hy / n_sub, sub = hy - (hy / n_sub) * n_sub;
   const int h0 = kvh * gqa + sub * G;
+  const int blk = lane % LPK;
+  const int t_end = min(n, (static_cast<int>(blockIdx.x) + 1) * kScoreKeys);
+  float q[G][16];
+  load_q_slices<D, G>(a, h0, blk, q);
   fill_cs_tables<256>(cst, a.src);
-  for (int i = threadIdx.x; i < G * D; i += 256) qs[i] = a.qscale * a.q[static_cast<int64_t>(h0) * D + i];
   __syncthreads();
-  for (int t = blockIdx.x * 1024 + threadIdx.x; t < min(n, (blockIdx.x + 1) * 1024); t += 256) {
-    float s[G];
-    score16<D, G, kPacked>(a, cst, qs, static_cast<int64_t>(kvh) * n + t, s);
+  for (int tb = blockIdx.x * kScoreKeys + wave * 64; tb < t_end; tb += 256) {
+    const int64_t gb0 = (static_cast<int64_t>(kvh) * n + tb) * LPK;
+    const int left = (t_end - tb) * LPK - 1;  // last block of the range
+    float r[G];
 #pragma unroll
-    for (int g = 0; g < G; ++g) a.scores[static_cast<int64_t>(h0 + g) * n + t] = s[g];
+    for (int g = 0; g < G; ++g) r[g] = 0.0f;
+    constexpr int UN = 4;  // batches in flight (LPK is a multiple of 4)
+    for (int i0 = 0; i0 < LPK; i0 += UN) {
+      Block16 o[UN];
+#pragma unroll
+      for (int i = 0; i < UN; ++i) o[i] = load_block16<kIdx>(a, gb0, min(64 * (i0 + i) + lane, left));
+#pragma unroll
+      for (int i = 0; i < UN; ++i) {
+        float s[G];
+        block_dots<G, kIdx>(cst, o[i], q, s);
+        // lane (kk, blk) keeps batch blk's score of key kk
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const float t = group_sum<LPK>(s[g]);
+          r[g] = blk == i0 + i ? t : r[g];
+        }
+      }
+    }
+    const int t = tb + blk * KPB + lane / LPK;
+    if (t < t_end) {
+#pragma unroll
+      for (int g = 0; g < G; ++g) a.scores[static_cast<int64_t>(h0 + g) * n + t] = r[g];
+    }
   }
 }
 
 // sdpa_tq_sequential (lib/turboquant.metal:166-224) as split-K flash decoding
-// + GQA: 64-key tiles per wave (one key per lane), fp32 V with lanes owning
-// dimensions, output acc / (l + 1e-8).
-template <int D, int G, bool kPacked>
-__global__ __launch_bounds__(256) void polar16_sdpa_kernel(SdpaParams p, Attn16 a) {
+// + GQA, output acc / (l + 1e-8).  Eight waves, a tile of four batches of keys
+// each (64 / 32 / 16 keys at D 64 / 128 / 256): the tile's V rows (16 float4 a
+// lane, 256 / D rows an instruction, lanes owning four dims) and the next
+// tile's indices are in flight while the tile is scored.
+// What bounds it: the fp32 V stream.  16 heads x 8,192 keys of 128 (85 MB): a
+// key per lane with V rows loaded as they were needed took 47.7 us; this form
+// 19.0 (4.5 TB/s).
+constexpr int kSdpa16Waves = 8;
+
+template <int D, int G, int kIdx>
+__global__ __launch_bounds__(kSdpa16Waves * 64) void polar16_sdpa_kernel(SdpaParams p, Attn16 a) {
   pin_args(p);
-  constexpr int NW = 4, VE = D / 64;
+  constexpr int NW = kSdpa16Waves;
+  constexpr int LPK = D / 16, KPB = 64 / LPK, NB = 4, T = NB * KPB;
+  constexpr int LPR = D / 4, RPI = 64 / LPR, NV = T / RPI;  // lanes a V row, rows and instructions
+  static_assert(NV == 16 && RPI * 4 == KPB, "one batch of keys per four V instructions");
+  typedef float f4 __attribute__((ext_vector_type(4)));
   __shared__ float2 cst[1024];
-  __shared__ __align__(16) float qs[G * D];
   using Fin = Finalize<G, D, NW>;
   __shared__ __align__(16) float arena[Fin::kArena];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   const int hy = blockIdx.y, split = blockIdx.x;
   const int kvh = hy / p.n_sub, sub = hy - kvh * p.n_sub;
   const int h0 = kvh * p.gqa + sub * G;
   const SplitRange rg = split_range(p, 0, split);
   if (split >= rg.S) return;
-  fill_cs_tables<256>(cst, a.src);
-  for (int i = threadIdx.x; i < G * D; i += 256) qs[i] = a.qscale * a.q[static_cast<int64_t>(h0) * D + i];
+  const int blk = lane % LPK;
+  const int64_t rowbase = static_cast<int64_t>(kvh) * p.cap;
+  Block16 o[NB];
+  auto load_idx = [&](int tb) {
+    const int left = (rg.t_end - tb) * LPK - 1;  // last block of the split
+#pragma unroll
+    for (int i = 0; i < NB; ++i) o[i] = load_block16<kIdx>(a, (rowbase + tb) * LPK, min(64 * i + lane, left));
+  };
+  const int t0 = rg.t_begin + wv * T;
+  if (t0 < rg.t_end) load_idx(t0);
+  float q[G][16];
+  load_q_slices<D, G>(a, h0, blk, q);
+  fill_cs_tables<NW * 64>(cst, a.src);
   __syncthreads();
 
-  float m_run[G], l_run[G], acc[G][VE];
+  float m_run[G], l_run[G];
+  f4 acc[G];
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     m_run[g] = -INFINITY;
     l_run[g] = 0.0f;
-#pragma unroll
-    for (int e = 0; e < VE; ++e) acc[g][e] = 0.0f;
+    acc[g] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   }
-  const int64_t rowbase = static_cast<int64_t>(kvh) * p.cap;
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
-  for (int tb = rg.t_begin + wv * 64; tb < rg.t_end; tb += NW * 64) {
-    const bool valid = tb + lane < rg.t_end;
-    const int t = min(tb + lane, rg.t_end - 1);
-    float s[G], pw[G];
-    score16<D, G, kPacked>(a, cst, qs, rowbase + t, s);
+  const int vr = lane / LPR;  // V row of an instruction
+#pragma unroll 1
+  for (int tb = t0; tb < rg.t_end; tb += NW * T) {
+    f4 v[NV];
+    const f4* vbase = reinterpret_cast<const f4*>(a.values + (rowbase + tb) * D);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const uint32_t t = min(j * RPI + vr, rg.t_end - 1 - tb);
+      v[j] = __builtin_nontemporal_load(vbase + (t * LPR + lane % LPR));
+    }
+    float s[NB][G];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      block_dots<G, kIdx>(cst, o[i], q, s[i]);
+      // the sums are finished here: left to itself the compiler reads every
+      // block's tables first (30 registers each) and spills
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        s[i][g] = group_sum<LPK>(s[i][g]);
+        asm volatile("" : "+v"(s[i][g]));
+      }
+    }
+    if (tb + NW * T < rg.t_end) load_idx(tb + NW * T);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-      const float sv = valid ? s[g] : -INFINITY;
-      const float m_new = fmaxf(m_run[g], wave_max_f(sv));
+      float mt = -INFINITY;
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        if (tb + i * KPB + lane / LPK >= rg.t_end) s[i][g] = -INFINITY;
+        mt = fmaxf(mt, s[i][g]);
+      }
+      const float m_new = fmaxf(m_run[g], wave_max_f(mt));
       if (m_new > m_run[g]) {  // wave-uniform
         const float f = merge_factor(m_run[g], m_new);
         l_run[g] *= f;
-#pragma unroll
-        for (int e = 0; e < VE; ++e) acc[g][e] *= f;
+        acc[g] *= f;
         m_run[g] = m_new;
       }
-      pw[g] = valid ? fast_exp2(sv - m_run[g]) : 0.0f;
-      l_run[g] += pw[g];
-    }
-    const int nk = min(64, rg.t_end - tb);
-    for (int kk = 0; kk < nk; ++kk) {
-      const float* vr = a.values + (rowbase + tb + kk) * D + lane;
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const float pg = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pw[g]), kk));
-#pragma unroll
-        for (int e = 0; e < VE; ++e) acc[g][e] = fmaf(pg, vr[64 * e], acc[g][e]);
+      for (int i = 0; i < NB; ++i) {
+        // a masked key has weight 0 also while every score seen is -inf
+        s[i][g] = tb + i * KPB + lane / LPK < rg.t_end ? fast_exp2(s[i][g] - m_run[g]) : 0.0f;
+        l_run[g] += s[i][g];
       }
+    }
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int src = ((j & 3) * RPI + vr) * LPK;  // a lane of the row's key in batch j / 4
+#pragma unroll
+      for (int g = 0; g < G; ++g) acc[g] += __shfl(s[j >> 2][g], src, 64) * v[j];
     }
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) {
+    // rows of one instruction: lanes LPR apart hold the same dims
 #pragma unroll
-    for (int e = 0; e < VE; ++e) Fin::o(arena, wave, g)[lane + 64 * e] = acc[g][e];
-    const float ls = wave_sum_f(l_run[g]);
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (RPI >= 2) acc[g][e] = xor32_sum(acc[g][e]);
+      if constexpr (RPI >= 4) acc[g][e] = xor16_sum(acc[g][e]);
+    }
+    if (lane < LPR) *reinterpret_cast<f4*>(Fin::o(arena, wv, g) + 4 * lane) = acc[g];
+    const float ls = wave_sum_f(blk == 0 ? l_run[g] : 0.0f);
     if (lane == 0) {
-      Fin::m(arena, wave)[g] = m_run[g];
-      Fin::l(arena, wave)[g] = ls;
+      Fin::m(arena, wv)[g] = m_run[g];
+      Fin::l(arena, wv)[g] = ls;
     }
   }
   Fin::run(p, arena, h0, rg.S, split, hy);
@@ -1964,28 +2117,34 @@ int decode16_common(const Keys16& k, const float* P, const float* codebooks, con
   return TQ_OK;
 }
 
-template <int D, int G, bool kPacked>
-void launch_score16(const Attn16& a, int n, int gqa, int n_sub, dim3 grid, hipStream_t s) {
-  polar16_score_kernel<D, G, kPacked><<<grid, 256, 0, s>>>(a, n, gqa, n_sub);
+// f(index layout constant) for the layout of the call's indices
+template <typename F>
+auto with_idx_layout(const Attn16& a, F&& f) {
+  if (a.k.p1) return f(std::integral_constant<int, kIdxPacked>{});
+  const bool wide = reinterpret_cast<uintptr_t>(a.k.i1) % 8 == 0 && reinterpret_cast<uintptr_t>(a.k.i2) % 4 == 0 &&
+                    reinterpret_cast<uintptr_t>(a.k.i3) % 2 == 0;
+  if (wide) return f(std::integral_constant<int, kIdxWide>{});
+  return f(std::integral_constant<int, kIdxBytes>{});
 }
 
-template <int D, bool kPacked>
+template <int D, int kIdx>
 int dispatch_score16_g(int G, const Attn16& a, int n, int gqa, int n_sub, dim3 grid, hipStream_t s) {
   switch (G) {
-    case 1: launch_score16<D, 1, kPacked>(a, n, gqa, n_sub, grid, s); break;
-    case 2: launch_score16<D, 2, kPacked>(a, n, gqa, n_sub, grid, s); break;
-    default: launch_score16<D, 4, kPacked>(a, n, gqa, n_sub, grid, s); break;
+    case 1: polar16_score_kernel<D, 1, kIdx><<<grid, 256, 0, s>>>(a, n, gqa, n_sub); break;
+    case 2: polar16_score_kernel<D, 2, kIdx><<<grid, 256, 0, s>>>(a, n, gqa, n_sub); break;
+    default: polar16_score_kernel<D, 4, kIdx><<<grid, 256, 0, s>>>(a, n, gqa, n_sub); break;
   }
   TQ_CHECK_LAUNCH("polar16_score_kernel");
   return TQ_OK;
 }
 
-template <int D, bool kPacked>
+template <int D, int kIdx>
 int dispatch_sdpa16_g(int G, const SdpaParams& p, const Attn16& a, dim3 grid, hipStream_t s) {
+  constexpr int NT = kSdpa16Waves * 64;
   switch (G) {
-    case 1: polar16_sdpa_kernel<D, 1, kPacked><<<grid, 256, 0, s>>>(p, a); break;
-    case 2: polar16_sdpa_kernel<D, 2, kPacked><<<grid, 256, 0, s>>>(p, a); break;
-    default: polar16_sdpa_kernel<D, 4, kPacked><<<grid, 256, 0, s>>>(p, a); break;
+    case 1: polar16_sdpa_kernel<D, 1, kIdx><<<grid, NT, 0, s>>>(p, a); break;
+    case 2: polar16_sdpa_kernel<D, 2, kIdx><<<grid, NT, 0, s>>>(p, a); break;
+    default: polar16_sdpa_kernel<D, 4, kIdx><<<grid, NT, 0, s>>>(p, a); break;
   }
   TQ_CHECK_LAUNCH("polar16_sdpa_kernel");
   return TQ_OK;
@@ -2020,8 +2179,7 @@ int attn16_setup(Attn16& a, const float* q, const uint8_t* i1, const uint8_t* i2
   return TQ_OK;
 }
 
-int score16_common(Attn16& a, int Hq, int Hkv, int n, float scale, float* scores, bool packed,
-                   void* stream, const char* fn) {
+int score16_common(Attn16& a, int Hq, int Hkv, int n, float scale, float* scores, void* stream, const char* fn) {
   TQ_CHECK_ARG(scores != nullptr, "%s: scores is NULL", fn);
   TQ_CHECK_ARG(std::isfinite(scale), "%s: scale must be finite", fn);
   if (n == 0) return TQ_OK;
@@ -2029,16 +2187,16 @@ int score16_common(Attn16& a, int Hq, int Hkv, int n, float scale, float* scores
   a.scores = scores;
   a.qscale = scale;
   TQ_CHECK_ARG(Hkv * n_sub <= 65535, "%s: too many heads", fn);
-  dim3 grid((n + 1023) / 1024, Hkv * n_sub);
+  dim3 grid((n + kScoreKeys - 1) / kScoreKeys, Hkv * n_sub);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (a.D) {
-    case 64: return packed ? dispatch_score16_g<64, true>(G, a, n, gqa, n_sub, grid, s)
-                           : dispatch_score16_g<64, false>(G, a, n, gqa, n_sub, grid, s);
-    case 128: return packed ? dispatch_score16_g<128, true>(G, a, n, gqa, n_sub, grid, s)
-                            : dispatch_score16_g<128, false>(G, a, n, gqa, n_sub, grid, s);
-    default: return packed ? dispatch_score16_g<256, true>(G, a, n, gqa, n_sub, grid, s)
-                           : dispatch_score16_g<256, false>(G, a, n, gqa, n_sub, grid, s);
-  }
+  return with_idx_layout(a, [&](auto idx) {
+    constexpr int kIdx = decltype(idx)::value;
+    switch (a.D) {
+      case 64: return dispatch_score16_g<64, kIdx>(G, a, n, gqa, n_sub, grid, s);
+      case 128: return dispatch_score16_g<128, kIdx>(G, a, n, gqa, n_sub, grid, s);
+      default: return dispatch_score16_g<256, kIdx>(G, a, n, gqa, n_sub, grid, s);
+    }
+  });
 }
 
 size_t polar_ws_size(int Hq, int Hkv, int D, int max_len, int max_g) {
@@ -2158,7 +2316,7 @@ int tq_compressed_score(const float* q, int num_heads, const uint8_t* idx_l1, co
                         radii, codebooks, n_codebook, false, num_heads, num_kv_heads, n_keys, dim,
                         block_size, fn);
   if (st != TQ_OK) return st;
-  return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, false, stream, fn);
+  return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, stream, fn);
 }
 
 int tq_compressed_score_packed(const float* q, int num_heads, const uint32_t* packed_l1,
@@ -2173,7 +2331,7 @@ int tq_compressed_score_packed(const float* q, int num_heads, const uint32_t* pa
                         packed_l4, radii, codebooks, n_codebook, true, num_heads, num_kv_heads,
                         n_keys, dim, block_size, fn);
   if (st != TQ_OK) return st;
-  return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, true, stream, fn);
+  return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, stream, fn);
 }
 
 size_t tq_compressed_sdpa_workspace_size(int num_heads, int num_kv_heads, int dim, int max_n_keys) {
@@ -2202,11 +2360,18 @@ int tq_compressed_sdpa(const float* q, int num_heads, const uint8_t* idx_l1, con
   a.values = values;
   a.qscale = scale * kLog2e;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (dim) {
-    case 64: return dispatch_sdpa16_g<64, false>(G, p, a, grid, s);
-    case 128: return dispatch_sdpa16_g<128, false>(G, p, a, grid, s);
-    default: return dispatch_sdpa16_g<256, false>(G, p, a, grid, s);
-  }
+  return with_idx_layout(a, [&](auto idx) {
+    constexpr int kIdx = decltype(idx)::value;
+    if constexpr (kIdx == kIdxPacked) {
+      return static_cast<int>(TQ_ERR_UNSUPPORTED);  // no packed entry point
+    } else {
+      switch (dim) {
+        case 64: return dispatch_sdpa16_g<64, kIdx>(G, p, a, grid, s);
+        case 128: return dispatch_sdpa16_g<128, kIdx>(G, p, a, grid, s);
+        default: return dispatch_sdpa16_g<256, kIdx>(G, p, a, grid, s);
+      }
+    }
+  });
 }
 
 int tq_polar_rotate(const float* x, const float* precondition, int64_t rows, int dim, float* y,

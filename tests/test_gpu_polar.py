@@ -174,6 +174,30 @@ def test_compressed_sdpa(pq, D, Hq, Hkv, N):
     assert_close(got, ref, f"compressed_sdpa D{D} Hq{Hq} Hkv{Hkv} N{N}")
 
 
+@pytest.mark.parametrize("D,Hq,Hkv,N", [(64, 4, 4, 65), (64, 8, 2, 513), (128, 2, 2, 31), (128, 4, 2, 1025),
+                                        (128, 8, 2, 64), (256, 3, 3, 17), (256, 4, 2, 511), (256, 4, 1, 4096)])
+def test_compressed_tiles_and_odd_addresses(pq, D, Hq, Hkv, N):
+    """Key counts at the edges of the 64 / 32 / 16-key tiles and of the
+    splits, for 1, 2 and 4 heads a key set, with the unpacked index arrays at
+    aligned and at odd addresses (loaded a level at a time and by bytes)."""
+    rng = np.random.default_rng(11 * D + Hq + N)
+    cbs = rand_codebooks(rng, packed=False)
+    k = rng.standard_normal((Hkv * N, D)).astype(f32)
+    v = rng.standard_normal((Hkv * N, D)).astype(f32)
+    q = rng.standard_normal((Hq, D)).astype(f32)
+    idx = PQ.polar_quantize(k, None, cbs)
+    gqa, scale = Hq // Hkv, 0.3
+    ref_s = PQ.compressed_score(q, *idx, cbs, N, scale, gqa=gqa)
+    ref_o = PQ.compressed_sdpa(q, *idx, cbs, v, scale, gqa=gqa)
+    for off in (0, 1):
+        di = [dev(np.concatenate([np.zeros(off, np.uint8), a]))[off:] for a in idx[:4]] + [dev(idx[4])]
+        args = [dev(q), *di, *[dev(c) for c in cbs]]
+        got = host(pq.compressed_score(*args, N, scale=scale, num_kv_heads=Hkv))
+        assert np.max(np.abs(got - ref_s)) < SCORE_ATOL, off
+        got = host(pq.compressed_sdpa(*args, dev(v), scale=scale, num_kv_heads=Hkv))
+        assert_close(got, ref_o, f"compressed_sdpa D{D} Hq{Hq} Hkv{Hkv} N{N} offset {off}")
+
+
 # --------------------------------------------------------------- polar7 --------
 
 def p7_inputs(seed, n, rot=True):
