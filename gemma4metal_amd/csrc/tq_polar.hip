@@ -393,28 +393,16 @@ struct Keys16 {
   const uint16_t* radii;
 };
 
-// indices of one 16-value block
-template <bool kPacked>
-__device__ __forceinline__ void load_block_idx(const Keys16& k, int64_t gb, int k1[8], int k2[4],
-                                               int k3[2], int& k4) {
-  if constexpr (kPacked) {
-    const uint32_t w = k.p1[gb], b2 = k.p2[gb], b3 = k.p3[gb];
+// unpacked indices of one 16-value block
+__device__ __forceinline__ void load_block_idx(const Keys16& k, int64_t gb, int k1[8], int k2[4], int k3[2],
+                                               int& k4) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) k1[j] = (w >> (4 * j)) & 0xF;
+  for (int j = 0; j < 8; ++j) k1[j] = k.i1[gb * 8 + j];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) k2[j] = (b2 >> (2 * j)) & 0x3;
+  for (int j = 0; j < 4; ++j) k2[j] = k.i2[gb * 4 + j];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) k3[j] = (b3 >> (2 * j)) & 0x3;
-    k4 = k.p4[gb] & 0x3;
-  } else {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) k1[j] = k.i1[gb * 8 + j];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) k2[j] = k.i2[gb * 4 + j];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) k3[j] = k.i3[gb * 2 + j];
-    k4 = k.i4[gb];
-  }
+  for (int j = 0; j < 2; ++j) k3[j] = k.i3[gb * 2 + j];
+  k4 = k.i4[gb];
 }
 
 // Top-down decode of one block with the (cos, sin) tables cst[level][256]
@@ -458,21 +446,16 @@ struct CsSource {
   int off[4];
 };
 
+__device__ __forceinline__ float2 cs_entry(const CsSource& s, int l, int c) {
+  if (c >= s.ncb[l]) return make_float2(0.0f, 0.0f);
+  if (s.cs) return make_float2(s.cs[2 * (s.off[l] + c)], s.cs[2 * (s.off[l] + c) + 1]);
+  const float th = s.cb[s.off[l] + c];
+  return make_float2(cosf(th), sinf(th));
+}
+
 template <int NT>
 __device__ __forceinline__ void fill_cs_tables(float2* cst, const CsSource& s) {
-  for (int i = threadIdx.x; i < 1024; i += NT) {
-    const int l = i >> 8, c = i & 255;
-    float2 v = make_float2(0.0f, 0.0f);
-    if (c < s.ncb[l]) {
-      if (s.cs) {
-        v = make_float2(s.cs[2 * (s.off[l] + c)], s.cs[2 * (s.off[l] + c) + 1]);
-      } else {
-        const float th = s.cb[s.off[l] + c];
-        v = make_float2(cosf(th), sinf(th));
-      }
-    }
-    cst[i] = v;
-  }
+  for (int i = threadIdx.x; i < 1024; i += NT) cst[i] = cs_entry(s, i >> 8, i & 255);
 }
 
 struct Dec16Params {
@@ -485,7 +468,49 @@ struct Dec16Params {
   int rows;
 };
 
-template <bool kPacked>
+// Packed blocks without a rotation, any D: kDecQuads quarter blocks a thread.
+// Four lanes decode a block, four values each, so a wave's stores are
+// contiguous (a thread per block stored 16 bytes every 64, four times).  Only
+// the codebook entries that a packed index can name are tabled.
+// What bounds it: the fp32 output.  32,768 vectors of 128: 9.8 us before.
+constexpr int kDecQuads = 4;
+
+__global__ __launch_bounds__(256) void polar_decode16_packed_kernel(Dec16Params p, int64_t quads) {
+  __shared__ float2 cst[4][16];
+  if (threadIdx.x < 64) {
+    const int l = threadIdx.x >> 4, c = threadIdx.x & 15;
+    cst[l][c] = cs_entry(p.src, l, c);
+  }
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * (256 * kDecQuads) + threadIdx.x;
+  uint32_t w1[kDecQuads], w2[kDecQuads], w3[kDecQuads], w4[kDecQuads];
+  uint16_t rad[kDecQuads];
+#pragma unroll
+  for (int i = 0; i < kDecQuads; ++i) {
+    const int64_t gb = min(t0 + 256 * i, quads - 1) >> 2;
+    w1[i] = p.k.p1[gb];
+    w2[i] = p.k.p2[gb];
+    w3[i] = p.k.p3[gb];
+    w4[i] = p.k.p4[gb];
+    rad[i] = p.k.radii[gb];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kDecQuads; ++i) {
+    const int64_t t = t0 + 256 * i;
+    if (t >= quads) break;
+    const int b = static_cast<int>(t & 3);  // quarter: level-2 pair b, level-1 pairs 2b and 2b + 1
+    const float2 c4 = cst[3][w4[i] & 0x3];
+    const float2 c3 = cst[2][(w3[i] >> (2 * (b >> 1))) & 0x3];
+    const float2 c2 = cst[1][(w2[i] >> (2 * b)) & 0x3];
+    const float2 a = cst[0][(w1[i] >> (8 * b)) & 0xF], c = cst[0][(w1[i] >> (8 * b + 4)) & 0xF];
+    float v = __half2float(__ushort_as_half(rad[i]));
+    v *= b & 2 ? c4.y : c4.x;
+    v *= b & 1 ? c3.y : c3.x;
+    const float v0 = v * c2.x, v1 = v * c2.y;
+    *reinterpret_cast<float4*>(p.out + 4 * t) = make_float4(v0 * a.x, v0 * a.y, v1 * c.x, v1 * c.y);
+  }
+}
+
 __global__ __launch_bounds__(256) void polar_decode16_kernel(Dec16Params p) {
   extern __shared__ __align__(16) float smem[];
   float2* cst = reinterpret_cast<float2*>(smem);  // [4][256]
@@ -498,7 +523,7 @@ __global__ __launch_bounds__(256) void polar_decode16_kernel(Dec16Params p) {
   for (int blk = threadIdx.x; blk < rows * nb; blk += 256) {
     const int64_t gb = row0 * nb + blk;
     int k1[8], k2[4], k3[2], k4;
-    load_block_idx<kPacked>(p.k, gb, k1, k2, k3, k4);
+    load_block_idx(p.k, gb, k1, k2, k3, k4);
     const float rad = __half2float(__ushort_as_half(p.k.radii[gb]));
     float v[16];
     decode_block16(cst, rad, k1, k2, k3, k4, v);
@@ -2108,11 +2133,17 @@ int decode16_common(const Keys16& k, const float* P, const float* codebooks, con
   p.D = D;
   p.rows = std::max(1, 2048 / D);
   if (n == 0) return TQ_OK;
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  if (packed) {  // never with a preconditioner
+    const int64_t quads = n * (D / 4), blocks = (quads + 256 * kDecQuads - 1) / (256 * kDecQuads);
+    TQ_CHECK_ARG(blocks <= (int64_t{1} << 31) - 1, "%s: too many vectors", fn);
+    polar_decode16_packed_kernel<<<static_cast<unsigned>(blocks), 256, 0, hs>>>(p, quads);
+    TQ_CHECK_LAUNCH("polar_decode16_packed_kernel");
+    return TQ_OK;
+  }
   const int64_t grid = (n + p.rows - 1) / p.rows;
   const size_t shm = sizeof(float) * (2048 + static_cast<size_t>(p.rows) * D);
-  hipStream_t hs = static_cast<hipStream_t>(stream);
-  if (packed) polar_decode16_kernel<true><<<static_cast<unsigned>(grid), 256, shm, hs>>>(p);
-  else polar_decode16_kernel<false><<<static_cast<unsigned>(grid), 256, shm, hs>>>(p);
+  polar_decode16_kernel<<<static_cast<unsigned>(grid), 256, shm, hs>>>(p);
   TQ_CHECK_LAUNCH("polar_decode16_kernel");
   return TQ_OK;
 }

@@ -133,6 +133,19 @@ def test_polar_dequantize_variants(pq, D):
     assert np.max(np.abs(ypf - y_ref) / norm) < 1e-5
 
 
+@pytest.mark.parametrize("n,D", [(1, 16), (7, 48), (33, 256), (1025, 64)])
+def test_polar_dequantize_packed_equals_unpacked(pq, n, D):
+    """The packed decoder (four lanes a block) forms the same products in the
+    same order as the unpacked one: equal bit for bit."""
+    rng = np.random.default_rng(n + D)
+    cbs = rand_codebooks(rng, packed=True)
+    idx = PQ.polar_quantize(rng.standard_normal((n, D)).astype(f32), None, cbs)
+    dcb, rad = [dev(c) for c in cbs], dev(idx[4])
+    want = host(pq.polar_dequantize_fast(*[dev(a) for a in idx[:4]], rad, *dcb, D))
+    got = host(pq.polar_dequantize_packed(*[dev(a) for a in PQ.pack_ref(idx[:4])], rad, *dcb, D))
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+
+
 # ------------------------------------------------- reference scores / sdpa ----
 
 @pytest.mark.parametrize("D,Hq,Hkv,N", [(128, 4, 4, 300), (128, 8, 4, 1500), (64, 2, 1, 77),
