@@ -1,27 +1,37 @@
 // Multi-query (prefill) attention over the int4 cache with K/V tiles shared
-// by a workgroup's 64 (query, head) rows -- the engine's prefill fallback
+// by a workgroup's (query, head) rows -- the engine's prefill fallback
 // (engine/gemma4_multilayer.cpp:343-364: dequantize, then masked
 // scaled_dot_product_attention), for head_dim 128 / 256 / 512.
 //
-// A workgroup takes all gqa heads of one kv head for 64 / gqa consecutive
-// queries (16 rows per wave) and streams the union of their key ranges in
-// tiles of 32 keys.  Each tile is dequantized once into LDS:
-//   K as fp16 hi / lo rows [key][dim], V transposed as bf16 hi / lo [dim][slot]
-// (value = s * nibble + b in fp32, split into a rounded high part and the
-// rounded remainder).  V^T slot 8c + 4h + j holds key 16h + 4c + j, so the
-// eight keys lane group c weights (below) are one 16 B read.
-// Per tile and wave, on the matrix cores (l = lane, m = l % 16, c = l / 16):
-//   S^T = K q^T   v_mfma_f32_16x16x32_f16, A = 16 keys x 32 dims of K, B =
-//                 32 dims x 16 rows of q (hi / lo in registers); the three
-//                 products hi*hi + hi*lo + lo*hi keep ~22 bits.  Lane l then
-//                 holds scores of keys 16 tile + 4c + i for row m.
-//   O^T += V^T P^T  v_mfma_f32_16x16x32_bf16, A = 16 dims x 32 keys of V^T,
-//                 B = the bf16 hi / lo split of the weights: key slot j of
-//                 lane group c is key 16 (j / 4) + 4c + j % 4 -- exactly the
-//                 scores lane l already holds, so no exchange is needed.  Lane
-//                 l accumulates dims 16 blk + 4c + i of row m.
-// The online softmax state (max, denominator) of row m lives in the lanes of
-// column m; each row has its own causal / window limit.
+// A workgroup takes RS sets of 16 consecutive (query, head) rows of one kv
+// head and streams the union of their key ranges in tiles of 32 KH keys; wave
+// (rs, kh) runs set rs against keys 32 kh .. 32 kh + 31 of every tile.  Tiles
+// are staged in LDS, double-buffered with one barrier a tile, as centred
+// nibbles n - 8 in fp16 (one AND-OR into 1024 + n and one packed add per two
+// values; exact), in the order of the matrix-core operands, so an A operand is
+// one 16-byte read.  They are never dequantized: the group scales go where
+// they are cheap, and with b' = b + 8 s
+//
+//   S^T[key][row] = sum_g s_k[key][g] ((n - 8) . q)_g + b'_k[key][g] (sum q)_g
+//     (. . q)_g: v_mfma_f32_16x16x32_f16 over the group's 64 dims, A = nibbles
+//     of 16 keys, B = q of 16 rows, scaled by a power of two per row (so bf16
+//     and fp16 queries are exact in one product, fp32 ones 22 bits in two);
+//     one fma per (key, row, group) applies s_k.  The bias term is one more
+//     product a 16-key half: A = biases and scales, B = the group sums of q in
+//     three fp16 parts.
+//   O^T[dim][row] = sum_key (n - 8) (p s_v) + sum_key p b'_v
+//     A = nibbles of 16 dims (one group) x 32 keys, B = p s_v as fp16 high part
+//     and remainder (22 bits).  The powers of two in p's reference keep p s_v
+//     below 2^15 (see m_ref below).  The bias term is summed in fp32.
+// Centred nibbles keep the sums small: the matrix cores' accumulation error
+// grows with the running sum, and with n in place of n - 8 the results were
+// three times as far from 64 bits.
+//
+// Lane l = 16 c + m.  S^T leaves it keys 16 h + 4 c + i (h = 0, 1; i = 0 .. 3) of
+// row m, and the same keys are slots 4 h + i of lane group c in the P.V
+// products: no exchange between the two.  Row r of a P.V product x of group g
+// is dim 64 g + 8 (r % 8) + 2 x + r / 8, the odd ones scaled by 16 (bits 4-7 of
+// a byte are masked in place).
 #include "tq_sdpa_common.h"
 
 #include <type_traits>
@@ -30,643 +40,634 @@ namespace tq {
 namespace {
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kPfWaves = 4;
-constexpr int kPfThreads = 64 * kPfWaves;
-constexpr int kPfRows = 16 * kPfWaves;  // (query, head) rows per workgroup
-constexpr int kPfKeys = 32;             // keys per tile
+// A running reference moves only when a score passes it by this much (log2).
+constexpr float kPfLazy = 12.0f;
+// log2 of the largest p s_v under the reference (fp16 overflows at 2^16).
+constexpr float kPfHead = 3.0f;
 
-template <int D>
+template <int D, bool F32, int NS, int RS>
 struct PfGeom {
-  static constexpr int W = D / 8;                     // packed words per row
-  static constexpr int KSTR = D + 8;                  // K rows in LDS (halves; 16 B pad)
-  static constexpr int KPT = kPfKeys * W / kPfThreads;  // keys per thread in the dequant
-  // V^T rows in LDS (halves): 16 B aligned for the 8-slot reads; a 16-row
-  // read phase at this stride (20 dwords) covers all 64 banks once
-  static constexpr int VSTR = kPfKeys + 8;
-  static constexpr int CH = D / 32;                   // K.q k-steps of 32 dims
-  static constexpr int DB = D / 16;                   // 16-dim output blocks
-  static_assert(KPT == 2 || KPT == 4 || KPT == 8, "D");
-  // D = 512: each lane loads one scale and one bias value of a tile per
-  // tensor, and the dequantization takes the ones its keys need from the
-  // lanes that hold them (ds_bpermute): 4 loads and registers instead of 32
-  // while the tile's words are in flight
-  static constexpr bool LANE_SB = D == 512;
-  static constexpr int NS = LANE_SB ? 1 : KPT;
-  static_assert(!LANE_SB || (W == 64 && KPT == 8 && kPfThreads == 256), "lane roles of the D = 512 scales");
+  using SB = typename std::conditional<F32, float, _Float16>::type;
+  static constexpr int W = D / 8;        // packed words per row
+  static constexpr int NG = D / 64;      // quant groups per row
+  static constexpr int DH = D == 512 ? 2 : 1;  // waves that share a row set's dims
+  static constexpr int KH = 2 / DH;            // 32-key parts of a tile
+  static constexpr int NW_ = NG / DH;          // groups of a wave
+  static constexpr int OW = D / DH;            // dims of a wave
+  static constexpr int TK = 32 * KH, NW = RS * KH * DH, NT = 64 * NW;
+  // 16-byte units of a 16-key slice of K (8 NG operands) and of V^T per 32 keys
+  // (4 NG operands).  An operand is 64 units [c][m]; unit m sits at m ^ swizzle(g),
+  // so that the 16 lanes of a store (of several groups) reach distinct banks, as
+  // those of a read do.
+  static constexpr int KU = 64 * 2 * NG, VU = 64 * 4 * NG;
+  static __device__ __forceinline__ constexpr int kswz(int g) { return (16 / NG) * g; }
+  static __device__ __forceinline__ constexpr int vswz(int g) { return 8 * (g & 1); }
+  static constexpr int UNITS = TK * W / 8;                      // 8-word staging units of K; as many of V
+  static constexpr int NU = (2 * UNITS + NT - 1) / NT;
+  static constexpr int SDW = TK * NG * static_cast<int>(sizeof(SB)) / 4;  // dwords of one scale tensor a tile
+  static constexpr int NSD = (4 * SDW + NT - 1) / NT;
+  static constexpr int OSTR = OW + 2;    // partial output rows (floats): conflict-free 4-byte stores
+  struct Stage {
+    u32x4 k[2][2 * KH * KU];             // [16-key slice][g][s][c][key]: word 8 g + 2 c + s
+    u32x4 v[2][KH * VU];                 // [kh][g][x][c][dim row]: slots 0-7 of lane group c
+    SB sb[2][4][TK * NG];                // k scale, k bias, v scale, v bias
+    v4f xch[DH == 2 ? NW : 1][2 * NS][64];  // score parts of a row set's waves
+  };
+  union Lds {
+    Stage st;
+    float o[NW][16 * NS * OSTR];
+  };
+  static_assert(SDW % 64 == 0 && UNITS % 64 == 0, "wave-uniform staging roles");
 };
 
-// Raw int4 words and the scale / bias (fp16 bits, or fp32 with F32) of
-// this thread's keys of one tile (with LANE_SB: one value of the wave's).
-template <int D, bool F32>
+// One tile's words and scales, in this thread's registers: a unit is 8 words
+// of a key (K), or one word of the 8 keys of a lane group's slots (V).
+template <class Gm>
 struct PfRaw {
-  using SB = typename std::conditional<F32, float, uint16_t>::type;
-  uint32_t kw[PfGeom<D>::KPT], vw[PfGeom<D>::KPT];
-  SB ks[PfGeom<D>::NS], kb[PfGeom<D>::NS], vs[PfGeom<D>::NS], vb[PfGeom<D>::NS];
+  uint32_t w[Gm::NU][8];
+  uint32_t s[Gm::NSD];
 };
 
-// The 32-bit value v of lane src of the wave.
-__device__ __forceinline__ uint32_t pf_from_lane(uint32_t v, int src) {
-  return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(src << 2, static_cast<int>(v)));
+template <class Gm>
+__device__ __forceinline__ void pf_load(PfRaw<Gm>& R, const SdpaParams& p, int64_t row0, int t0, int last) {
+  typedef uint32_t u32_a2 __attribute__((aligned(2)));  // scale tensors may start at any element
+  // rows past the last key repeat it (the mask drops them); the tile's first
+  // row is uniform, so every address is a scalar base and a 32-bit offset
+  auto row = [&](int r) { return static_cast<uint32_t>(min(r, last - t0)); };
+  const int64_t base = row0 + t0;
+#pragma unroll
+  for (int i = 0; i < Gm::NU; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    const int role = __builtin_amdgcn_readfirstlane(e / Gm::UNITS);
+    const int u = e % Gm::UNITS;
+    if (role == 0) {
+      const u32x4* src = reinterpret_cast<const u32x4*>(p.kq + base * Gm::W) + (row(u / Gm::NG) * (Gm::W / 4) + 2 * (u % Gm::NG));
+      const u32x4 a = src[0], b = src[1];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        R.w[i][k] = a[k];
+        R.w[i][4 + k] = b[k];
+      }
+    } else if (role == 1) {
+      const int w = u % Gm::W, kc = u / Gm::W;  // kc = 4 kh + c
+      const int r0 = 32 * (kc >> 2) + 4 * (kc & 3);
+      const uint32_t* src = p.vq + base * Gm::W;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int r = 16 * (j >> 2) + (j & 3);
+        R.w[i][j] = src[row(r0 + r) * Gm::W + w];
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < Gm::NSD; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    const int t = __builtin_amdgcn_readfirstlane(e / Gm::SDW), d = e % Gm::SDW;
+    constexpr int DPR = Gm::SDW / Gm::TK;  // dwords a row
+    const void* src = t == 0 ? p.ks : t == 1 ? p.kb : t == 2 ? p.vs : p.vb;
+    if ((4 * Gm::SDW) % Gm::NT == 0 || t < 4)
+      R.s[i] = (reinterpret_cast<const u32_a2*>(src) + base * DPR)[row(d / DPR) * DPR + d % DPR];
+  }
 }
 
-// The key (0 .. 31 within the tile) held by V^T slot s.
-__device__ __forceinline__ int pf_vkey(int s) { return 16 * ((s >> 2) & 1) + 4 * (s >> 3) + (s & 3); }
+// Nibbles in bits 0-3 (HI: 4-7) of both halves of t as fp16 n - 8 (16 (n - 8)).
+// mask: 0x000F000F (0x00F000F0) in a vector register -- as a literal beside the
+// other one, the AND and the OR are two instructions.
+template <bool HI>
+__device__ __forceinline__ uint32_t pf_centre(uint32_t t, uint32_t mask) {
+  uint32_t b;  // 1024 + n, 1024 + 16 n
+  asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(b) : "v"(t), "v"(mask), "s"(0x64006400u));
+  const _Float16 off = static_cast<_Float16>(HI ? -1152.0f : -1032.0f);
+  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, b) + v2h{off, off});
+}
 
-__device__ __forceinline__ float h2f(uint16_t h) { return __half2float(__ushort_as_half(h)); }
-__device__ __forceinline__ float sbf(uint16_t h) { return h2f(h); }
-__device__ __forceinline__ float sbf(float x) { return x; }
-
-// K and V use different thread roles (word w, keys k0 .. k0 + KPT - 1 for
-// K, V^T slots k0 .. k0 + KPT - 1 for V): K's lanes run along the words of a
-// key (its LDS rows are key-major), V's along the slots of a word (V^T rows
-// are dim-major), so that both LDS stores of a 16-lane phase land in
-// distinct banks.
-// Dequantization of one tile's raw words (this thread's keys) into the LDS
-// images: K as fp16 hi / lo rows, V^T as bf16 hi / lo (value s * n + b in
-// fp32, then its rounded high part and the rounded remainder).
-// Nibbles of a word as floats: the low and high nibble of each byte are
-// masked into bytes of their own and converted by byte (v_cvt_f32_ubyte0-3),
-// so no nibble needs a shift of its own.  Element i of the word is bits 4i.
-__device__ __forceinline__ void pf_nibbles(uint32_t wd, float (&n)[8]) {
-  uint32_t lo = wd & 0x0F0F0F0Fu, hi = (wd >> 4) & 0x0F0F0F0Fu;
-  // opaque: otherwise each byte conversion is folded back into a shift and
-  // a mask of the raw word
-  asm("" : "+v"(lo), "+v"(hi));
+// Into LDS buffer b.  vmax: this thread's largest |V scale| so far.
+template <class Gm>
+__device__ __forceinline__ void pf_store(typename Gm::Stage& S, const PfRaw<Gm>& R, int b, float& vmax) {
+  const uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u;
 #pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    n[2 * b] = static_cast<float>((lo >> (8 * b)) & 0xFFu);
-    n[2 * b + 1] = static_cast<float>((hi >> (8 * b)) & 0xFFu);
+  for (int i = 0; i < Gm::NU; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    const int role = __builtin_amdgcn_readfirstlane(e / Gm::UNITS);
+    const int u = e % Gm::UNITS;
+    if (role == 0) {
+      // word 8 g + 2 c + s: nibbles 0, 4, 1, 5, 2, 6, 3, 7
+      const int r = u / Gm::NG, g = u % Gm::NG;
+      u32x4* d = &S.k[b][(r >> 4) * Gm::KU + 128 * g + ((r & 15) ^ Gm::kswz(g))];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t w = R.w[i][k], h = w >> 8;
+        d[64 * (k & 1) + 16 * (k >> 1)] =
+            u32x4{pf_centre<false>(w, mlo), pf_centre<true>(w, mhi), pf_centre<false>(h, mlo), pf_centre<true>(h, mhi)};
+      }
+    } else if (role == 1) {
+      const int w = u % Gm::W, kc = u / Gm::W;
+      const int g = w >> 3;
+      u32x4* d = &S.v[b][(kc >> 2) * Gm::VU + 256 * g + (kc & 3) * 16 + (w & 7)];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        u32x4 lo, hi;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          // byte x of two keys' words into the low bytes of the halves
+          const uint32_t t = __builtin_amdgcn_perm(R.w[i][2 * q + 1], R.w[i][2 * q], 0x0C040C00u + 0x00010001u * x);
+          lo[q] = pf_centre<false>(t, mlo);
+          hi[q] = pf_centre<true>(t, mhi);
+        }
+        d[64 * x + Gm::vswz(g)] = lo;
+        d[64 * x + (8 ^ Gm::vswz(g))] = hi;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < Gm::NSD; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    const int t = __builtin_amdgcn_readfirstlane(e / Gm::SDW);
+    if ((4 * Gm::SDW) % Gm::NT != 0 && t >= 4) continue;
+    reinterpret_cast<uint32_t*>(S.sb[b][0])[e] = R.s[i];
+    if (t == 2) {
+      if constexpr (sizeof(typename Gm::SB) == 2) {
+        uint32_t mx = 0;
+        asm("v_max3_f16 %0, %0, abs(%1), abs(%1) op_sel:[0,0,1,0]" : "+v"(mx) : "v"(R.s[i]));
+        vmax = fmaxf(vmax, static_cast<float>(__builtin_bit_cast(v2h, mx)[0]));
+      } else {
+        vmax = fmaxf(vmax, fabsf(__uint_as_float(R.s[i])));
+      }
+    }
   }
 }
 
 // The fp16 remainders x0 - h0, x1 - h1 of a pair whose fp16 high parts are
-// packed in hp, as a packed fp16 pair: one mixed-precision fma each (fp16
-// source, fp32 addend, fp16 result into the low / high half).  The
-// remainder is exact in fp32 and rounded once, to fp16.
+// packed in hp, as a packed fp16 pair: one mixed-precision fma each.  The
+// difference is exact in fp32 and rounded once, to fp16.
 __device__ __forceinline__ uint32_t pf_rem_pair(uint32_t hp, float x0, float x1) {
   uint32_t r;
-  asm volatile(
-      "v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
+  asm("v_fma_mixlo_f16 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
       "v_fma_mixhi_f16 %0, %1, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
       : "=&v"(r)
       : "v"(hp), "v"(x0), "v"(x1));
   return r;
 }
 
-template <int D, bool F32>
-__device__ __forceinline__ void pf_dequant(const PfRaw<D, F32>& raw, _Float16* khi, _Float16* klo, __bf16* vthi,
-                                           __bf16* vtlo, int w, int kb0, int wv, int kv0) {
-  using Gm = PfGeom<D>;
-  constexpr int KSTR = Gm::KSTR, VSTR = Gm::VSTR, KPT = Gm::KPT;
-  typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-  // scale and bias of this thread's K keys and V slots
-  float kS[KPT], kB[KPT], vS[KPT], vB[KPT];
-  if constexpr (Gm::LANE_SB) {
-    // lane s holds K key kb0 + s / 8 of group s % 8, and V key s % 32 of
-    // group wv / 8 (lanes 0-31 and 32-63 hold the wave's two V groups)
-    const int lane = threadIdx.x & 63;
-    uint32_t kp = 0, vp = 0;
-    if constexpr (!F32) {
-      kp = static_cast<uint32_t>(raw.ks[0]) | (static_cast<uint32_t>(raw.kb[0]) << 16);
-      vp = static_cast<uint32_t>(raw.vs[0]) | (static_cast<uint32_t>(raw.vb[0]) << 16);
-    }
-#pragma unroll
-    for (int e = 0; e < KPT; ++e) {
-      const int sk = (e << 3) | (lane >> 3);
-      const int sv = (lane & 32) | (4 * (lane & 3) + (e & 3) + 16 * (e >> 2));
-      if constexpr (F32) {
-        kS[e] = __uint_as_float(pf_from_lane(__float_as_uint(raw.ks[0]), sk));
-        kB[e] = __uint_as_float(pf_from_lane(__float_as_uint(raw.kb[0]), sk));
-        vS[e] = __uint_as_float(pf_from_lane(__float_as_uint(raw.vs[0]), sv));
-        vB[e] = __uint_as_float(pf_from_lane(__float_as_uint(raw.vb[0]), sv));
-      } else {
-        const uint32_t kx = pf_from_lane(kp, sk), vx = pf_from_lane(vp, sv);
-        kS[e] = h2f(static_cast<uint16_t>(kx & 0xFFFFu));
-        kB[e] = h2f(static_cast<uint16_t>(kx >> 16));
-        vS[e] = h2f(static_cast<uint16_t>(vx & 0xFFFFu));
-        vB[e] = h2f(static_cast<uint16_t>(vx >> 16));
-      }
-    }
-  } else {
-#pragma unroll
-    for (int e = 0; e < KPT; ++e) {
-      kS[e] = sbf(raw.ks[e]);
-      kB[e] = sbf(raw.kb[e]);
-      vS[e] = sbf(raw.vs[e]);
-      vB[e] = sbf(raw.vb[e]);
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < KPT; ++e) {
-    const int key = kb0 + e;
-    const float ks = kS[e], kbias = kB[e];
-    float n[8];
-    pf_nibbles(raw.kw[e], n);
-    u32x4 kh, kl;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float x0 = fmaf(ks, n[2 * q], kbias), x1 = fmaf(ks, n[2 * q + 1], kbias);
-      const uint32_t hp = __builtin_bit_cast(uint32_t, v2h{static_cast<_Float16>(x0), static_cast<_Float16>(x1)});
-      kh[q] = hp;
-      kl[q] = pf_rem_pair(hp, x0, x1);
-    }
-    *reinterpret_cast<u32x4*>(&khi[key * KSTR + 8 * w]) = kh;
-    *reinterpret_cast<u32x4*>(&klo[key * KSTR + 8 * w]) = kl;
-  }
-  // V^T: the KPT slots of one dim are adjacent -- one 4 / 8 / 16 B store each;
-  // the bf16 high and low parts of a key pair each take one packed conversion
-  typedef __bf16 vkpt __attribute__((ext_vector_type(KPT)));
-  typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-  float nv[KPT][8];
-#pragma unroll
-  for (int e = 0; e < KPT; ++e) pf_nibbles(raw.vw[e], nv[e]);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    vkpt vh, vl;
-#pragma unroll
-    for (int e = 0; e < KPT; e += 2) {
-      const float x0 = fmaf(vS[e], nv[e][j], vB[e]);
-      const float x1 = fmaf(vS[e + 1], nv[e + 1][j], vB[e + 1]);
-      const v2bf_t h = v2bf_t{static_cast<__bf16>(x0), static_cast<__bf16>(x1)};
-      const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-      const float h0 = __uint_as_float(hb << 16), h1 = __uint_as_float(hb & 0xFFFF0000u);
-      const v2bf_t l = v2bf_t{static_cast<__bf16>(x0 - h0), static_cast<__bf16>(x1 - h1)};
-      vh[e] = h[0];
-      vh[e + 1] = h[1];
-      vl[e] = l[0];
-      vl[e + 1] = l[1];
-    }
-    *reinterpret_cast<vkpt*>(&vthi[(8 * wv + j) * VSTR + kv0]) = vh;
-    *reinterpret_cast<vkpt*>(&vtlo[(8 * wv + j) * VSTR + kv0]) = vl;
-  }
-}
-
-template <int D, bool F32>
-__device__ __forceinline__ void pf_load(PfRaw<D, F32>& R, const SdpaParams& p, int64_t row0, int t0,
-                                        int last, int wk, int kk0, int wv, int kv0) {
-  using Gm = PfGeom<D>;
-  using SB = typename PfRaw<D, F32>::SB;
-  const SB* ks = static_cast<const SB*>(p.ks);
-  const SB* kb = static_cast<const SB*>(p.kb);
-  const SB* vs = static_cast<const SB*>(p.vs);
-  const SB* vb = static_cast<const SB*>(p.vb);
-#pragma unroll
-  for (int e = 0; e < Gm::KPT; ++e) {
-    const int64_t rk = row0 + min(t0 + kk0 + e, last);
-    // slots kv0 .. kv0 + KPT - 1 hold keys vkey(kv0) + e % 4 + 16 (e / 4)
-    const int64_t rv = row0 + min(t0 + pf_vkey(kv0) + (e & 3) + 16 * (e >> 2), last);
-    R.kw[e] = __builtin_nontemporal_load(p.kq + rk * Gm::W + wk);
-    R.vw[e] = __builtin_nontemporal_load(p.vq + rv * Gm::W + wv);
-    if constexpr (!Gm::LANE_SB) {
-      R.ks[e] = ks[rk * (D / 64) + (wk >> 3)];
-      R.kb[e] = kb[rk * (D / 64) + (wk >> 3)];
-      R.vs[e] = vs[rv * (D / 64) + (wv >> 3)];
-      R.vb[e] = vb[rv * (D / 64) + (wv >> 3)];
-    }
-  }
-  if constexpr (Gm::LANE_SB) {
-    // K key kk0 + lane / 8 (the wave's keys) of group lane % 8; V key
-    // lane % 32 of group wv / 8
-    const int lane = threadIdx.x & 63;
-    const int64_t rk = row0 + min(t0 + kk0 + (lane >> 3), last);
-    const int64_t rv = row0 + min(t0 + (lane & 31), last);
-    R.ks[0] = ks[rk * (D / 64) + (lane & 7)];
-    R.kb[0] = kb[rk * (D / 64) + (lane & 7)];
-    R.vs[0] = vs[rv * (D / 64) + (wv >> 3)];
-    R.vb[0] = vb[rv * (D / 64) + (wv >> 3)];
-  }
-}
-
-// D = 512: one wave per SIMD (q hi / lo and the O^T accumulators take 256
-// registers), 145 KB of LDS.  With one wave per SIMD nothing hides LDS
-// latency: the products' operands are read four k-steps / blocks ahead,
-// which the scale / bias lane sharing (LANE_SB) leaves registers for.
-template <int D, bool F32>
-__global__ __launch_bounds__(kPfThreads)
-__attribute__((amdgpu_waves_per_eu(D == 512 ? 1 : 2, D == 512 ? 1 : 2)))
-void prefill_int4_kernel(SdpaParams p) {
-  pin_args(p);
-  using Gm = PfGeom<D>;
-  constexpr int W = Gm::W, KSTR = Gm::KSTR, VSTR = Gm::VSTR, CH = Gm::CH, DB = Gm::DB;
-  constexpr int KPT = Gm::KPT;
-  __shared__ __attribute__((aligned(16))) _Float16 khi[kPfKeys * KSTR], klo[kPfKeys * KSTR];
-  __shared__ __attribute__((aligned(16))) __bf16 vthi[D * VSTR], vtlo[D * VSTR];
-  static_assert(CH % 4 == 0 && DB % 4 == 0, "reads are issued four k-steps / blocks ahead");
-
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int m = lane & 15, c = lane >> 4;
-  const int kvh = blockIdx.y;
-  const int gqa = p.gqa;
-  const int qpw = kPfRows / gqa;          // queries per workgroup
-  const int q0 = blockIdx.x * qpw;        // first query of this workgroup
-  const int q_last = min(q0 + qpw, p.nq) - 1;
-  // this lane's row (column m of the wave): query q0 + r / gqa, head r % gqa
-  const int r = 16 * wave + m;
-  const int qo = r / gqa, ho = r - qo * gqa;
-  const bool row_ok = q0 + qo <= q_last;
-  const int qi = min(q0 + qo, q_last);
-  const int pos = p.n + qi;               // absolute position of the query
-  const int W_ = p.window;
-  const int lo = W_ > 0 ? max(0, p.n + q0 + 1 - W_) : 0;  // union of the rows' key ranges
-  const int hi = p.n + q_last + 1;
-  const int last = hi - 1;
-  const int ntile = (hi - lo + kPfKeys - 1) / kPfKeys;
-  const int64_t row0 = static_cast<int64_t>(kvh) * p.cap;
-  const int64_t qrow = static_cast<int64_t>(qi) * p.Hq + kvh * gqa + ho;
-
-  // ---- q of this lane's row: dims 32 ch + 8c .. +7, fp16 hi / lo ----------
-  v8h qh[CH], ql[CH];
-#pragma unroll
-  for (int ch = 0; ch < CH; ++ch) {
-    float f[8];
-    const int64_t e0 = qrow * D + 32 * ch + 8 * c;
-    if (p.q_dtype == TQ_F32) {
-      const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
-      const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
-      f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-    } else {
-      const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
-      const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint16_t a = wd[i] & 0xFFFFu, b = wd[i] >> 16;
-        f[2 * i] = p.q_dtype == TQ_F16 ? h2f(a) : __uint_as_float(static_cast<uint32_t>(a) << 16);
-        f[2 * i + 1] = p.q_dtype == TQ_F16 ? h2f(b) : __uint_as_float(static_cast<uint32_t>(b) << 16);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = f[i] * p.scale_log2;
-      const _Float16 h = static_cast<_Float16>(x);
-      qh[ch][i] = h;
-      ql[ch][i] = static_cast<_Float16>(x - static_cast<float>(h));
-    }
-  }
-
-  // dequant roles: word w of keys kb0 .. kb0 + KPT - 1 of a tile (K), word
-  // wv of V^T slots kv0 .. (V)
-  constexpr int KB = kPfKeys / KPT;  // key blocks per tile
-  const int w = threadIdx.x % W, kb0 = (threadIdx.x / W) * KPT;
-  const int wv = threadIdx.x / KB, kv0 = (threadIdx.x % KB) * KPT;
-  // raw words of the tiles in flight: two (tiles it + 1 and it + 2 load
-  // while tile it is computed), one at D = 512 (registers)
-  constexpr int NB = D == 512 ? 1 : 2;
-  PfRaw<D, F32> rawA, rawB;
-  pf_load<D, F32>(rawA, p, row0, lo, last, w, kb0, wv, kv0);
-  if constexpr (NB == 2) pf_load<D, F32>(rawB, p, row0, min(lo + kPfKeys, last), last, w, kb0, wv, kv0);
-
-  float m_run = -INFINITY, l_run = 0.0f;
-  v4f o[DB];
-#pragma unroll
-  for (int b = 0; b < DB; ++b) o[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-
-  auto tile = [&](PfRaw<D, F32>& raw, int it) {
-    const int t0 = lo + it * kPfKeys;
-    __syncthreads();  // every wave is done with the previous tile's LDS
-    // ---- dequantize this thread's K / V words into LDS ----------------------
-    pf_dequant<D, F32>(raw, khi, klo, vthi, vtlo, w, kb0, wv, kv0);
-    __syncthreads();
-    // the words of tile it + NB go into this buffer while tiles it .. run
-    pf_load<D, F32>(raw, p, row0, min(t0 + NB * kPfKeys, last), last, w, kb0, wv, kv0);
-
-    // ---- S^T = K q^T: two 16-key halves -----------------------------------
-    float sc[8];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-      // K reads of four k-steps issued ahead of their products
-#pragma unroll
-      for (int c0 = 0; c0 < CH; c0 += 4) {
-        v8h ah[4], al[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int off = (16 * half + m) * KSTR + 32 * (c0 + j) + 8 * c;
-          ah[j] = *reinterpret_cast<const v8h*>(&khi[off]);
-          al[j] = *reinterpret_cast<const v8h*>(&klo[off]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], qh[c0 + j], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], ql[c0 + j], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[j], qh[c0 + j], acc, 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + 16 * half + 4 * c + i;
-        const bool keep = row_ok && t <= last && t <= pos && (W_ == 0 || pos - t < W_);
-        sc[4 * half + i] = keep ? acc[i] : -INFINITY;
-      }
-    }
-
-    // ---- online softmax (log2 domain) for row m --------------------------
-    float mt = sc[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) mt = fmaxf(mt, sc[j]);
-    mt = xor16_max(mt);
-    mt = xor32_max(mt);
-    const float m_new = fmaxf(m_run, mt);
-    if (it == 0) {
-      m_run = m_new;  // first tile: nothing accumulated yet
-    } else if (__any(m_new > m_run + kLazyMax)) {
-      const float f = (m_new == m_run) ? 1.0f : merge_factor(m_run, m_new);
-      l_run *= f;
-#pragma unroll
-      for (int b = 0; b < DB; ++b) o[b] *= f;
-      m_run = m_new;
-    }
-    __bf16 ph[8], pl[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float pw = sc[j] == -INFINITY ? 0.0f : fast_exp2(sc[j] - m_run);
-      l_run += pw;
-      ph[j] = static_cast<__bf16>(pw);
-      pl[j] = static_cast<__bf16>(pw - static_cast<float>(ph[j]));
-    }
-    const v8bf bh = v8bf{ph[0], ph[1], ph[2], ph[3], ph[4], ph[5], ph[6], ph[7]};
-    const v8bf bl = v8bf{pl[0], pl[1], pl[2], pl[3], pl[4], pl[5], pl[6], pl[7]};
-
-    // ---- O^T += V^T P^T ------------------------------------------------------
-    // four blocks' V^T reads issued ahead of their products (the compiler
-    // otherwise keeps one block's reads in flight)
-#pragma unroll
-    for (int b0 = 0; b0 < DB; b0 += 4) {
-      v8bf ah[4], al[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int off = (16 * (b0 + j) + m) * VSTR + 8 * c;
-        ah[j] = *reinterpret_cast<const v8bf*>(&vthi[off]);
-        al[j] = *reinterpret_cast<const v8bf*>(&vtlo[off]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int b = b0 + j;
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[j], bh, o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[j], bl, o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[j], bh, o[b], 0, 0, 0);
-      }
-    }
-  };
-  if constexpr (NB == 2) {
-    for (int it = 0; it < ntile; it += 2) {
-      tile(rawA, it);
-      if (it + 1 < ntile) tile(rawB, it + 1);
-    }
-  } else {
-    for (int it = 0; it < ntile; ++it) tile(rawA, it);
-  }
-
-  // ---- normalise and store row m: dims 16 b + 4c + i -------------------------
-  float l_sum = xor16_sum(l_run);
-  l_sum = xor32_sum(l_sum);
-  if (row_ok) {
-    float* out = p.out + qrow * D;
-#pragma unroll
-    for (int b = 0; b < DB; ++b)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[16 * b + 4 * c + i] = normalise(o[b][i], l_sum, 0.0f);
-  }
-}
-
-// ---- wave-specialised variant (D = 128, 256) ------------------------------
-// The kernel above has every wave dequantize its share of a tile, wait at a
-// barrier, then run its matrix-core products: at one workgroup per CU the
-// two phases never overlap.  Here eight waves (two per SIMD) split them:
-// loader waves 0-3 dequantize tile st + 1 into one of two LDS image slots
-// while compute waves 4-7 run tile st from the other; one barrier per step.
-// Both roles pass the same number of barriers (an even number of steps;
-// a step past the last tile dequantizes clamped rows, whose scores the
-// mask drops).  Two slots take 146 KB at D = 256, so D = 512 keeps the
-// kernel above.
-template <int D, bool F32>
-__global__ __launch_bounds__(2 * kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void prefill_int4_ws_kernel(SdpaParams p) {
-  pin_args(p);
-  using Gm = PfGeom<D>;
-  constexpr int W = Gm::W, KSTR = Gm::KSTR, VSTR = Gm::VSTR, CH = Gm::CH, DB = Gm::DB;
-  constexpr int KPT = Gm::KPT;
-  constexpr int KI = kPfKeys * KSTR, VI = D * VSTR;  // halves per K / V^T image
-  static_assert(CH % 4 == 0 && DB % 4 == 0, "reads are issued four k-steps / blocks ahead");
-  __shared__ __attribute__((aligned(16))) _Float16 khi[2][KI], klo[2][KI];
-  __shared__ __attribute__((aligned(16))) __bf16 vthi[2][VI], vtlo[2][VI];
+template <int D, bool F32, int QP, int NS, int RS>
+__device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
+  using Gm = PfGeom<D, F32, NS, RS>;
+  using SB = typename Gm::SB;
+  constexpr int NG = Gm::NG, NWG = Gm::NW_, TK = Gm::TK, KH = Gm::KH, DH = Gm::DH;
+  __shared__ __attribute__((aligned(16))) typename Gm::Lds L;
+  __shared__ uint32_t vmx[2];               // bits of the largest |V scale| up to a buffer's tile
+  __shared__ float ml[Gm::NW][16 * NS], ll[Gm::NW][16 * NS];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const bool loader = wave < kPfWaves;
+  const int rs = wave % RS, kh = wave / RS % KH, dh = wave / (RS * KH);
   const int m = lane & 15, c = lane >> 4;
-  const int kvh = blockIdx.y;
-  const int gqa = p.gqa;
-  const int qpw = kPfRows / gqa;          // queries per workgroup
-  const int q0 = blockIdx.x * qpw;        // first query of this workgroup
-  const int q_last = min(q0 + qpw, p.nq) - 1;
+  // heads vary fastest: with Hkv a multiple or a divisor of 8, an XCD's
+  // workgroups (every eighth) stay on a few heads, whose caches its L2 holds;
+  // the longest key ranges (last queries) start first
+  const int nblk = gridDim.x / p.Hkv;
+  const int kvh = blockIdx.x % p.Hkv, blk = nblk - 1 - static_cast<int>(blockIdx.x / p.Hkv);
+  const int total = p.nq * p.gqa;           // rows of this kv head
+  const int r0 = blk * 16 * NS * RS;        // first row of this workgroup
   const int W_ = p.window;
-  const int lo = W_ > 0 ? max(0, p.n + q0 + 1 - W_) : 0;  // union of the rows' key ranges
-  const int hi = p.n + q_last + 1;
-  const int last = hi - 1;
-  const int ntile = (hi - lo + kPfKeys - 1) / kPfKeys;
-  const int nt2 = ntile + (ntile & 1);
+  const int lo = W_ > 0 ? max(0, p.n + r0 / p.gqa + 1 - W_) : 0;
+  const int last = p.n + (min(r0 + 16 * NS * RS, total) - 1) / p.gqa;  // last key of the last row
+  const int ntile = (last - lo) / TK + 1;
   const int64_t row0 = static_cast<int64_t>(kvh) * p.cap;
 
-  if (loader) {
-    // ================= loaders: raw words -> LDS images ======================
-    const int tid = threadIdx.x;
-    constexpr int KB = kPfKeys / KPT;
-    const int w = tid % W, kb0 = (tid / W) * KPT;
-    const int wv = tid / KB, kv0 = (tid % KB) * KPT;
-    PfRaw<D, F32> rawA, rawB;
-    pf_load<D, F32>(rawA, p, row0, lo, last, w, kb0, wv, kv0);
-    for (int st = 0; st < nt2; st += 2) {
-      pf_load<D, F32>(rawB, p, row0, min(lo + (st + 1) * kPfKeys, last), last, w, kb0, wv, kv0);
-      pf_dequant<D, F32>(rawA, khi[0], klo[0], vthi[0], vtlo[0], w, kb0, wv, kv0);
-      __syncthreads();
-      pf_load<D, F32>(rawA, p, row0, min(lo + (st + 2) * kPfKeys, last), last, w, kb0, wv, kv0);
-      pf_dequant<D, F32>(rawB, khi[1], klo[1], vthi[1], vtlo[1], w, kb0, wv, kv0);
-      __syncthreads();
-    }
-    __syncthreads();  // the compute waves' last tile
-    return;
-  }
+  PfRaw<Gm> raw;
+  pf_load<Gm>(raw, p, row0, lo, last);
 
-  // =================== compute waves: S^T, softmax, O^T ======================
-  // the compute waves bind each step: they win issue over the loader waves
-  // sharing their SIMDs
-  __builtin_amdgcn_s_setprio(3);
-  // this lane's row (column m of its wave): query q0 + r / gqa, head r % gqa
-  const int r = 16 * (wave - kPfWaves) + m;
-  const int qo = r / gqa, ho = r - qo * gqa;
-  const bool row_ok = q0 + qo <= q_last;
-  const int qi = min(q0 + qo, q_last);
-  const int pos = p.n + qi;               // absolute position of the query
-  const int64_t qrow = static_cast<int64_t>(qi) * p.Hq + kvh * gqa + ho;
+  const int rw = r0 + 16 * NS * rs;         // the wave's first row
+  const int pos_lo = p.n + min(rw, total - 1) / p.gqa, pos_hi = p.n + min(rw + 16 * NS - 1, total - 1) / p.gqa;
+  int pos[NS];                              // absolute position of this lane's rows (column m of each set)
 
-  // q of this lane's row: dims 32 ch + 8c .. +7, fp16 hi / lo
-  v8h qh[CH], ql[CH];
+  // ---- q: B operands of k-step s of group g are dims 64 g + 16 c + 8 s + {0, 4,
+  // 1, 5, 2, 6, 3, 7}, times 2^(15 - ex) (the row's largest below 2^15), the odd
+  // ones over 16.  The sign of a negative scale goes into q.
+  v8h qf[NS][2 * NWG][QP], qb[NS];
+  float rf[NS];                             // score = rf * products
 #pragma unroll
-  for (int ch = 0; ch < CH; ++ch) {
-    float f[8];
-    const int64_t e0 = qrow * D + 32 * ch + 8 * c;
-    if (p.q_dtype == TQ_F32) {
-      const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
-      const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
-      f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-    } else {
-      const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
-      const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
+  for (int n = 0; n < NS; ++n) {
+    const int R = min(rw + 16 * n + m, total - 1);
+    const int qi = R / p.gqa;
+    pos[n] = p.n + qi;
+    const int64_t qrow = static_cast<int64_t>(qi) * p.Hq + kvh * p.gqa + (R - qi * p.gqa);
+    float f[2 * NWG][8];
+    float mx = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint16_t a = wd[i] & 0xFFFFu, b = wd[i] >> 16;
-        f[2 * i] = p.q_dtype == TQ_F16 ? h2f(a) : __uint_as_float(static_cast<uint32_t>(a) << 16);
-        f[2 * i + 1] = p.q_dtype == TQ_F16 ? h2f(b) : __uint_as_float(static_cast<uint32_t>(b) << 16);
-      }
-    }
+    for (int j = 0; j < 2 * NWG; ++j) {
+      const int64_t e0 = qrow * D + Gm::OW * dh + 64 * (j >> 1) + 16 * c + 8 * (j & 1);
+      if (p.q_dtype == TQ_F32) {
+        const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
+        const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
+        f[j][0] = a.x; f[j][1] = a.y; f[j][2] = a.z; f[j][3] = a.w;
+        f[j][4] = b.x; f[j][5] = b.y; f[j][6] = b.z; f[j][7] = b.w;
+      } else {
+        const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
+        const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = f[i] * p.scale_log2;
-      const _Float16 h = static_cast<_Float16>(x);
-      qh[ch][i] = h;
-      ql[ch][i] = static_cast<_Float16>(x - static_cast<float>(h));
-    }
-  }
-
-  float m_run = -INFINITY, l_run = 0.0f;
-  v4f o[DB];
-#pragma unroll
-  for (int b = 0; b < DB; ++b) o[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-
-  auto tile = [&](const _Float16* kh_, const _Float16* kl_, const __bf16* vh_, const __bf16* vl_, int it) {
-    const int t0 = lo + it * kPfKeys;
-    // ---- S^T = K q^T: two 16-key halves -----------------------------------
-    float sc[8];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      v4f acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-      // K reads of four k-steps issued ahead of their products
-#pragma unroll
-      for (int c0 = 0; c0 < CH; c0 += 4) {
-        v8h ah[4], al[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int off = (16 * half + m) * KSTR + 32 * (c0 + j) + 8 * c;
-          ah[j] = *reinterpret_cast<const v8h*>(&kh_[off]);
-          al[j] = *reinterpret_cast<const v8h*>(&kl_[off]);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], qh[c0 + j], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[j], ql[c0 + j], acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[j], qh[c0 + j], acc, 0, 0, 0);
+        for (int i = 0; i < 4; ++i) {
+          if (p.q_dtype == TQ_F16) {
+            const v2h h = __builtin_bit_cast(v2h, wd[i]);
+            f[j][2 * i] = static_cast<float>(h[0]);
+            f[j][2 * i + 1] = static_cast<float>(h[1]);
+          } else {
+            f[j][2 * i] = __uint_as_float(wd[i] << 16);
+            f[j][2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
+          }
         }
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + 16 * half + 4 * c + i;
-        const bool keep = row_ok && t <= last && t <= pos && (W_ == 0 || pos - t < W_);
-        sc[4 * half + i] = keep ? acc[i] : -INFINITY;
+      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(f[j][i]));
+    }
+    mx = xor32_max(xor16_max(mx));
+    const int ex = __builtin_amdgcn_frexp_expf(mx);
+    rf[n] = ldexpf(fabsf(p.scale_log2), ex - 15);
+    const bool neg = p.scale_log2 < 0.0f;
+    float qs[NWG];
+#pragma unroll
+    for (int g = 0; g < NWG; ++g) qs[g] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 2 * NWG; ++j) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float x = ldexpf(f[j][i], 15 - ex);
+        x = neg ? -x : x;
+        qs[j >> 1] += x;
+        const int slot = (i & 2) ? 4 + 2 * (i & 1) + (i >> 2) : 2 * (i & 1) + (i >> 2);
+        const float y = (i & 1) ? x * 0.0625f : x;
+        const _Float16 h = static_cast<_Float16>(y);
+        qf[n][j][0][slot] = h;
+        if constexpr (QP == 2) qf[n][j][1][slot] = static_cast<_Float16>(y - static_cast<float>(h));
       }
     }
-    // ---- online softmax (log2 domain) for row m --------------------------
-    float mt = sc[0];
+    // group sums over 512 (|.| < 2^12) in fp16 parts.  fp16 scale/bias: part c
+    // in lane group c (parts 0-2) for the biases, 8 times it for the scales;
+    // fp32: b' = high + low half, high half times parts 0, 1 in lane groups
+    // 0, 1 and low half in 2, 3.
 #pragma unroll
-    for (int j = 1; j < 8; ++j) mt = fmaxf(mt, sc[j]);
-    mt = xor16_max(mt);
-    mt = xor32_max(mt);
-    const float m_new = fmaxf(m_run, mt);
-    if (it == 0) {
-      m_run = m_new;  // first tile: nothing accumulated yet
-    } else if (__any(m_new > m_run + kLazyMax)) {
-      const float f = (m_new == m_run) ? 1.0f : merge_factor(m_run, m_new);
-      l_run *= f;
-#pragma unroll
-      for (int b = 0; b < DB; ++b) o[b] *= f;
-      m_run = m_new;
-    }
-    __bf16 ph[8], pl[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float pw = sc[j] == -INFINITY ? 0.0f : fast_exp2(sc[j] - m_run);
-      l_run += pw;
-      ph[j] = static_cast<__bf16>(pw);
-      pl[j] = static_cast<__bf16>(pw - static_cast<float>(ph[j]));
-    }
-    const v8bf bh = v8bf{ph[0], ph[1], ph[2], ph[3], ph[4], ph[5], ph[6], ph[7]};
-    const v8bf bl = v8bf{pl[0], pl[1], pl[2], pl[3], pl[4], pl[5], pl[6], pl[7]};
-    // ---- O^T += V^T P^T ------------------------------------------------------
-    // four blocks' V^T reads issued ahead of their products (the compiler
-    // otherwise keeps one block's reads in flight)
-#pragma unroll
-    for (int b0 = 0; b0 < DB; b0 += 4) {
-      v8bf ah[4], al[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int off = (16 * (b0 + j) + m) * VSTR + 8 * c;
-        ah[j] = *reinterpret_cast<const v8bf*>(&vh_[off]);
-        al[j] = *reinterpret_cast<const v8bf*>(&vl_[off]);
+    for (int g = 0; g < 4; ++g) {
+      _Float16 pt = static_cast<_Float16>(0.0f);
+      if (g < NWG) {
+        float x = xor32_sum(xor16_sum(qs[g < NWG ? g : 0])) * 0x1p-9f;
+        const _Float16 h0 = static_cast<_Float16>(x);
+        x -= static_cast<float>(h0);
+        const _Float16 h1 = static_cast<_Float16>(x);
+        x -= static_cast<float>(h1);
+        const _Float16 h2 = static_cast<_Float16>(x);
+        if constexpr (F32) pt = (c & 1) ? h1 : h0;
+        else pt = c == 0 ? h0 : c == 1 ? h1 : c == 2 ? h2 : pt;
       }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int b = b0 + j;
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[j], bh, o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah[j], bl, o[b], 0, 0, 0);
-        o[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[j], bh, o[b], 0, 0, 0);
-      }
+      qb[n][g] = pt;
+      qb[n][4 + g] = F32 ? static_cast<_Float16>(0.0f) : pt * static_cast<_Float16>(8.0f);
     }
+  }
+
+  if (threadIdx.x < 2) vmx[threadIdx.x] = 0;
+  __syncthreads();
+  float vmax = 0.0f;
+  auto stage = [&](int b) {
+    pf_store<Gm>(L.st, raw, b, vmax);
+    // each thread's maximum is over all its tiles so far, so the buffer's
+    // value is that of all tiles up to this one, whatever the timing
+    const float wm = wave_max_dpp(vmax);
+    if (lane == 0) atomicMax(&vmx[b], __float_as_uint(wm));
   };
+  stage(0);
+  __syncthreads();
 
-  __syncthreads();  // tile 0 is in slot 0
-  for (int st = 0; st < nt2; st += 2) {
-    tile(khi[0], klo[0], vthi[0], vtlo[0], st);
-    __syncthreads();
-    tile(khi[1], klo[1], vthi[1], vtlo[1], st + 1);
+  // p = 2^(x - m_ref).  m_ref >= x + (exponent of the largest |V scale|) -
+  // kPfHead - kPfLazy for every score so far: p s_v stays below 2^15, and the
+  // remainder's absolute step of 2^-24 is 2^-27 of the weight of the largest.
+  float m_ref[NS], l_run[NS], bsum[NS][NWG];
+  v4f o[NS][4 * NWG];
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    m_ref[n] = -INFINITY;
+    l_run[n] = 0.0f;
+#pragma unroll
+    for (int b = 0; b < 4 * NWG; ++b) o[n][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int g = 0; g < NWG; ++g) bsum[n][g] = 0.0f;
+  }
+  const v4f z = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+
+#pragma unroll 1
+  for (int it = 0; it < ntile; ++it) {
+    const int buf = it & 1;
+    if (it + 1 < ntile) pf_load<Gm>(raw, p, row0, lo + (it + 1) * TK, last);
+    const int t0 = lo + it * TK + 32 * kh;  // this wave's keys t0 .. t0 + 31
+    const bool any = t0 <= pos_hi && (W_ == 0 || pos_lo - (t0 + 31) < W_);  // wave-uniform
+    // this wave's groups
+    const u32x4* ku = L.st.k[buf] + 2 * kh * Gm::KU + 128 * NWG * dh + 16 * c;
+    const u32x4* vu = L.st.v[buf] + kh * Gm::VU + 256 * NWG * dh + 16 * c;
+    const SB* sks = L.st.sb[buf][0] + 32 * kh * NG + NWG * dh;
+    const SB* skb = L.st.sb[buf][1] + 32 * kh * NG + NWG * dh;
+    const SB* svs = L.st.sb[buf][2] + 32 * kh * NG + NWG * dh;
+    const SB* svb = L.st.sb[buf][3] + 32 * kh * NG + NWG * dh;
+
+    float sc[NS][8];
+    if (any) {
+      // ---- S^T: two 16-key halves ------------------------------------------
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        v8h kb;
+        {
+          const SB* br = skb + (16 * h + m) * NG;
+          const SB* sr = sks + (16 * h + m) * NG;
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const _Float16 zero = static_cast<_Float16>(0.0f);
+            if constexpr (F32) {
+              const float bv = g < NWG ? fmaf(8.0f, sr[g < NWG ? g : 0], br[g < NWG ? g : 0]) : 0.0f;
+              const _Float16 bh = static_cast<_Float16>(bv);
+              kb[g] = c < 2 ? bh : static_cast<_Float16>(bv - static_cast<float>(bh));
+              kb[4 + g] = zero;
+            } else {
+              kb[g] = g < NWG ? br[g < NWG ? g : 0] : zero;
+              kb[4 + g] = g < NWG ? sr[g < NWG ? g : 0] : zero;
+            }
+          }
+        }
+        v4f acc[NS][NWG], bt[NS];
+#pragma unroll
+        for (int n = 0; n < NS; ++n) bt[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qb[n], z, 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < NWG; ++g) {
+          const u32x4* kr = ku + h * Gm::KU + 128 * g + (m ^ Gm::kswz(NWG * dh + g));
+          const v8h a0 = __builtin_bit_cast(v8h, kr[0]), a1 = __builtin_bit_cast(v8h, kr[64]);
+#pragma unroll
+          for (int n = 0; n < NS; ++n) {
+            v4f a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g][0], z, 0, 0, 0);
+            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1][0], a, 0, 0, 0);
+            if constexpr (QP == 2) {
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g][1], a, 0, 0, 0);
+              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1][1], a, 0, 0, 0);
+            }
+            acc[n][g] = a;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int n = 0; n < NS; ++n) {
+            float s = bt[n][i] * 512.0f;
+#pragma unroll
+            for (int g = 0; g < NWG; ++g)
+              s = fmaf(static_cast<float>(sks[(16 * h + 4 * c + i) * NG + g]), acc[n][g][i], s);
+            sc[n][4 * h + i] = s * rf[n];
+          }
+      }
+    }
+    if constexpr (DH == 2) {
+      // the other wave's groups: its parts of the same scores
+      if (any) {
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            L.st.xch[wave][2 * n + h][lane] = v4f{sc[n][4 * h], sc[n][4 * h + 1], sc[n][4 * h + 2], sc[n][4 * h + 3]};
+      }
+      __syncthreads();
+      if (any) {
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const v4f x = L.st.xch[wave ^ RS][2 * n + h][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sc[n][4 * h + i] += x[i];
+          }
+      }
+    }
+    if (any) {
+      const bool inside = t0 + 31 <= pos_lo && (W_ == 0 || pos_hi - t0 < W_);  // wave-uniform
+      if (!inside) {
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const int t = t0 + 16 * (j >> 2) + 4 * c + (j & 3);
+            sc[n][j] = t <= pos[n] && (W_ == 0 || pos[n] - t < W_) ? sc[n][j] : -INFINITY;
+          }
+      }
+
+      // ---- online softmax (log2 domain) of rows m ------------------------------
+      const float vm = __uint_as_float(vmx[buf]);
+      const int ve = vm < 0x1p-40f ? -40 : min(__builtin_amdgcn_frexp_expf(vm), 100);
+      const float up = static_cast<float>(ve) - kPfHead;
+      float need[NS];
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        float mt = sc[n][0];
+#pragma unroll
+        for (int j = 1; j < 8; ++j) mt = fmaxf(mt, sc[n][j]);
+        need[n] = xor32_max(xor16_max(mt)) + up;
+      }
+      // (a row with nothing attended yet and nothing here keeps -inf)
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        if (!__any(need[n] > m_ref[n] + kPfLazy)) continue;
+        const float m_new = need[n] > m_ref[n] ? need[n] : m_ref[n];
+        const float f = m_new == m_ref[n] ? 1.0f : merge_factor(m_ref[n], m_new);
+        l_run[n] *= f;
+#pragma unroll
+        for (int b = 0; b < 4 * NWG; ++b) o[n][b] *= f;
+#pragma unroll
+        for (int g = 0; g < NWG; ++g) bsum[n][g] *= f;
+        m_ref[n] = m_new;
+      }
+      float pw[NS][8];
+#pragma unroll
+      for (int n = 0; n < NS; ++n) {
+        // (with nothing attended so far, -inf - -inf would be NaN)
+        const float ms = m_ref[n] == -INFINITY ? 0.0f : m_ref[n];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          pw[n][j] = fast_exp2(sc[n][j] - ms);
+          l_run[n] += pw[n][j];
+        }
+      }
+
+      // ---- O^T += V^T P^T ----------------------------------------------------
+      SB s[8][NWG], bb[8][NWG];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = 16 * (j >> 2) + 4 * c + (j & 3);
+#pragma unroll
+        for (int g = 0; g < NWG; ++g) {
+          s[j][g] = svs[key * NG + g];
+          bb[j][g] = svb[key * NG + g];
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < NWG; ++g) {
+        v8h bh[NS], bl[NS];
+        uint32_t hi[NS][4], lw[NS][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          // b' = b + 8 s
+          const float b0 = fmaf(static_cast<float>(s[2 * q][g]), 8.0f, static_cast<float>(bb[2 * q][g]));
+          const float b1 = fmaf(static_cast<float>(s[2 * q + 1][g]), 8.0f, static_cast<float>(bb[2 * q + 1][g]));
+#pragma unroll
+          for (int n = 0; n < NS; ++n) {
+            const float x0 = fmaf(static_cast<float>(s[2 * q][g]), pw[n][2 * q], 0.0f);
+            const float x1 = fmaf(static_cast<float>(s[2 * q + 1][g]), pw[n][2 * q + 1], 0.0f);
+            hi[n][q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+            lw[n][q] = pf_rem_pair(hi[n][q], x0, x1);
+            bsum[n][g] = fmaf(b0, pw[n][2 * q], bsum[n][g]);
+            bsum[n][g] = fmaf(b1, pw[n][2 * q + 1], bsum[n][g]);
+          }
+        }
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+          bh[n] = __builtin_bit_cast(v8h, u32x4{hi[n][0], hi[n][1], hi[n][2], hi[n][3]});
+          bl[n] = __builtin_bit_cast(v8h, u32x4{lw[n][0], lw[n][1], lw[n][2], lw[n][3]});
+        }
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const v8h a = __builtin_bit_cast(v8h, vu[(4 * g + x) * 64 + (m ^ Gm::vswz(g))]);
+#pragma unroll
+          for (int n = 0; n < NS; ++n) {
+            v4f& acc = o[n][4 * g + x];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh[n], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl[n], acc, 0, 0, 0);
+          }
+        }
+      }
+    }
+    if (it + 1 < ntile) stage(buf ^ 1);
     __syncthreads();
   }
 
-  // ---- normalise and store row m: dims 16 b + 4c + i -------------------------
-  float l_sum = xor16_sum(l_run);
-  l_sum = xor32_sum(l_sum);
-  if (row_ok) {
-    float* out = p.out + qrow * D;
+  // ---- merge of the KH partials of every row, and the output ------------------
+  const float un = c < 2 ? 1.0f : 0.0625f;  // odd nibbles (rows 8-15) were 16 times as large
 #pragma unroll
-    for (int b = 0; b < DB; ++b)
+  for (int n = 0; n < NS; ++n) {
+    const float lt = xor32_sum(xor16_sum(l_run[n]));
+    if (c == 0) {
+      ml[wave][16 * n + m] = m_ref[n];
+      ll[wave][16 * n + m] = lt;
+    }
+    float* orow = L.o[wave] + (16 * n + m) * Gm::OSTR;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) out[16 * b + 4 * c + i] = normalise(o[b][i], l_sum, 0.0f);
+    for (int g = 0; g < NWG; ++g) {
+      const float bg = xor32_sum(xor16_sum(bsum[n][g]));
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          orow[64 * g + 8 * (4 * (c & 1) + i) + 2 * x + (c >> 1)] = fmaf(o[n][4 * g + x][i], un, bg);
+    }
+  }
+  __syncthreads();
+  for (int u = threadIdx.x; u < 16 * NS * RS * (D / 2); u += Gm::NT) {
+    // a wave's 64 units lie in one row and in one wave's dims
+    const int r = __builtin_amdgcn_readfirstlane(u / (D / 2)), d = 2 * (u % (D / 2));
+    const int Ro = r0 + r;
+    if (Ro >= total) break;
+    const int rm = r % (16 * NS), w0 = r / (16 * NS) + RS * KH * (d / Gm::OW);
+    float M = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < KH; ++k) M = fmaxf(M, ml[w0 + RS * k][rm]);
+    float l = 0.0f, x0 = 0.0f, x1 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < KH; ++k) {
+      const int wv = w0 + RS * k;
+      const float f = merge_factor(ml[wv][rm], M);
+      const float2 v = *reinterpret_cast<const float2*>(&L.o[wv][rm * Gm::OSTR + d % Gm::OW]);
+      l = fmaf(ll[wv][rm], f, l);
+      x0 = fmaf(v.x, f, x0);
+      x1 = fmaf(v.y, f, x1);
+    }
+    const int qo = Ro / p.gqa;
+    float* out = p.out + (static_cast<int64_t>(qo) * p.Hq + kvh * p.gqa + (Ro - qo * p.gqa)) * D + d;
+    *reinterpret_cast<float2*>(out) = make_float2(normalise(x0, l, 0.0f), normalise(x1, l, 0.0f));
   }
 }
 
-template <bool F32>
-void launch_tiles(const SdpaParams& p, int D, bool ws, dim3 grid, hipStream_t s) {
-  if (D == 128 && ws) prefill_int4_ws_kernel<128, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
-  else if (D == 256 && ws) prefill_int4_ws_kernel<256, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
-  else if (D == 128) prefill_int4_kernel<128, F32><<<grid, kPfThreads, 0, s>>>(p);
-  else if (D == 256) prefill_int4_kernel<256, F32><<<grid, kPfThreads, 0, s>>>(p);
-  else prefill_int4_kernel<512, F32><<<grid, kPfThreads, 0, s>>>(p);
+// Tiles of 64 keys and two waves a row set, one per 32 keys (D 128 / 256), or
+// of 32 keys and two waves a row set, one per half of the dims (D 512; a tile's
+// two buffers fill the LDS): eight waves, two per SIMD.
+//
+// What bounds it: the VALU (about 430 instructions a wave and 32 keys -- weights
+// times scales and their split 80, exponentials and masks 90, staging 80, bias
+// terms 64, score scales 40 -- against 50 products), busy 60% of the time, the
+// rest being phases of the two waves that do not overlap.  Measured (512 queries
+// after 3,584 keys, whole calls; before: loader waves that dequantized every
+// tile into hi / lo images, whose LDS reads, three products each, bound it):
+//   Hq 32 Hkv 16 D 256, window 1,024: 94.9 -> 67.9 us; without window 275 -> 193
+//   Hq 32 Hkv 4 D 512: 678 -> 404 us;  Hq 16 Hkv 8 D 128: 148 -> 117 us
+// Slower: nibbles expanded by every wave (no operand images; 70 us before they
+// were centred, which would add 128 instructions), two row sets a wave at one
+// wave per SIMD (97 us), operand reads half a tile ahead (68), the two waves of
+// a SIMD staging at opposite ends of a tile (69).
+template <int D, bool F32, int QP, int NS, int RS>
+__global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
+void prefill_int4_ws_kernel(SdpaParams p) {
+  pin_args(p);
+  prefill_rows<D, F32, QP, NS, RS>(p);
+}
+
+template <int D, bool F32, int QP, int NS, int RS>
+__global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
+void prefill_int4_kernel(SdpaParams p) {
+  pin_args(p);
+  prefill_rows<D, F32, QP, NS, RS>(p);
+}
+
+template <int D, bool F32, int QP, int NS, int RS>
+void launch_sets(const SdpaParams& p, unsigned grid, hipStream_t s) {
+  if constexpr (D == 512) prefill_int4_kernel<D, F32, QP, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
+  else prefill_int4_ws_kernel<D, F32, QP, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
+}
+
+constexpr int kPfNS = 1;  // row sets a wave
+
+// 64 rows per workgroup where those fill the CUs, else 32 on four waves (twice
+// the workgroups; 100 queries of Hq 32 Hkv 8 D 128: 24.7 against 26.6 us, and 16
+// rows on two waves, which then stage a whole tile, 29.0).
+template <int D, bool F32, int QP>
+void launch_rows(const SdpaParams& p, hipStream_t s) {
+  constexpr int NR = 16 * kPfNS, RSM = 4 / kPfNS;
+  const int64_t rows = static_cast<int64_t>(p.nq) * p.gqa;
+  const auto grid = [&](int rs) { return static_cast<unsigned>((rows + NR * rs - 1) / (NR * rs) * p.Hkv); };
+  if (grid(RSM) >= static_cast<unsigned>(target_wgs())) launch_sets<D, F32, QP, kPfNS, RSM>(p, grid(RSM), s);
+  else launch_sets<D, F32, QP, kPfNS, 2>(p, grid(2), s);
+}
+
+template <bool F32, int QP>
+void launch_dim(const SdpaParams& p, int D, hipStream_t s) {
+  if (D == 128) launch_rows<128, F32, QP>(p, s);
+  else if (D == 256) launch_rows<256, F32, QP>(p, s);
+  else launch_rows<512, F32, QP>(p, s);
 }
 
 }  // namespace
 
-// Returns -1 when the tile kernel does not serve the shape (the caller then
+// Returns false when the tile kernels do not serve the shape (the caller then
 // runs the split-K decode kernels in prefill mode).
 bool prefill_tiles_serve(int D, int sb_dtype, int gqa) {
   if ((sb_dtype != TQ_F16 && sb_dtype != TQ_F32) || (D != 128 && D != 256 && D != 512)) return false;
-  return gqa >= 1 && gqa <= kPfRows && kPfRows % gqa == 0;
+  return gqa >= 1 && gqa <= 64 && 64 % gqa == 0;
 }
 
 int launch_prefill_tiles(const SdpaParams& p, int D, int sb_dtype, hipStream_t s) {
   if (!prefill_tiles_serve(D, sb_dtype, p.gqa)) return -1;
-  const int qpw = kPfRows / p.gqa;
-  dim3 grid((p.nq + qpw - 1) / qpw, p.Hkv);
-  // TQ_PREFILL_WS=0 selects the one-role kernel at D 128 / 256
-  const bool ws = options().prefill_ws;
-  if (sb_dtype == TQ_F32) launch_tiles<true>(p, D, ws, grid, s);
-  else launch_tiles<false>(p, D, ws, grid, s);
+  const bool two = p.q_dtype == TQ_F32;  // fp32 queries: two products
+  if (sb_dtype == TQ_F32) {
+    if (two) launch_dim<true, 2>(p, D, s);
+    else launch_dim<true, 1>(p, D, s);
+  } else {
+    if (two) launch_dim<false, 2>(p, D, s);
+    else launch_dim<false, 1>(p, D, s);
+  }
   TQ_CHECK_LAUNCH("prefill_int4_kernel");
   return TQ_OK;
 }

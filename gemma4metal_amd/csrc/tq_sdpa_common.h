@@ -612,13 +612,11 @@ WsLayout ws_layout(int batch, int Hq, int D, int max_splits);
 //   TQ_SDPA_IMPL=valu       the VALU decode kernel for every shape
 //   TQ_SDPA_CHUNK=n         keys per split (overrides the planner)
 //   TQ_PREFILL_IMPL=splitk  prefill on the split-K decode kernels
-//   TQ_PREFILL_WS=0         the one-role prefill tile kernel
 //   TQ_HC_IMPL=1            the one-wave D=512 heads-as-columns kernel
 struct Options {
   bool sdpa_valu;
   int sdpa_chunk;
   bool prefill_splitk;
-  bool prefill_ws;
   bool hc_one;
 };
 Options options();
@@ -660,8 +658,8 @@ int launch_sdpa_mfma(const SdpaParams& p, int D, int G, int sb_dtype, dim3 grid,
 // scale/bias: tq_sdpa_hc.hip.
 int launch_sdpa_hc(const SdpaParams& p, int sb_dtype, dim3 grid, hipStream_t stream);
 // Prefill with K/V tiles shared by 64 (query, head) rows (tq_prefill.hip);
-// -1 when the shape is not served (D other than 128 / 256, fp32 scales,
-// gqa not dividing 64).
+// -1 when the shape is not served (D other than 128 / 256 / 512, gqa not
+// dividing 64).
 int launch_prefill_tiles(const SdpaParams& p, int D, int sb_dtype, hipStream_t stream);
 // Merge of the split partials of a launch with ext_merge = 1 (batch b of
 // grid.y): tq_sdpa_hc.hip.

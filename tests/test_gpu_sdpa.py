@@ -538,6 +538,40 @@ def test_sdpa_prefill_tile_kernel(gpu, Hq, Hkv, D, S, prior, W, qdt, sb):
     assert_close(host(out), ref, f"tiles S{S} prior{prior} W{W} D{D} gqa{Hq // Hkv}")
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,S,prior,W,scale,qmag,vmag", [
+    (32, 16, 256, 513, 31, 0, 1.0, 1.0, 1.0),        # 64 rows a workgroup, one row set past the last
+    (16, 16, 128, 517, 0, 33, -0.5, 1.0, 1.0),       # negative scale, window across tile edges
+    (64, 1, 128, 65, 700, 0, 1.0, 1.0, 300.0),       # GQA 64: a query's rows over four row sets; large V
+    (32, 2, 512, 67, 29, 40, 1.0, 1.0, 1e-3),        # D 512, GQA 16, small V, 32 rows a workgroup
+    (8, 4, 256, 64, 0, 0, 1e-4, 1e4, 1.0),           # large queries (normed entries < 6: inside fp16, < 65504)
+    (8, 4, 512, 300, 5, 0, 30.0, 1e-3, 1.0),
+    (2, 1, 256, 90, 1, 1, 0.0, 1.0, 1.0),            # window 1, scale 0
+])
+@pytest.mark.parametrize("qdt,sb", [("bf16", "f16"), ("f32", "f32"), ("f32", "f16"), ("f16", "f32")])
+def test_sdpa_prefill_rows_edges(gpu, Hq, Hkv, D, S, prior, W, scale, qmag, vmag, qdt, sb):
+    """Edges of the row sets (16), workgroups (32 / 64 rows), tiles (32 / 64
+    keys) and value ranges of the prefill tile kernel.  Its operands carry 22
+    bits and its sums fp32: with a score of magnitude x, an output is off by
+    about x 2^-22 of itself, so 2e-5 covers |x| up to 80."""
+    rng = np.random.default_rng(S * 3 + prior + Hq + D)
+    n = prior + S
+    k = O.rms_norm(rng.standard_normal((Hkv, n, D)).astype(np.float32))
+    v = (rng.standard_normal((Hkv, n, D)) * vmag).astype(np.float32)
+    c = O.quantize_int4(k, sb) + O.quantize_int4(v, sb)
+    q32 = O.rms_norm(rng.standard_normal((S, Hq, D)).astype(np.float32)) * np.float32(qmag)
+    if qdt == "bf16":
+        bits = O.f32_to_bf16_bits(q32)
+        qd, qv = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16), O.bf16_bits_to_f32(bits)
+    else:
+        qn = q32.astype(np.float16) if qdt == "f16" else q32
+        qd, qv = torch.from_numpy(qn).cuda(), qn.astype(np.float32)
+    got = host(gpu.sdpa_int4_prefill(qd, *[dev(a) for a in c], prior, Hq // Hkv, scale, W)).astype(np.float64)
+    ref = np.asarray(O.sdpa_int4_prefill(qv, *c, prior, Hq // Hkv, scale, W), np.float64)
+    assert np.isfinite(got).all()
+    rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert rel < 2e-5, rel
+
+
 @pytest.mark.parametrize("Hq,Hkv,L,W", [(32, 4, 5000, 0), (32, 4, 3001, 1024), (16, 2, 129, 0)])
 def test_d512_one_wave_and_wave_specialised_kernels_agree(gpu, tq_env, Hq, Hkv, L, W):
     """The two D=512 GQA-8 kernels (TQ_HC_IMPL=1 selects the one-wave one)
