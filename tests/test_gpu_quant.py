@@ -49,6 +49,29 @@ def test_quantize_dims(gpu, D):
     assert np.array_equal(host(wq), rq) and np.array_equal(host(s), rs) and np.array_equal(host(b), rb)
 
 
+@pytest.mark.parametrize("mode", ["mlx", "minmax"])
+@pytest.mark.parametrize("mag", [1e-30, 1e-6, 1.0, 1e20, 3e36])
+def test_quantize_near_half_bit_exact(gpu, mode, mag):
+    """Values at and within a few ulp of half-integer quotients (where the
+    kernel divides instead of using the reciprocal), over the float range."""
+    rng = np.random.default_rng(int(np.log10(mag)) + 100)
+    rows = 2000
+    lo = rng.uniform(-4, 3, (rows, 1))
+    step = rng.uniform(0.01, 0.5, (rows, 1))
+    x = lo + step * (rng.integers(0, 15, (rows, 64)) + 0.5)
+    x[:, 0], x[:, 1] = lo[:, 0], lo[:, 0] + 15 * step[:, 0]
+    x[::3] = np.round(x[::3] * 8) / 8            # exact ties
+    x = (x * mag).astype(np.float32)
+    # a few ulp off (not the zeros: those bit patterns are NaN, whose order in
+    # a maximum the rule does not define)
+    x.view(np.int32)[:] += np.where(x != 0, rng.integers(-3, 4, x.shape), 0).astype(np.int32)
+    wq, s, b = gpu.quantize(dev(x), scale_dtype=torch.float32, mode=mode)
+    rq, rs, rb = O.quantize_int4(x, "f32", mode)
+    # by value: the minimum of -0 and 0 is either
+    assert np.array_equal(host(s), rs) and np.array_equal(host(b), rb)
+    assert np.array_equal(host(wq), rq)
+
+
 def test_dequantize_matches(gpu):
     rng = np.random.default_rng(5)
     x = rng.standard_normal((64, 256)).astype(np.float32)
