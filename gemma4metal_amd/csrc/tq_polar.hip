@@ -130,9 +130,8 @@ struct Enc16Params {
   int64_t n;       // vectors
   int D;
   int rows;        // vectors per workgroup
-  const float* cb; // concatenated codebooks of levels 1..4
+  const float* cb[4];  // codebooks of levels 1..4
   int ncb[4];
-  int cb_off[4];
   uint8_t *i1, *i2, *i3, *i4;  // unpacked outputs
   uint32_t* p1;                 // packed outputs
   uint8_t *p2, *p3, *p4;
@@ -224,7 +223,7 @@ __device__ __forceinline__ void fill_codebooks(float* cbs, const Enc16Params& p)
 #pragma unroll
   for (int l = 0; l < 4; ++l)
     for (int c = threadIdx.x; c < ((p.ncb[l] + 3) & ~3); c += NT)
-      cbs[256 * l + c] = c < p.ncb[l] ? p.cb[p.cb_off[l] + c] : INFINITY;
+      cbs[256 * l + c] = c < p.ncb[l] ? p.cb[l][c] : INFINITY;
 }
 
 // Encodes one 16-value block (global block gb) and stores its indices and radius.
@@ -440,16 +439,15 @@ __device__ __forceinline__ void decode_block16(const float2* cst, float rad, con
 // given (the reference's "_fast" variants), else cos/sin of the codebook
 // angles (zero beyond each codebook's size, so any u8 index stays in range).
 struct CsSource {
-  const float* cb;   // concatenated codebooks, or null
-  const float* cs;   // concatenated (cos, sin) pairs, or null
+  const float* cb[4];  // codebooks, or null
+  const float* cs[4];  // (cos, sin) pairs, or null
   int ncb[4];
-  int off[4];
 };
 
 __device__ __forceinline__ float2 cs_entry(const CsSource& s, int l, int c) {
   if (c >= s.ncb[l]) return make_float2(0.0f, 0.0f);
-  if (s.cs) return make_float2(s.cs[2 * (s.off[l] + c)], s.cs[2 * (s.off[l] + c) + 1]);
-  const float th = s.cb[s.off[l] + c];
+  if (s.cs[l]) return make_float2(s.cs[l][2 * c], s.cs[l][2 * c + 1]);
+  const float th = s.cb[l][c];
   return make_float2(cosf(th), sinf(th));
 }
 
@@ -2024,19 +2022,40 @@ int polar_splits_bound(int L, int64_t groups) {
   return static_cast<int>(std::max<int64_t>(1, std::min({by_len, by_wgs, int64_t{kMaxSplits}})));
 }
 
-int check_codebooks(const float* cb, const int* ncb, int max_first, int max_rest, CsSource& s,
+// The four levels' tables of a call: one device array with the levels back to
+// back, or an array of their own per level (no copy to join them).
+struct Books {
+  const float* p[4];
+  bool null() const { return !(p[0] && p[1] && p[2] && p[3]); }
+};
+
+Books books_joined(const float* base, const int* sizes, int width) {
+  Books b{};
+  if (!base || !sizes) return b;
+  for (int l = 0; l < 4; ++l) {
+    b.p[l] = base;
+    base += static_cast<int64_t>(width) * sizes[l];
+  }
+  return b;
+}
+
+Books books_of(const float* const* levels) {
+  Books b{};
+  if (levels)
+    for (int l = 0; l < 4; ++l) b.p[l] = levels[l];
+  return b;
+}
+
+int check_codebooks(const Books& cb, const int* ncb, int max_first, int max_rest, CsSource& s,
                      const char* fn) {
   TQ_CHECK_ARG(ncb != nullptr, "%s: n_codebook is NULL", fn);
-  int off = 0;
   for (int l = 0; l < 4; ++l) {
     const int mx = l == 0 ? max_first : max_rest;
     TQ_CHECK_ARG(ncb[l] >= 1 && ncb[l] <= mx, "%s: codebook %d size %d not in [1, %d]", fn, l + 1,
                  ncb[l], mx);
     s.ncb[l] = ncb[l];
-    s.off[l] = off;
-    off += ncb[l];
+    s.cb[l] = cb.p[l];
   }
-  s.cb = cb;
   return TQ_OK;
 }
 
@@ -2081,7 +2100,7 @@ int launch_encode16(const Enc16Params& p, hipStream_t s, const char* fn) {
   return TQ_OK;
 }
 
-int encode16_common(const float* x, const float* P, const float* codebooks, const int* n_codebook,
+int encode16_common(const float* x, const float* P, const Books& codebooks, const int* n_codebook,
                     int64_t n, int D, int block_size, bool packed, uint8_t* i1, uint8_t* i2,
                     uint8_t* i3, uint8_t* i4, uint32_t* p1, uint8_t* p2, uint8_t* p3, uint8_t* p4,
                     uint16_t* radii, void* stream, const char* fn) {
@@ -2091,7 +2110,7 @@ int encode16_common(const float* x, const float* P, const float* codebooks, cons
   }
   TQ_CHECK_ARG(D >= 16 && D <= 2048 && D % 16 == 0, "%s: dim must be a multiple of 16 in [16, 2048]", fn);
   TQ_CHECK_ARG(n >= 0, "%s: n_vectors must be >= 0", fn);
-  TQ_CHECK_ARG(x && codebooks && radii, "%s: null pointer", fn);
+  TQ_CHECK_ARG(x && radii && (!codebooks.null() || !n_codebook), "%s: null pointer", fn);
   CsSource s{};
   const int st = check_codebooks(codebooks, n_codebook, packed ? 16 : 256, packed ? 4 : 256, s, fn);
   if (st != TQ_OK) return st;
@@ -2101,8 +2120,10 @@ int encode16_common(const float* x, const float* P, const float* codebooks, cons
   Enc16Params p{};
   p.x = x; p.P = P; p.n = n; p.D = D;
   p.rows = std::max(1, 2048 / D);
-  p.cb = codebooks;
-  for (int l = 0; l < 4; ++l) { p.ncb[l] = s.ncb[l]; p.cb_off[l] = s.off[l]; }
+  for (int l = 0; l < 4; ++l) {
+    p.ncb[l] = s.ncb[l];
+    p.cb[l] = s.cb[l];
+  }
   p.i1 = i1; p.i2 = i2; p.i3 = i3; p.i4 = i4;
   p.p1 = p1; p.p2 = p2; p.p3 = p3; p.p4 = p4;
   p.radii = radii;
@@ -2112,7 +2133,7 @@ int encode16_common(const float* x, const float* P, const float* codebooks, cons
   return packed ? launch_encode16<true>(p, hs, fn) : launch_encode16<false>(p, hs, fn);
 }
 
-int decode16_common(const Keys16& k, const float* P, const float* codebooks, const float* cs_tables,
+int decode16_common(const Keys16& k, const float* P, const Books& codebooks, const Books& cs_tables,
                     const int* n_codebook, int64_t n, int D, int block_size, bool packed, float* out,
                     void* stream, const char* fn) {
   if (block_size != 16) {
@@ -2121,11 +2142,11 @@ int decode16_common(const Keys16& k, const float* P, const float* codebooks, con
   }
   TQ_CHECK_ARG(D >= 16 && D <= 2048 && D % 16 == 0, "%s: dim must be a multiple of 16 in [16, 2048]", fn);
   TQ_CHECK_ARG(n >= 0 && out && k.radii, "%s: null pointer or negative n", fn);
-  TQ_CHECK_ARG(codebooks || cs_tables, "%s: codebooks or cos/sin tables required", fn);
+  TQ_CHECK_ARG(!codebooks.null() || !cs_tables.null() || !n_codebook, "%s: codebooks or cos/sin tables required", fn);
   Dec16Params p{};
   const int st = check_codebooks(codebooks, n_codebook, packed ? 16 : 256, packed ? 4 : 256, p.src, fn);
   if (st != TQ_OK) return st;
-  p.src.cs = cs_tables;
+  for (int l = 0; l < 4; ++l) p.src.cs[l] = cs_tables.p[l];
   p.k = k;
   p.P = P;
   p.out = out;
@@ -2183,7 +2204,7 @@ int dispatch_sdpa16_g(int G, const SdpaParams& p, const Attn16& a, dim3 grid, hi
 
 int attn16_setup(Attn16& a, const float* q, const uint8_t* i1, const uint8_t* i2, const uint8_t* i3,
                  const uint8_t* i4, const uint32_t* p1, const uint8_t* p2, const uint8_t* p3,
-                 const uint8_t* p4, const uint16_t* radii, const float* codebooks,
+                 const uint8_t* p4, const uint16_t* radii, const Books& codebooks,
                  const int* n_codebook, bool packed, int Hq, int Hkv, int n, int D, int block_size,
                  const char* fn) {
   if (block_size != 16) {
@@ -2196,7 +2217,7 @@ int attn16_setup(Attn16& a, const float* q, const uint8_t* i1, const uint8_t* i2
   }
   TQ_CHECK_ARG(Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0, "%s: num_heads must be a multiple of num_kv_heads", fn);
   TQ_CHECK_ARG(n >= 0, "%s: n_keys must be >= 0", fn);
-  TQ_CHECK_ARG(q && radii && codebooks, "%s: null pointer", fn);
+  TQ_CHECK_ARG(q && radii && (!codebooks.null() || !n_codebook), "%s: null pointer", fn);
   if (packed) TQ_CHECK_ARG(p1 && p2 && p3 && p4, "%s: null index array", fn);
   else TQ_CHECK_ARG(i1 && i2 && i3 && i4, "%s: null index array", fn);
   a = Attn16{};
@@ -2292,56 +2313,53 @@ int p7_keys_setup(P7Keys& k, const float* q_tables, const uint32_t* angles, cons
 
 }  // namespace
 
-extern "C" {
+namespace {
 
-int tq_polar_quantize(const float* x, const float* precondition, const float* codebooks,
-                      const int* n_codebook, int64_t n_vectors, int dim, int block_size,
-                      uint8_t* idx_l1, uint8_t* idx_l2, uint8_t* idx_l3, uint8_t* idx_l4,
-                      uint16_t* radii, void* stream) {
+int polar_quantize_impl(const float* x, const float* precondition, const Books& codebooks, const int*
+                        n_codebook, int64_t n_vectors, int dim, int block_size, uint8_t* idx_l1, uint8_t*
+                        idx_l2, uint8_t* idx_l3, uint8_t* idx_l4, uint16_t* radii, void* stream, const char*
+                        fn) {
   return encode16_common(x, precondition, codebooks, n_codebook, n_vectors, dim, block_size, false,
                          idx_l1, idx_l2, idx_l3, idx_l4, nullptr, nullptr, nullptr, nullptr, radii,
-                         stream, "tq_polar_quantize");
+                         stream, fn);
 }
 
-int tq_polar_quantize_packed(const float* x, const float* precondition, const float* codebooks,
-                             const int* n_codebook, int64_t n_vectors, int dim, int block_size,
-                             uint32_t* packed_l1, uint8_t* packed_l2, uint8_t* packed_l3,
-                             uint8_t* packed_l4, uint16_t* radii, void* stream) {
+int polar_quantize_packed_impl(const float* x, const float* precondition, const Books& codebooks, const int*
+                               n_codebook, int64_t n_vectors, int dim, int block_size, uint32_t* packed_l1,
+                               uint8_t* packed_l2, uint8_t* packed_l3, uint8_t* packed_l4, uint16_t* radii,
+                               void* stream, const char* fn) {
   return encode16_common(x, precondition, codebooks, n_codebook, n_vectors, dim, block_size, true,
                          nullptr, nullptr, nullptr, nullptr, packed_l1, packed_l2, packed_l3,
-                         packed_l4, radii, stream, "tq_polar_quantize_packed");
+                         packed_l4, radii, stream, fn);
 }
 
-int tq_polar_dequantize(const uint8_t* idx_l1, const uint8_t* idx_l2, const uint8_t* idx_l3,
-                        const uint8_t* idx_l4, const uint16_t* radii, const float* precondition,
-                        const float* codebooks, const int* n_codebook, int64_t n_vectors, int dim,
-                        int block_size, float* out, void* stream) {
+int polar_dequantize_impl(const uint8_t* idx_l1, const uint8_t* idx_l2, const uint8_t* idx_l3, const uint8_t*
+                          idx_l4, const uint16_t* radii, const float* precondition, const Books& codebooks,
+                          const int* n_codebook, int64_t n_vectors, int dim, int block_size, float* out, void*
+                          stream, const char* fn) {
   Keys16 k{};
   k.i1 = idx_l1; k.i2 = idx_l2; k.i3 = idx_l3; k.i4 = idx_l4; k.radii = radii;
-  TQ_CHECK_ARG(idx_l1 && idx_l2 && idx_l3 && idx_l4, "tq_polar_dequantize: null index array");
-  return decode16_common(k, precondition, codebooks, nullptr, n_codebook, n_vectors, dim, block_size,
-                         false, out, stream, "tq_polar_dequantize");
+  TQ_CHECK_ARG(idx_l1 && idx_l2 && idx_l3 && idx_l4, "%s: null index array", fn);
+  return decode16_common(k, precondition, codebooks, Books{}, n_codebook, n_vectors, dim, block_size,
+                         false, out, stream, fn);
 }
 
-int tq_polar_dequantize_packed(const uint32_t* packed_l1, const uint8_t* packed_l2,
-                               const uint8_t* packed_l3, const uint8_t* packed_l4,
-                               const uint16_t* radii, const float* codebooks,
-                               const float* cs_tables, const int* n_codebook, int64_t n_vectors,
-                               int dim, int block_size, float* out, void* stream) {
+int polar_dequantize_packed_impl(const uint32_t* packed_l1, const uint8_t* packed_l2, const uint8_t*
+                                 packed_l3, const uint8_t* packed_l4, const uint16_t* radii, const Books&
+                                 codebooks, const Books& cs_tables, const int* n_codebook, int64_t n_vectors,
+                                 int dim, int block_size, float* out, void* stream, const char* fn) {
   Keys16 k{};
   k.p1 = packed_l1; k.p2 = packed_l2; k.p3 = packed_l3; k.p4 = packed_l4; k.radii = radii;
   TQ_CHECK_ARG(packed_l1 && packed_l2 && packed_l3 && packed_l4,
-               "tq_polar_dequantize_packed: null index array");
+               "%s: null index array", fn);
   return decode16_common(k, nullptr, codebooks, cs_tables, n_codebook, n_vectors, dim, block_size,
-                         true, out, stream, "tq_polar_dequantize_packed");
+                         true, out, stream, fn);
 }
 
-int tq_compressed_score(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2,
-                        const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii,
-                        const float* codebooks, const int* n_codebook, int num_kv_heads,
-                        int n_keys, int dim, int block_size, float scale, float* scores,
-                        void* stream) {
-  const char* fn = "tq_compressed_score";
+int compressed_score_impl(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2, const
+                          uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const Books&
+                          codebooks, const int* n_codebook, int num_kv_heads, int n_keys, int dim, int
+                          block_size, float scale, float* scores, void* stream, const char* fn) {
   Attn16 a;
   int st = attn16_setup(a, q, idx_l1, idx_l2, idx_l3, idx_l4, nullptr, nullptr, nullptr, nullptr,
                         radii, codebooks, n_codebook, false, num_heads, num_kv_heads, n_keys, dim,
@@ -2350,13 +2368,11 @@ int tq_compressed_score(const float* q, int num_heads, const uint8_t* idx_l1, co
   return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, stream, fn);
 }
 
-int tq_compressed_score_packed(const float* q, int num_heads, const uint32_t* packed_l1,
-                               const uint8_t* packed_l2, const uint8_t* packed_l3,
-                               const uint8_t* packed_l4, const uint16_t* radii,
-                               const float* codebooks, const int* n_codebook, int num_kv_heads,
-                               int n_keys, int dim, int block_size, float scale, float* scores,
-                               void* stream) {
-  const char* fn = "tq_compressed_score_packed";
+int compressed_score_packed_impl(const float* q, int num_heads, const uint32_t* packed_l1, const uint8_t*
+                                 packed_l2, const uint8_t* packed_l3, const uint8_t* packed_l4, const
+                                 uint16_t* radii, const Books& codebooks, const int* n_codebook, int
+                                 num_kv_heads, int n_keys, int dim, int block_size, float scale, float*
+                                 scores, void* stream, const char* fn) {
   Attn16 a;
   int st = attn16_setup(a, q, nullptr, nullptr, nullptr, nullptr, packed_l1, packed_l2, packed_l3,
                         packed_l4, radii, codebooks, n_codebook, true, num_heads, num_kv_heads,
@@ -2365,17 +2381,11 @@ int tq_compressed_score_packed(const float* q, int num_heads, const uint32_t* pa
   return score16_common(a, num_heads, num_kv_heads, n_keys, scale, scores, stream, fn);
 }
 
-size_t tq_compressed_sdpa_workspace_size(int num_heads, int num_kv_heads, int dim, int max_n_keys) {
-  if (num_kv_heads < 1 || num_heads < num_kv_heads || max_n_keys < 0 || dim < 1) return 0;
-  return polar_ws_size(num_heads, num_kv_heads, dim, max_n_keys, 4);
-}
-
-int tq_compressed_sdpa(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2,
-                       const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii,
-                       const float* codebooks, const int* n_codebook, const float* values,
-                       int num_kv_heads, int n_keys, int dim, int block_size, float scale,
-                       float* out, void* workspace, size_t workspace_bytes, void* stream) {
-  const char* fn = "tq_compressed_sdpa";
+int compressed_sdpa_impl(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2, const
+                         uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const Books&
+                         codebooks, const int* n_codebook, const float* values, int num_kv_heads, int n_keys,
+                         int dim, int block_size, float scale, float* out, void* workspace, size_t
+                         workspace_bytes, void* stream, const char* fn) {
   Attn16 a;
   int st = attn16_setup(a, q, idx_l1, idx_l2, idx_l3, idx_l4, nullptr, nullptr, nullptr, nullptr,
                         radii, codebooks, n_codebook, false, num_heads, num_kv_heads, n_keys, dim,
@@ -2403,6 +2413,144 @@ int tq_compressed_sdpa(const float* q, int num_heads, const uint8_t* idx_l1, con
       }
     }
   });
+}
+
+}  // namespace
+
+extern "C" {
+
+int tq_polar_quantize(const float* x, const float* precondition, const float* codebooks, const int*
+                      n_codebook, int64_t n_vectors, int dim, int block_size, uint8_t* idx_l1, uint8_t*
+                      idx_l2, uint8_t* idx_l3, uint8_t* idx_l4, uint16_t* radii, void* stream) {
+  return polar_quantize_impl(x, precondition, books_joined(codebooks, n_codebook, 1), n_codebook, n_vectors,
+                             dim, block_size, idx_l1, idx_l2, idx_l3, idx_l4, radii, stream,
+                             "tq_polar_quantize");
+}
+
+int tq_polar_quantize_levels(const float* x, const float* precondition, const float* const* codebooks, const
+                             int* n_codebook, int64_t n_vectors, int dim, int block_size, uint8_t* idx_l1,
+                             uint8_t* idx_l2, uint8_t* idx_l3, uint8_t* idx_l4, uint16_t* radii, void* stream)
+                             {
+  return polar_quantize_impl(x, precondition, books_of(codebooks), n_codebook, n_vectors, dim, block_size,
+                             idx_l1, idx_l2, idx_l3, idx_l4, radii, stream, "tq_polar_quantize_levels");
+}
+
+int tq_polar_quantize_packed(const float* x, const float* precondition, const float* codebooks, const int*
+                             n_codebook, int64_t n_vectors, int dim, int block_size, uint32_t* packed_l1,
+                             uint8_t* packed_l2, uint8_t* packed_l3, uint8_t* packed_l4, uint16_t* radii,
+                             void* stream) {
+  return polar_quantize_packed_impl(x, precondition, books_joined(codebooks, n_codebook, 1), n_codebook,
+                                    n_vectors, dim, block_size, packed_l1, packed_l2, packed_l3, packed_l4,
+                                    radii, stream, "tq_polar_quantize_packed");
+}
+
+int tq_polar_quantize_packed_levels(const float* x, const float* precondition, const float* const* codebooks,
+                                    const int* n_codebook, int64_t n_vectors, int dim, int block_size,
+                                    uint32_t* packed_l1, uint8_t* packed_l2, uint8_t* packed_l3, uint8_t*
+                                    packed_l4, uint16_t* radii, void* stream) {
+  return polar_quantize_packed_impl(x, precondition, books_of(codebooks), n_codebook, n_vectors, dim,
+                                    block_size, packed_l1, packed_l2, packed_l3, packed_l4, radii, stream,
+                                    "tq_polar_quantize_packed_levels");
+}
+
+int tq_polar_dequantize(const uint8_t* idx_l1, const uint8_t* idx_l2, const uint8_t* idx_l3, const uint8_t*
+                        idx_l4, const uint16_t* radii, const float* precondition, const float* codebooks,
+                        const int* n_codebook, int64_t n_vectors, int dim, int block_size, float* out, void*
+                        stream) {
+  return polar_dequantize_impl(idx_l1, idx_l2, idx_l3, idx_l4, radii, precondition, books_joined(codebooks,
+                               n_codebook, 1), n_codebook, n_vectors, dim, block_size, out, stream,
+                               "tq_polar_dequantize");
+}
+
+int tq_polar_dequantize_levels(const uint8_t* idx_l1, const uint8_t* idx_l2, const uint8_t* idx_l3, const
+                               uint8_t* idx_l4, const uint16_t* radii, const float* precondition, const float*
+                               const* codebooks, const int* n_codebook, int64_t n_vectors, int dim, int
+                               block_size, float* out, void* stream) {
+  return polar_dequantize_impl(idx_l1, idx_l2, idx_l3, idx_l4, radii, precondition, books_of(codebooks),
+                               n_codebook, n_vectors, dim, block_size, out, stream,
+                               "tq_polar_dequantize_levels");
+}
+
+int tq_polar_dequantize_packed(const uint32_t* packed_l1, const uint8_t* packed_l2, const uint8_t* packed_l3,
+                               const uint8_t* packed_l4, const uint16_t* radii, const float* codebooks, const
+                               float* cs_tables, const int* n_codebook, int64_t n_vectors, int dim, int
+                               block_size, float* out, void* stream) {
+  return polar_dequantize_packed_impl(packed_l1, packed_l2, packed_l3, packed_l4, radii,
+                                      books_joined(codebooks, n_codebook, 1), books_joined(cs_tables,
+                                      n_codebook, 2), n_codebook, n_vectors, dim, block_size, out, stream,
+                                      "tq_polar_dequantize_packed");
+}
+
+int tq_polar_dequantize_packed_levels(const uint32_t* packed_l1, const uint8_t* packed_l2, const uint8_t*
+                                      packed_l3, const uint8_t* packed_l4, const uint16_t* radii, const float*
+                                      const* codebooks, const float* const* cs_tables, const int* n_codebook,
+                                      int64_t n_vectors, int dim, int block_size, float* out, void* stream) {
+  return polar_dequantize_packed_impl(packed_l1, packed_l2, packed_l3, packed_l4, radii, books_of(codebooks),
+                                      books_of(cs_tables), n_codebook, n_vectors, dim, block_size, out,
+                                      stream, "tq_polar_dequantize_packed_levels");
+}
+
+int tq_compressed_score(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2, const
+                        uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const float* codebooks,
+                        const int* n_codebook, int num_kv_heads, int n_keys, int dim, int block_size, float
+                        scale, float* scores, void* stream) {
+  return compressed_score_impl(q, num_heads, idx_l1, idx_l2, idx_l3, idx_l4, radii, books_joined(codebooks,
+                               n_codebook, 1), n_codebook, num_kv_heads, n_keys, dim, block_size, scale,
+                               scores, stream, "tq_compressed_score");
+}
+
+int tq_compressed_score_levels(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2,
+                               const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const
+                               float* const* codebooks, const int* n_codebook, int num_kv_heads, int n_keys,
+                               int dim, int block_size, float scale, float* scores, void* stream) {
+  return compressed_score_impl(q, num_heads, idx_l1, idx_l2, idx_l3, idx_l4, radii, books_of(codebooks),
+                               n_codebook, num_kv_heads, n_keys, dim, block_size, scale, scores, stream,
+                               "tq_compressed_score_levels");
+}
+
+int tq_compressed_score_packed(const float* q, int num_heads, const uint32_t* packed_l1, const uint8_t*
+                               packed_l2, const uint8_t* packed_l3, const uint8_t* packed_l4, const uint16_t*
+                               radii, const float* codebooks, const int* n_codebook, int num_kv_heads, int
+                               n_keys, int dim, int block_size, float scale, float* scores, void* stream) {
+  return compressed_score_packed_impl(q, num_heads, packed_l1, packed_l2, packed_l3, packed_l4, radii,
+                                      books_joined(codebooks, n_codebook, 1), n_codebook, num_kv_heads,
+                                      n_keys, dim, block_size, scale, scores, stream,
+                                      "tq_compressed_score_packed");
+}
+
+int tq_compressed_score_packed_levels(const float* q, int num_heads, const uint32_t* packed_l1, const uint8_t*
+                                      packed_l2, const uint8_t* packed_l3, const uint8_t* packed_l4, const
+                                      uint16_t* radii, const float* const* codebooks, const int* n_codebook,
+                                      int num_kv_heads, int n_keys, int dim, int block_size, float scale,
+                                      float* scores, void* stream) {
+  return compressed_score_packed_impl(q, num_heads, packed_l1, packed_l2, packed_l3, packed_l4, radii,
+                                      books_of(codebooks), n_codebook, num_kv_heads, n_keys, dim, block_size,
+                                      scale, scores, stream, "tq_compressed_score_packed_levels");
+}
+
+size_t tq_compressed_sdpa_workspace_size(int num_heads, int num_kv_heads, int dim, int max_n_keys) {
+  if (num_kv_heads < 1 || num_heads < num_kv_heads || max_n_keys < 0 || dim < 1) return 0;
+  return polar_ws_size(num_heads, num_kv_heads, dim, max_n_keys, 4);
+}
+
+int tq_compressed_sdpa(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2, const
+                       uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const float* codebooks,
+                       const int* n_codebook, const float* values, int num_kv_heads, int n_keys, int dim, int
+                       block_size, float scale, float* out, void* workspace, size_t workspace_bytes, void*
+                       stream) {
+  return compressed_sdpa_impl(q, num_heads, idx_l1, idx_l2, idx_l3, idx_l4, radii, books_joined(codebooks,
+                              n_codebook, 1), n_codebook, values, num_kv_heads, n_keys, dim, block_size,
+                              scale, out, workspace, workspace_bytes, stream, "tq_compressed_sdpa");
+}
+
+int tq_compressed_sdpa_levels(const float* q, int num_heads, const uint8_t* idx_l1, const uint8_t* idx_l2,
+                              const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const
+                              float* const* codebooks, const int* n_codebook, const float* values, int
+                              num_kv_heads, int n_keys, int dim, int block_size, float scale, float* out,
+                              void* workspace, size_t workspace_bytes, void* stream) {
+  return compressed_sdpa_impl(q, num_heads, idx_l1, idx_l2, idx_l3, idx_l4, radii, books_of(codebooks),
+                              n_codebook, values, num_kv_heads, n_keys, dim, block_size, scale, out,
+                              workspace, workspace_bytes, stream, "tq_compressed_sdpa_levels");
 }
 
 int tq_polar_rotate(const float* x, const float* precondition, int64_t rows, int dim, float* y,

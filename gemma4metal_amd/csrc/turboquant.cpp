@@ -93,30 +93,19 @@ void* workspace(size_t bytes, size_t* have, StreamOrDevice s) {
   return w.ptr;
 }
 
-// The four codebooks back to back in one device buffer + their sizes.
+// The four levels' tables (entries of `width` floats) as the C ABI takes them.
 struct Codebooks {
-  array buf;
+  const float* levels[4];
   int sizes[4];
 };
 
-Codebooks concat_codebooks(const array& c1, const array& c2, const array& c3, const array& c4,
-                           int width, StreamOrDevice s) {
+Codebooks codebooks_of(const array& c1, const array& c2, const array& c3, const array& c4, int width) {
   Codebooks cb;
   const array* cs[4] = {&c1, &c2, &c3, &c4};
-  int64_t total = 0;
   for (int i = 0; i < 4; ++i) {
     need(cs[i]->dtype() == Dtype::float32, "codebooks must be float32");
+    cb.levels[i] = static_cast<const float*>(cs[i]->data());
     cb.sizes[i] = static_cast<int>(cs[i]->size() / width);
-    total += cs[i]->size();
-  }
-  cb.buf = array::empty({total}, Dtype::float32);
-  size_t off = 0;
-  for (int i = 0; i < 4; ++i) {
-    check_hip(hipMemcpyAsync(static_cast<char*>(cb.buf.data()) + off, cs[i]->data(),
-                             cs[i]->nbytes(), hipMemcpyDeviceToDevice,
-                             static_cast<hipStream_t>(s)),
-              "hipMemcpyAsync");
-    off += cs[i]->nbytes();
   }
   return cb;
 }
@@ -364,13 +353,13 @@ std::vector<array> polar_quantize(const array& vectors, const array& preconditio
                                   const array& cb_l4, int block_size, StreamOrDevice s) {
   need(vectors.ndim() == 2 && vectors.dtype() == Dtype::float32, "vectors must be (N, D) float32");
   const int64_t N = vectors.shape(0), D = vectors.shape(1), nb = N * (D / 16);
-  Codebooks cb = concat_codebooks(cb_l1, cb_l2, cb_l3, cb_l4, 1, s);
+  Codebooks cb = codebooks_of(cb_l1, cb_l2, cb_l3, cb_l4, 1);
   array i1 = array::empty({nb * 8}, Dtype::uint8), i2 = array::empty({nb * 4}, Dtype::uint8);
   array i3 = array::empty({nb * 2}, Dtype::uint8), i4 = array::empty({nb}, Dtype::uint8);
   array r = array::empty({nb}, Dtype::float16);
-  check(tq_polar_quantize(static_cast<const float*>(vectors.data()),
+  check(tq_polar_quantize_levels(static_cast<const float*>(vectors.data()),
                           static_cast<const float*>(precondition.data()),
-                          static_cast<const float*>(cb.buf.data()), cb.sizes, N,
+                          cb.levels, cb.sizes, N,
                           static_cast<int>(D), block_size, static_cast<uint8_t*>(i1.data()),
                           static_cast<uint8_t*>(i2.data()), static_cast<uint8_t*>(i3.data()),
                           static_cast<uint8_t*>(i4.data()), static_cast<uint16_t*>(r.data()), s),
@@ -384,13 +373,13 @@ std::vector<array> polar_quantize_packed(const array& vectors, const array& prec
                                          StreamOrDevice s) {
   need(vectors.ndim() == 2 && vectors.dtype() == Dtype::float32, "vectors must be (N, D) float32");
   const int64_t N = vectors.shape(0), D = vectors.shape(1), nb = N * (D / 16);
-  Codebooks cb = concat_codebooks(cb_l1, cb_l2, cb_l3, cb_l4, 1, s);
+  Codebooks cb = codebooks_of(cb_l1, cb_l2, cb_l3, cb_l4, 1);
   array p1 = array::empty({nb}, Dtype::uint32), p2 = array::empty({nb}, Dtype::uint8);
   array p3 = array::empty({nb}, Dtype::uint8), p4 = array::empty({nb}, Dtype::uint8);
   array r = array::empty({nb}, Dtype::float16);
-  check(tq_polar_quantize_packed(
+  check(tq_polar_quantize_packed_levels(
             static_cast<const float*>(vectors.data()), static_cast<const float*>(precondition.data()),
-            static_cast<const float*>(cb.buf.data()), cb.sizes, N, static_cast<int>(D), block_size,
+            cb.levels, cb.sizes, N, static_cast<int>(D), block_size,
             static_cast<uint32_t*>(p1.data()), static_cast<uint8_t*>(p2.data()),
             static_cast<uint8_t*>(p3.data()), static_cast<uint8_t*>(p4.data()),
             static_cast<uint16_t*>(r.data()), s),
@@ -404,14 +393,14 @@ array dequant_unpacked(const array& i1, const array& i2, const array& i3, const 
                        const array& c3, const array& c4, int64_t D, int block_size,
                        StreamOrDevice s, const char* fn) {
   const int64_t N = radii.size() * 16 / D;
-  Codebooks cb = concat_codebooks(c1, c2, c3, c4, 1, s);
+  Codebooks cb = codebooks_of(c1, c2, c3, c4, 1);
   array out = array::empty({N, D}, Dtype::float32);
-  check(tq_polar_dequantize(static_cast<const uint8_t*>(i1.data()),
+  check(tq_polar_dequantize_levels(static_cast<const uint8_t*>(i1.data()),
                             static_cast<const uint8_t*>(i2.data()),
                             static_cast<const uint8_t*>(i3.data()),
                             static_cast<const uint8_t*>(i4.data()),
                             static_cast<const uint16_t*>(radii.data()), P,
-                            static_cast<const float*>(cb.buf.data()), cb.sizes, N,
+                            cb.levels, cb.sizes, N,
                             static_cast<int>(D), block_size, static_cast<float*>(out.data()), s),
         fn);
   return out;
@@ -422,15 +411,14 @@ array dequant_packed(const array& p1, const array& p2, const array& p3, const ar
                      const array& c4, bool cs, int64_t D, int block_size, StreamOrDevice s,
                      const char* fn) {
   const int64_t N = radii.size() * 16 / D;
-  Codebooks cb = concat_codebooks(c1, c2, c3, c4, cs ? 2 : 1, s);
+  Codebooks cb = codebooks_of(c1, c2, c3, c4, cs ? 2 : 1);
   array out = array::empty({N, D}, Dtype::float32);
-  const float* buf = static_cast<const float*>(cb.buf.data());
-  check(tq_polar_dequantize_packed(static_cast<const uint32_t*>(p1.data()),
+  check(tq_polar_dequantize_packed_levels(static_cast<const uint32_t*>(p1.data()),
                                    static_cast<const uint8_t*>(p2.data()),
                                    static_cast<const uint8_t*>(p3.data()),
                                    static_cast<const uint8_t*>(p4.data()),
-                                   static_cast<const uint16_t*>(radii.data()), cs ? nullptr : buf,
-                                   cs ? buf : nullptr, cb.sizes, N, static_cast<int>(D),
+                                   static_cast<const uint16_t*>(radii.data()), cs ? nullptr : cb.levels,
+                                   cs ? cb.levels : nullptr, cb.sizes, N, static_cast<int>(D),
                                    block_size, static_cast<float*>(out.data()), s),
         fn);
   return out;
@@ -477,15 +465,15 @@ array compressed_score(const array& queries, const array& indices_l1, const arra
                        const array& cb_l4, int N, int block_size, float scale, StreamOrDevice s) {
   need(queries.ndim() == 2 && queries.dtype() == Dtype::float32, "queries must be (Nq, D) float32");
   const int Nq = static_cast<int>(queries.shape(0)), D = static_cast<int>(queries.shape(1));
-  Codebooks cb = concat_codebooks(cb_l1, cb_l2, cb_l3, cb_l4, 1, s);
+  Codebooks cb = codebooks_of(cb_l1, cb_l2, cb_l3, cb_l4, 1);
   array out = array::empty({Nq, N}, Dtype::float32);
-  check(tq_compressed_score(static_cast<const float*>(queries.data()), Nq,
+  check(tq_compressed_score_levels(static_cast<const float*>(queries.data()), Nq,
                             static_cast<const uint8_t*>(indices_l1.data()),
                             static_cast<const uint8_t*>(indices_l2.data()),
                             static_cast<const uint8_t*>(indices_l3.data()),
                             static_cast<const uint8_t*>(indices_l4.data()),
                             static_cast<const uint16_t*>(radii.data()),
-                            static_cast<const float*>(cb.buf.data()), cb.sizes, Nq, N, D,
+                            cb.levels, cb.sizes, Nq, N, D,
                             block_size, scale, static_cast<float*>(out.data()), s),
         "compressed_score");
   return out;
@@ -499,17 +487,17 @@ array compressed_sdpa(const array& queries, const array& indices_l1, const array
   need(queries.ndim() == 2 && values.ndim() == 2, "queries (Nq, D), values (Nq * N, D)");
   const int Nq = static_cast<int>(queries.shape(0)), D = static_cast<int>(queries.shape(1));
   const int N = static_cast<int>(values.shape(0) / Nq);
-  Codebooks cb = concat_codebooks(cb_l1, cb_l2, cb_l3, cb_l4, 1, s);
+  Codebooks cb = codebooks_of(cb_l1, cb_l2, cb_l3, cb_l4, 1);
   array out = array::empty({Nq, D}, Dtype::float32);
   size_t have = 0;
   void* ws = workspace(tq_compressed_sdpa_workspace_size(Nq, Nq, D, N), &have, s);
-  check(tq_compressed_sdpa(static_cast<const float*>(queries.data()), Nq,
+  check(tq_compressed_sdpa_levels(static_cast<const float*>(queries.data()), Nq,
                            static_cast<const uint8_t*>(indices_l1.data()),
                            static_cast<const uint8_t*>(indices_l2.data()),
                            static_cast<const uint8_t*>(indices_l3.data()),
                            static_cast<const uint8_t*>(indices_l4.data()),
                            static_cast<const uint16_t*>(radii.data()),
-                           static_cast<const float*>(cb.buf.data()), cb.sizes,
+                           cb.levels, cb.sizes,
                            static_cast<const float*>(values.data()), Nq, N, D, block_size, scale,
                            static_cast<float*>(out.data()), ws, have, s),
         "compressed_sdpa");

@@ -6,8 +6,7 @@ Every computation runs in ``libturboquant_hip.so`` (C ABI in
 ``include/tq_c_api.h``); torch only holds device memory and the stream.
 Function names, argument order and defaults follow the reference; its
 ``StreamOrDevice`` argument becomes ``stream``.  Codebooks are passed per
-level, as in the reference, and concatenated into one device buffer for the
-C ABI.
+level, as in the reference.
 """
 from __future__ import annotations
 
@@ -27,19 +26,26 @@ QJL_M = 128
 P7_QTAB = 5136  # floats of per-head query tables (TQ_POLAR7_QTAB)
 
 
+def _levels(tables: Sequence[torch.Tensor], width: int, name: str):
+    """The four per-level tables as the C ABI takes them: a host array of
+    their device pointers, a host int[4] of their entries (``width`` floats
+    each), and the tensors the pointers belong to."""
+    _need(len(tables) == 4, "four codebooks (levels 1..4) are required")
+    keep = []
+    for i, c in enumerate(tables):
+        _check_cuda(f"{name}_l{i + 1}", c)
+        keep.append(c if c.dtype == torch.float32 else c.to(torch.float32))
+    ptrs = (ctypes.c_void_p * 4)(*[c.data_ptr() for c in keep])
+    sizes = (ctypes.c_int * 4)(*[c.numel() // width for c in keep])
+    return ptrs, sizes, keep
+
+
 def _codebooks(cbs: Sequence[torch.Tensor]):
-    """Concatenate the four per-level codebooks into one f32 device tensor and
-    a host int[4] of their sizes."""
-    _need(len(cbs) == 4, "four codebooks (levels 1..4) are required")
-    for i, c in enumerate(cbs):
-        _check_cuda(f"cb_l{i + 1}", c)
-    cat = torch.cat([c.reshape(-1).to(torch.float32) for c in cbs]).contiguous()
-    sizes = (ctypes.c_int * 4)(*[int(c.numel()) for c in cbs])
-    return cat, sizes
+    return _levels(cbs, 1, "cb")
 
 
-def _sizes_ptr(sizes):
-    return ctypes.cast(sizes, ctypes.c_void_p)
+def _host_array(sizes):
+    return ctypes.cast(sizes, ctypes.c_void_p) if sizes is not None else None
 
 
 def _rows(vectors: torch.Tensor):
@@ -63,11 +69,11 @@ def polar_quantize(vectors: torch.Tensor, precondition: Optional[torch.Tensor],
     nb = D // 16
     if precondition is not None:
         _check_cuda("precondition", precondition)
-    cb, sizes = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
+    cb, sizes, keep = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
     dev = vectors.device
     outs = [torch.empty(N * nb * k, dtype=torch.uint8, device=dev) for k in (8, 4, 2, 1)]
     radii = torch.empty(N * nb, dtype=torch.float16, device=dev)
-    call("tq_polar_quantize", _ptr(vectors), _ptr(precondition), _ptr(cb), _sizes_ptr(sizes), N, D,
+    call("tq_polar_quantize_levels", _ptr(vectors), _ptr(precondition), _host_array(cb), _host_array(sizes), N, D,
          int(block_size), *[_ptr(o) for o in outs], _ptr(radii), _stream(stream))
     return outs + [radii]
 
@@ -82,13 +88,13 @@ def polar_quantize_packed(vectors: torch.Tensor, precondition: Optional[torch.Te
     nbt = N * (D // 16)
     if precondition is not None:
         _check_cuda("precondition", precondition)
-    cb, sizes = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
+    cb, sizes, keep = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
     dev = vectors.device
     p1 = torch.empty(nbt, dtype=torch.uint32, device=dev)
     p2, p3, p4 = (torch.empty(nbt, dtype=torch.uint8, device=dev) for _ in range(3))
     radii = torch.empty(nbt, dtype=torch.float16, device=dev)
-    call("tq_polar_quantize_packed", _ptr(vectors), _ptr(precondition), _ptr(cb),
-         _sizes_ptr(sizes), N, D, int(block_size), _ptr(p1), _ptr(p2), _ptr(p3), _ptr(p4),
+    call("tq_polar_quantize_packed_levels", _ptr(vectors), _ptr(precondition), _host_array(cb),
+         _host_array(sizes), N, D, int(block_size), _ptr(p1), _ptr(p2), _ptr(p3), _ptr(p4),
          _ptr(radii), _stream(stream))
     return [p1, p2, p3, p4, radii]
 
@@ -120,10 +126,10 @@ def _dequant_unpacked(i1, i2, i3, i4, radii, P, cbs, D, block_size, stream):
     _need(radii.dtype == torch.float16, "radii must be float16")
     nbt = radii.numel()
     N = nbt * 16 // D
-    cb, sizes = _codebooks(list(cbs))
+    cb, sizes, keep = _codebooks(list(cbs))
     out = torch.empty((N, D), dtype=torch.float32, device=radii.device)
-    call("tq_polar_dequantize", _ptr(i1), _ptr(i2), _ptr(i3), _ptr(i4), _ptr(radii), _ptr(P),
-         _ptr(cb), _sizes_ptr(sizes), N, D, int(block_size), _ptr(out), _stream(stream))
+    call("tq_polar_dequantize_levels", _ptr(i1), _ptr(i2), _ptr(i3), _ptr(i4), _ptr(radii), _ptr(P),
+         _host_array(cb), _host_array(sizes), N, D, int(block_size), _ptr(out), _stream(stream))
     return out
 
 
@@ -152,17 +158,14 @@ def _dequant_packed(p1, p2, p3, p4, radii, cbs, cs, D, block_size, stream):
     nbt = radii.numel()
     N = nbt * 16 // D
     if cs is not None:
-        for i, c in enumerate(cs):
-            _check_cuda(f"cs_l{i + 1}", c)
-        cst = torch.cat([c.reshape(-1).to(torch.float32) for c in cs]).contiguous()
-        sizes = (ctypes.c_int * 4)(*[int(c.shape[0]) for c in cs])
+        cst, sizes, keep = _levels(cs, 2, "cs")
         cb = None
     else:
-        cb, sizes = _codebooks(list(cbs))
+        cb, sizes, keep = _codebooks(list(cbs))
         cst = None
     out = torch.empty((N, D), dtype=torch.float32, device=radii.device)
-    call("tq_polar_dequantize_packed", _ptr(p1), _ptr(p2), _ptr(p3), _ptr(p4), _ptr(radii),
-         _ptr(cb), _ptr(cst), _sizes_ptr(sizes), N, D, int(block_size), _ptr(out),
+    call("tq_polar_dequantize_packed_levels", _ptr(p1), _ptr(p2), _ptr(p3), _ptr(p4), _ptr(radii),
+         _host_array(cb), _host_array(cst), _host_array(sizes), N, D, int(block_size), _ptr(out),
          _stream(stream))
     return out
 
@@ -178,10 +181,10 @@ def compressed_score(queries, indices_l1, indices_l2, indices_l3, indices_l4, ra
     _need(queries.dim() == 2 and queries.dtype == torch.float32, "queries must be (Nq, D) f32")
     Nq, D = queries.shape
     Hkv = Nq if num_kv_heads is None else int(num_kv_heads)
-    cb, sizes = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
+    cb, sizes, keep = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
     out = torch.empty((Nq, N), dtype=torch.float32, device=queries.device)
-    call("tq_compressed_score", _ptr(queries), Nq, _ptr(indices_l1), _ptr(indices_l2),
-         _ptr(indices_l3), _ptr(indices_l4), _ptr(radii), _ptr(cb), _sizes_ptr(sizes), Hkv, int(N),
+    call("tq_compressed_score_levels", _ptr(queries), Nq, _ptr(indices_l1), _ptr(indices_l2),
+         _ptr(indices_l3), _ptr(indices_l4), _ptr(radii), _host_array(cb), _host_array(sizes), Hkv, int(N),
          D, int(block_size), float(scale), _ptr(out), _stream(stream))
     return out
 
@@ -194,10 +197,10 @@ def compressed_score_packed(queries, packed_l1, packed_l2, packed_l3, packed_l4,
     _check_cuda("queries", queries)
     Nq, D = queries.shape
     Hkv = Nq if num_kv_heads is None else int(num_kv_heads)
-    cb, sizes = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
+    cb, sizes, keep = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
     out = torch.empty((Nq, N), dtype=torch.float32, device=queries.device)
-    call("tq_compressed_score_packed", _ptr(queries), Nq, _ptr(packed_l1), _ptr(packed_l2),
-         _ptr(packed_l3), _ptr(packed_l4), _ptr(radii), _ptr(cb), _sizes_ptr(sizes), Hkv, int(N),
+    call("tq_compressed_score_packed_levels", _ptr(queries), Nq, _ptr(packed_l1), _ptr(packed_l2),
+         _ptr(packed_l3), _ptr(packed_l4), _ptr(radii), _host_array(cb), _host_array(sizes), Hkv, int(N),
          D, int(block_size), float(scale), _ptr(out), _stream(stream))
     return out
 
@@ -216,13 +219,13 @@ def compressed_sdpa(queries, indices_l1, indices_l2, indices_l3, indices_l4, rad
     _need(values.dim() == 2 and values.shape[1] == D and values.shape[0] % Hkv == 0,
           "values must be (num_kv_heads * N, D)")
     N = values.shape[0] // Hkv
-    cb, sizes = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
+    cb, sizes, keep = _codebooks([cb_l1, cb_l2, cb_l3, cb_l4])
     out = torch.empty((Nq, D), dtype=torch.float32, device=queries.device)
     nbytes = _lib.load().tq_compressed_sdpa_workspace_size(Nq, Hkv, D, N)
     sh = _stream(stream)
     ws = workspace(nbytes, queries.device, sh)
-    call("tq_compressed_sdpa", _ptr(queries), Nq, _ptr(indices_l1), _ptr(indices_l2),
-         _ptr(indices_l3), _ptr(indices_l4), _ptr(radii), _ptr(cb), _sizes_ptr(sizes),
+    call("tq_compressed_sdpa_levels", _ptr(queries), Nq, _ptr(indices_l1), _ptr(indices_l2),
+         _ptr(indices_l3), _ptr(indices_l4), _ptr(radii), _host_array(cb), _host_array(sizes),
          _ptr(values), Hkv, N, D, int(block_size), float(scale), _ptr(out), _ptr(ws), ws.numel(),
          sh)
     return out

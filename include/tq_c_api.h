@@ -302,6 +302,41 @@ int tq_compressed_sdpa(const float* q, int num_heads, const uint8_t* idx_l1, con
                        int num_kv_heads, int n_keys, int dim, int block_size, float scale,
                        float* out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The calls above with each level's table in a device array of its own:
+ * `codebooks` (`cs_tables`) is a HOST array of four device pointers, levels 1
+ * to 4, in place of one array with the levels back to back.  The reference's
+ * callers hold the levels apart (lib/turboquant.h:52-165); joining them costs
+ * a copy per call.  (No other difference.) */
+int tq_polar_quantize_levels(const float* x, const float* precondition, const float* const*
+        codebooks, const int* n_codebook, int64_t n_vectors, int dim, int block_size, uint8_t*
+        idx_l1, uint8_t* idx_l2, uint8_t* idx_l3, uint8_t* idx_l4, uint16_t* radii, void*
+        stream);
+int tq_polar_quantize_packed_levels(const float* x, const float* precondition, const float*
+        const* codebooks, const int* n_codebook, int64_t n_vectors, int dim, int block_size,
+        uint32_t* packed_l1, uint8_t* packed_l2, uint8_t* packed_l3, uint8_t* packed_l4,
+        uint16_t* radii, void* stream);
+int tq_polar_dequantize_levels(const uint8_t* idx_l1, const uint8_t* idx_l2, const uint8_t*
+        idx_l3, const uint8_t* idx_l4, const uint16_t* radii, const float* precondition, const
+        float* const* codebooks, const int* n_codebook, int64_t n_vectors, int dim, int
+        block_size, float* out, void* stream);
+int tq_polar_dequantize_packed_levels(const uint32_t* packed_l1, const uint8_t* packed_l2, const
+        uint8_t* packed_l3, const uint8_t* packed_l4, const uint16_t* radii, const float* const*
+        codebooks, const float* const* cs_tables, const int* n_codebook, int64_t n_vectors, int
+        dim, int block_size, float* out, void* stream);
+int tq_compressed_score_levels(const float* q, int num_heads, const uint8_t* idx_l1, const
+        uint8_t* idx_l2, const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii,
+        const float* const* codebooks, const int* n_codebook, int num_kv_heads, int n_keys, int
+        dim, int block_size, float scale, float* scores, void* stream);
+int tq_compressed_score_packed_levels(const float* q, int num_heads, const uint32_t* packed_l1,
+        const uint8_t* packed_l2, const uint8_t* packed_l3, const uint8_t* packed_l4, const
+        uint16_t* radii, const float* const* codebooks, const int* n_codebook, int num_kv_heads,
+        int n_keys, int dim, int block_size, float scale, float* scores, void* stream);
+int tq_compressed_sdpa_levels(const float* q, int num_heads, const uint8_t* idx_l1, const
+        uint8_t* idx_l2, const uint8_t* idx_l3, const uint8_t* idx_l4, const uint16_t* radii,
+        const float* const* codebooks, const int* n_codebook, const float* values, int
+        num_kv_heads, int n_keys, int dim, int block_size, float scale, float* out, void*
+        workspace, size_t workspace_bytes, void* stream);
+
 /* ---- 7-level PolarQuant + QJL ("polar7"; D = 128) ---------------------------
  * No reference kernel: the same polar recursion as polar_quantize over one
  * 128-value block (7 levels; level-1 angles 4-bit, levels 2-7 2-bit) plus
