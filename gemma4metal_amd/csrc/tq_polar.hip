@@ -141,8 +141,8 @@ struct Enc16Params {
 
 constexpr int kEncThreads = 512;
 // Values up to which a workgroup takes 16 (D 64: 32) vectors, more above it.
-// Whole calls, few against many vectors: D 256, 4,096 vectors 43 / 51 us, 5,120
-// 61 / 51; D 128, 8,192 vectors 28 / 28, 10,240 34 / 28, 32,768 68 / 47.
+// Whole calls, few against many vectors: D 256, 4,096 vectors 28 / 36 us, 5,120
+// 39 / 37; D 128, 2,048 vectors 18 / 22, 10,240 24.5 / 22.5, 32,768 52 / 41.
 constexpr int64_t kEnc16Small = 1 << 20;
 // LDS row strides of the encoders are 16 bytes past a multiple of the 256-byte
 // bank period (rows of 64 k floats, padded by 4): a 16-lane phase of row
@@ -152,20 +152,22 @@ constexpr int kEncColStr = 64 + 4;  // 64 columns of a matrix
 // Rows r0 .. r0 + ROWS - 1, columns c0 .. c0 + 63 of a matrix with rows of DIM
 // floats (the 16-byte global loads here need the 4-byte alignment of a float
 // only): into registers, ROWS / 32 float4 a thread, and from there into LDS.
+typedef float vf4 __attribute__((ext_vector_type(4)));  // (arrays of HIP's float4 stayed in scratch)
+
 template <int ROWS, int DIM>
-__device__ __forceinline__ void load_cols(const float* m, int r0, int c0, float4 (&r)[ROWS / 32]) {
+__device__ __forceinline__ void load_cols(const float* m, int r0, int c0, vf4 (&r)[ROWS / 32]) {
 #pragma unroll
   for (int i = 0; i < ROWS / 32; ++i) {
     const int e = threadIdx.x + kEncThreads * i;
-    r[i] = *reinterpret_cast<const float4*>(m + (r0 + (e >> 4)) * DIM + c0 + 4 * (e & 15));
+    r[i] = *reinterpret_cast<const vf4*>(m + (r0 + (e >> 4)) * DIM + c0 + 4 * (e & 15));
   }
 }
 template <int N>
-__device__ __forceinline__ void store_cols(float* ms, const float4 (&r)[N]) {
+__device__ __forceinline__ void store_cols(float* ms, const vf4 (&r)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     const int e = threadIdx.x + kEncThreads * i;
-    *reinterpret_cast<float4*>(ms + (e >> 4) * kEncColStr + 4 * (e & 15)) = r[i];
+    *reinterpret_cast<vf4*>(ms + (e >> 4) * kEncColStr + 4 * (e & 15)) = r[i];
   }
 }
 
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(kEncThreads) void polar_encode16_tile_kernel(Enc16P
   const int tid = threadIdx.x;
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * V;
   const int rows = static_cast<int>(min(static_cast<int64_t>(V), p.n - row0));
-  float4 mreg[ROWS / 32];
+  vf4 mreg[ROWS / 32];
   if (p.P) load_cols<ROWS, D>(p.P, 0, 0, mreg);
   fill_codebooks<kEncThreads>(cbs, p);
 #pragma unroll
@@ -882,7 +884,7 @@ constexpr float kSketchSlack = 4.0f * 129.0f * 0x1p-24f;
 // share a CU and one's matrix-core and memory phases run under the other's
 // VALU phases.  A wave per vector with P and S rows read from L2 at a 1 KB
 // lane stride took 901 us there; V = 128 with whole matrices in LDS, one
-// workgroup a CU, 112 us; this form 105 us.
+// workgroup a CU, 112 us; this form 90 us.
 template <int V, int TV, int TI, int PPL>
 __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams p) {
 #pragma clang fp contract(off)
@@ -900,8 +902,16 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t row0 = static_cast<int64_t>(blockIdx.x) * V;
-  float4 mreg[4];
-  if (p.P) load_cols<128, 128>(p.P, 0, 0, mreg);
+  // Halves of P and S in flight: all four from the start in the small form (a
+  // memory round trip each otherwise), the next one else.
+  constexpr bool kAll = V == 16;
+  vf4 h0[4], h1[kAll ? 4 : 1], h2[kAll ? 4 : 1], h3[kAll ? 4 : 1];
+  if (p.P) load_cols<128, 128>(p.P, 0, 0, h0);
+  if constexpr (kAll) {
+    if (p.P) load_cols<128, 128>(p.P, 0, 64, h1);
+    load_cols<128, 128>(p.S, 0, 0, h2);
+    load_cols<128, 128>(p.S, 0, 64, h3);
+  }
   // uniform: scalar registers
   float cb1[16], cb2[4];
 #pragma unroll
@@ -935,12 +945,13 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
     for (int j = 0; j < TV; ++j)
 #pragma unroll
       for (int k = 0; k < TI; ++k) acc[j][k] = 0.0f;
-    store_cols(ms, mreg);
-    load_cols<128, 128>(p.P, 0, 64, mreg);
+    store_cols(ms, h0);
+    if constexpr (!kAll) load_cols<128, 128>(p.P, 0, 64, h0);
     __syncthreads();
     exact_dots<kEncStr>(xs, ms, v0, i0, IG, acc);
     __syncthreads();  // every wave is done with the first half
-    store_cols(ms, mreg);
+    if constexpr (kAll) store_cols(ms, h1);
+    else store_cols(ms, h0);
     __syncthreads();
     exact_dots<kEncStr>(xs + 64, ms, v0, i0, IG, acc);
     __syncthreads();  // every wave is done with x and P
@@ -949,7 +960,7 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
 #pragma unroll
       for (int k = 0; k < TI; ++k) xs[(v0 + j) * kEncStr + i0 + IG * k] = acc[j][k];
   }
-  load_cols<128, 128>(p.S, 0, 0, mreg);
+  if constexpr (!kAll) load_cols<128, 128>(p.S, 0, 0, h0);
   __syncthreads();
 
   // ---- encode: lane b of a vector has pairs PPL b .. PPL b + PPL - 1
@@ -1044,8 +1055,13 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
                         (static_cast<uint32_t>(__half_as_ushort(rn16)) << 16);
     }
   }
-  store_cols(ms, mreg);  // P is no longer read (barrier before the encoding)
-  load_cols<128, 128>(p.S, 0, 64, mreg);
+  // P is no longer read (barrier before the encoding)
+  if constexpr (kAll) {
+    store_cols(ms, h2);
+  } else {
+    store_cols(ms, h0);
+    load_cols<128, 128>(p.S, 0, 64, h0);
+  }
   __syncthreads();
   for (int i = tid; i < V * kP7Words; i += kEncThreads) {
     const int64_t orow = orow_s[i / kP7Words];
@@ -1082,7 +1098,8 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
     }
     if (half == 0) {
       __syncthreads();
-      store_cols(ms, mreg);
+      if constexpr (kAll) store_cols(ms, h3);
+      else store_cols(ms, h0);
     } else {
       s2 += __shfl_xor(s2, 1, 64);
       s2 += __shfl_xor(s2, 2, 64);
@@ -1117,10 +1134,10 @@ __global__ __launch_bounds__(kEncThreads) void polar7_encode_kernel(P7EncParams 
 
 // Vectors per workgroup: 64, or 16 for small inputs (four times the
 // workgroups, a quarter of a lane's chain of angles).  Whole calls, 16 against
-// 64 vectors: 17.6 / 31.0 us at 16 rows, 32.9 / 38.3 at 8,192, 44.6 / 38.8 at
-// 12,288, 181.7 / 104.7 at 65,536.
+// 64 vectors: 13.7 / 25.8 us at 16 rows, 24.3 / 31.8 at 8,192, 34.8 / 35.3 at
+// 12,288, 41.7 / 33.2 at 16,384, 129 / 93 at 65,536.
 int launch_p7_encode(const P7EncParams& p, hipStream_t s) {
-  constexpr int64_t kWide = 10240;
+  constexpr int64_t kWide = 12288;
   if (p.n > kWide) {
     polar7_encode_kernel<64, 4, 4, 8><<<static_cast<unsigned>((p.n + 63) / 64), kEncThreads, 0, s>>>(p);
   } else {

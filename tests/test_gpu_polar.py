@@ -234,7 +234,7 @@ def test_polar7_encode_bit_exact(pq, n, rot):
         assert mism.size == 0, f"{name}: rows {mism[:8]} differ ({mism.size} rows)"
 
 
-@pytest.mark.parametrize("n,rot", [(16, True), (17, False), (10240 - 8, True), (10240 - 7 + 64, True), (10240 + 129, False)])
+@pytest.mark.parametrize("n,rot", [(16, True), (17, False), (12288 - 4, True), (12288 - 3 + 64, True), (12288 + 129, False)])
 def test_polar7_encode_tiles_and_scales(pq, n, rot):
     """Row counts at the edges of the 16- and 64-vector workgroups, rows of
     very small and very large norm (the sketch's sign bound does not hold
