@@ -1,7 +1,8 @@
 // Multi-query (prefill) attention over the int4 cache with K/V tiles shared
 // by a workgroup's (query, head) rows -- the engine's prefill fallback
 // (engine/gemma4_multilayer.cpp:343-364: dequantize, then masked
-// scaled_dot_product_attention), for head_dim 128 / 256 / 512.
+// scaled_dot_product_attention), for head_dim 128 / 256 / 512 and 16-bit
+// queries (fp32 ones: tq_prefill_f32.hip).
 //
 // A workgroup takes RS sets of 16 consecutive (query, head) rows of one kv
 // head and streams the union of their key ranges in tiles of 32 KH keys; wave
@@ -14,8 +15,7 @@
 //
 //   S^T[key][row] = sum_g s_k[key][g] ((n - 8) . q)_g + b'_k[key][g] (sum q)_g
 //     (. . q)_g: v_mfma_f32_16x16x32_f16 over the group's 64 dims, A = nibbles
-//     of 16 keys, B = q of 16 rows, scaled by a power of two per row (so bf16
-//     and fp16 queries are exact in one product, fp32 ones 22 bits in two);
+//     of 16 keys, B = q of 16 rows, scaled by a power of two per row (exact);
 //     one fma per (key, row, group) applies s_k.  The bias term is one more
 //     product a 16-key half: A = biases and scales, B = the group sums of q in
 //     three fp16 parts.
@@ -113,7 +113,7 @@ __device__ __forceinline__ void pf_load(PfRaw<Gm>& R, const SdpaParams& p, int64
         R.w[i][k] = a[k];
         R.w[i][4 + k] = b[k];
       }
-    } else if (role == 1) {
+    } else {  // (D 128: threads past the units load one again and do not store it)
       const int w = u % Gm::W, kc = u / Gm::W;  // kc = 4 kh + c
       const int r0 = 32 * (kc >> 2) + 4 * (kc & 3);
       const uint32_t* src = p.vq + base * Gm::W;
@@ -127,11 +127,11 @@ __device__ __forceinline__ void pf_load(PfRaw<Gm>& R, const SdpaParams& p, int64
 #pragma unroll
   for (int i = 0; i < Gm::NSD; ++i) {
     const int e = threadIdx.x + i * Gm::NT;
-    const int t = __builtin_amdgcn_readfirstlane(e / Gm::SDW), d = e % Gm::SDW;
+    // (threads past the tensors load one again and do not store it)
+    const int t = min(__builtin_amdgcn_readfirstlane(e / Gm::SDW), 3), d = e % Gm::SDW;
     constexpr int DPR = Gm::SDW / Gm::TK;  // dwords a row
     const void* src = t == 0 ? p.ks : t == 1 ? p.kb : t == 2 ? p.vs : p.vb;
-    if ((4 * Gm::SDW) % Gm::NT == 0 || t < 4)
-      R.s[i] = (reinterpret_cast<const u32_a2*>(src) + base * DPR)[row(d / DPR) * DPR + d % DPR];
+    R.s[i] = (reinterpret_cast<const u32_a2*>(src) + base * DPR)[row(d / DPR) * DPR + d % DPR];
   }
 }
 
@@ -214,7 +214,7 @@ __device__ __forceinline__ uint32_t pf_rem_pair(uint32_t hp, float x0, float x1)
   return r;
 }
 
-template <int D, bool F32, int QP, int NS, int RS>
+template <int D, bool F32, int NS, int RS>
 __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
   using Gm = PfGeom<D, F32, NS, RS>;
   using SB = typename Gm::SB;
@@ -250,7 +250,7 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
   // ---- q: B operands of k-step s of group g are dims 64 g + 16 c + 8 s + {0, 4,
   // 1, 5, 2, 6, 3, 7}, times 2^(15 - ex) (the row's largest below 2^15), the odd
   // ones over 16.  The sign of a negative scale goes into q.
-  v8h qf[NS][2 * NWG][QP], qb[NS];
+  v8h qf[NS][2 * NWG], qb[NS];
   float rf[NS];                             // score = rf * products
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
@@ -263,24 +263,17 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 #pragma unroll
     for (int j = 0; j < 2 * NWG; ++j) {
       const int64_t e0 = qrow * D + Gm::OW * dh + 64 * (j >> 1) + 16 * c + 8 * (j & 1);
-      if (p.q_dtype == TQ_F32) {
-        const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
-        const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
-        f[j][0] = a.x; f[j][1] = a.y; f[j][2] = a.z; f[j][3] = a.w;
-        f[j][4] = b.x; f[j][5] = b.y; f[j][6] = b.z; f[j][7] = b.w;
-      } else {
-        const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
-        const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
+      const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
+      const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (p.q_dtype == TQ_F16) {
-            const v2h h = __builtin_bit_cast(v2h, wd[i]);
-            f[j][2 * i] = static_cast<float>(h[0]);
-            f[j][2 * i + 1] = static_cast<float>(h[1]);
-          } else {
-            f[j][2 * i] = __uint_as_float(wd[i] << 16);
-            f[j][2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
-          }
+      for (int i = 0; i < 4; ++i) {
+        if (p.q_dtype == TQ_F16) {
+          const v2h h = __builtin_bit_cast(v2h, wd[i]);
+          f[j][2 * i] = static_cast<float>(h[0]);
+          f[j][2 * i + 1] = static_cast<float>(h[1]);
+        } else {
+          f[j][2 * i] = __uint_as_float(wd[i] << 16);
+          f[j][2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
         }
       }
 #pragma unroll
@@ -302,9 +295,7 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
         qs[j >> 1] += x;
         const int slot = (i & 2) ? 4 + 2 * (i & 1) + (i >> 2) : 2 * (i & 1) + (i >> 2);
         const float y = (i & 1) ? x * 0.0625f : x;
-        const _Float16 h = static_cast<_Float16>(y);
-        qf[n][j][0][slot] = h;
-        if constexpr (QP == 2) qf[n][j][1][slot] = static_cast<_Float16>(y - static_cast<float>(h));
+        qf[n][j][slot] = static_cast<_Float16>(y);
       }
     }
     // group sums over 512 (|.| < 2^12) in fp16 parts.  fp16 scale/bias: part c
@@ -404,12 +395,8 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
           const v8h a0 = __builtin_bit_cast(v8h, kr[0]), a1 = __builtin_bit_cast(v8h, kr[64]);
 #pragma unroll
           for (int n = 0; n < NS; ++n) {
-            v4f a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g][0], z, 0, 0, 0);
-            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1][0], a, 0, 0, 0);
-            if constexpr (QP == 2) {
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g][1], a, 0, 0, 0);
-              a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1][1], a, 0, 0, 0);
-            }
+            v4f a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g], z, 0, 0, 0);
+            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1], a, 0, 0, 0);
             acc[n][g] = a;
           }
         }
@@ -608,45 +595,46 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 // were centred, which would add 128 instructions), two row sets a wave at one
 // wave per SIMD (97 us), operand reads half a tile ahead (68), the two waves of
 // a SIMD staging at opposite ends of a tile (69).
-template <int D, bool F32, int QP, int NS, int RS>
+template <int D, bool F32, int NS, int RS>
 __global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
 void prefill_int4_ws_kernel(SdpaParams p) {
   pin_args(p);
-  prefill_rows<D, F32, QP, NS, RS>(p);
+  prefill_rows<D, F32, NS, RS>(p);
 }
 
-template <int D, bool F32, int QP, int NS, int RS>
+template <int D, bool F32, int NS, int RS>
 __global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
 void prefill_int4_kernel(SdpaParams p) {
   pin_args(p);
-  prefill_rows<D, F32, QP, NS, RS>(p);
+  prefill_rows<D, F32, NS, RS>(p);
 }
 
-template <int D, bool F32, int QP, int NS, int RS>
+template <int D, bool F32, int NS, int RS>
 void launch_sets(const SdpaParams& p, unsigned grid, hipStream_t s) {
-  if constexpr (D == 512) prefill_int4_kernel<D, F32, QP, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
-  else prefill_int4_ws_kernel<D, F32, QP, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
+  if constexpr (D == 512) prefill_int4_kernel<D, F32, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
+  else prefill_int4_ws_kernel<D, F32, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
 }
 
 constexpr int kPfNS = 1;  // row sets a wave
 
-// 64 rows per workgroup where those fill the CUs, else 32 on four waves (twice
-// the workgroups; 100 queries of Hq 32 Hkv 8 D 128: 24.7 against 26.6 us, and 16
-// rows on two waves, which then stage a whole tile, 29.0).
-template <int D, bool F32, int QP>
+// 32 rows per workgroup of four waves while that gives every CU at most one
+// (twice the workgroups: 128 queries of Hq 32 Hkv 16 D 256 60 against 65 us, 100 of
+// Hq 32 Hkv 8 D 128 24.7 against 26.6; 16 rows on two waves, which then stage a
+// whole tile, 78 and 29), else 64.
+template <int D, bool F32>
 void launch_rows(const SdpaParams& p, hipStream_t s) {
   constexpr int NR = 16 * kPfNS, RSM = 4 / kPfNS;
   const int64_t rows = static_cast<int64_t>(p.nq) * p.gqa;
   const auto grid = [&](int rs) { return static_cast<unsigned>((rows + NR * rs - 1) / (NR * rs) * p.Hkv); };
-  if (grid(RSM) >= static_cast<unsigned>(target_wgs())) launch_sets<D, F32, QP, kPfNS, RSM>(p, grid(RSM), s);
-  else launch_sets<D, F32, QP, kPfNS, 2>(p, grid(2), s);
+  if (grid(2) <= static_cast<unsigned>(target_wgs())) launch_sets<D, F32, kPfNS, 2>(p, grid(2), s);
+  else launch_sets<D, F32, kPfNS, RSM>(p, grid(RSM), s);
 }
 
-template <bool F32, int QP>
+template <bool F32>
 void launch_dim(const SdpaParams& p, int D, hipStream_t s) {
-  if (D == 128) launch_rows<128, F32, QP>(p, s);
-  else if (D == 256) launch_rows<256, F32, QP>(p, s);
-  else launch_rows<512, F32, QP>(p, s);
+  if (D == 128) launch_rows<128, F32>(p, s);
+  else if (D == 256) launch_rows<256, F32>(p, s);
+  else launch_rows<512, F32>(p, s);
 }
 
 }  // namespace
@@ -660,14 +648,9 @@ bool prefill_tiles_serve(int D, int sb_dtype, int gqa) {
 
 int launch_prefill_tiles(const SdpaParams& p, int D, int sb_dtype, hipStream_t s) {
   if (!prefill_tiles_serve(D, sb_dtype, p.gqa)) return -1;
-  const bool two = p.q_dtype == TQ_F32;  // fp32 queries: two products
-  if (sb_dtype == TQ_F32) {
-    if (two) launch_dim<true, 2>(p, D, s);
-    else launch_dim<true, 1>(p, D, s);
-  } else {
-    if (two) launch_dim<false, 2>(p, D, s);
-    else launch_dim<false, 1>(p, D, s);
-  }
+  if (p.q_dtype == TQ_F32) return launch_prefill_tiles_f32(p, D, sb_dtype, s);
+  if (sb_dtype == TQ_F32) launch_dim<true>(p, D, s);
+  else launch_dim<false>(p, D, s);
   TQ_CHECK_LAUNCH("prefill_int4_kernel");
   return TQ_OK;
 }

@@ -68,7 +68,7 @@ namespace {
 // The switches of Options, as atomics so that a reload while other threads
 // plan calls is well defined (each call sees old or new values).
 struct OptionStore {
-  std::atomic<int> sdpa_valu{0}, sdpa_chunk{0}, prefill_splitk{0}, hc_one{0};
+  std::atomic<int> sdpa_valu{0}, sdpa_chunk{0}, prefill_splitk{0}, prefill_ws{1}, hc_one{0};
 };
 OptionStore g_opts;
 std::once_flag g_opts_once;
@@ -81,6 +81,8 @@ void read_options() {
   g_opts.sdpa_chunk.store(v ? std::atoi(v) : 0, std::memory_order_relaxed);
   v = env("TQ_PREFILL_IMPL");
   g_opts.prefill_splitk.store(v && std::string(v) == "splitk", std::memory_order_relaxed);
+  v = env("TQ_PREFILL_WS");
+  g_opts.prefill_ws.store(!(v && v[0] == '0'), std::memory_order_relaxed);
   v = env("TQ_HC_IMPL");
   g_opts.hc_one.store(v && v[0] == '1', std::memory_order_relaxed);
 }
@@ -92,6 +94,7 @@ Options options() {
   o.sdpa_valu = g_opts.sdpa_valu.load(std::memory_order_relaxed) != 0;
   o.sdpa_chunk = g_opts.sdpa_chunk.load(std::memory_order_relaxed);
   o.prefill_splitk = g_opts.prefill_splitk.load(std::memory_order_relaxed) != 0;
+  o.prefill_ws = g_opts.prefill_ws.load(std::memory_order_relaxed) != 0;
   o.hc_one = g_opts.hc_one.load(std::memory_order_relaxed) != 0;
   return o;
 }

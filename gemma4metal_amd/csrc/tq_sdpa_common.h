@@ -612,11 +612,13 @@ WsLayout ws_layout(int batch, int Hq, int D, int max_splits);
 //   TQ_SDPA_IMPL=valu       the VALU decode kernel for every shape
 //   TQ_SDPA_CHUNK=n         keys per split (overrides the planner)
 //   TQ_PREFILL_IMPL=splitk  prefill on the split-K decode kernels
+//   TQ_PREFILL_WS=0         fp32 queries: the one-role prefill tile kernel
 //   TQ_HC_IMPL=1            the one-wave D=512 heads-as-columns kernel
 struct Options {
   bool sdpa_valu;
   int sdpa_chunk;
   bool prefill_splitk;
+  bool prefill_ws;
   bool hc_one;
 };
 Options options();
@@ -661,6 +663,8 @@ int launch_sdpa_hc(const SdpaParams& p, int sb_dtype, dim3 grid, hipStream_t str
 // -1 when the shape is not served (D other than 128 / 256 / 512, gqa not
 // dividing 64).
 int launch_prefill_tiles(const SdpaParams& p, int D, int sb_dtype, hipStream_t stream);
+// The same for fp32 queries (tq_prefill_f32.hip).
+int launch_prefill_tiles_f32(const SdpaParams& p, int D, int sb_dtype, hipStream_t stream);
 // Merge of the split partials of a launch with ext_merge = 1 (batch b of
 // grid.y): tq_sdpa_hc.hip.
 int launch_merge_splits(const SdpaParams& p, int D, int batch, hipStream_t stream);

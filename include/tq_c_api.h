@@ -120,8 +120,7 @@ int tq_sdpa_int4_plan(int mode, int batch, int num_heads, int num_kv_heads, int 
 /* Re-reads the kernel-choice switches from the environment (no counterpart
  * in the reference).  They are read once per process otherwise:
  * TQ_SDPA_IMPL=valu, TQ_SDPA_CHUNK=<keys>, TQ_PREFILL_IMPL=splitk,
- * TQ_HC_IMPL=1 (TQ_PREFILL_WS is accepted and has no effect: one prefill tile
- * kernel is left).  For tests and measurement; calls that run
+ * TQ_PREFILL_WS=0 (fp32 queries), TQ_HC_IMPL=1.  For tests and measurement; calls that run
  * while it executes see the old or the new values. */
 int tq_reload_options(void);
 int tq_sdpa_int4(const void* q, tq_dtype q_dtype,
