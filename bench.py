@@ -343,9 +343,9 @@ def main():
                   "value": round(tflops, 2), "unit": "TFLOP/s", "n_gpus": 1, "steps": args.steps,
                   "warmup": args.warmup, "ms_per_step": round(ms, 5),
                   "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-                  "dtype": (f"int4 K/V ({args.sb} scale/bias), bf16 Q; K dequantized to fp16 hi+lo "
-                            "(q.k as three fp16 matrix-core products, ~22-bit), V and P as bf16 "
-                            "hi+lo, fp32 accumulate"),
+                  "dtype": (f"int4 K/V ({args.sb} scale/bias), bf16 Q (exact in fp16); exact fp16 "
+                            "nibbles on the matrix cores, scales in fp32, p*s_v as fp16 hi+lo "
+                            "(~22-bit), fp32 accumulate"),
                   "data": "synthetic", "kernel": plan["kernel"],
                   "config": {"workload": f"prefill n_new={S} n_prior={prior} Hq={Hq_} Hkv={Hkv_} "
                                          f"D={D_} W={W}, {args.sb} scale/bias", "global_batch": 1,
