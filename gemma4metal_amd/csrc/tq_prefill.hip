@@ -21,8 +21,11 @@
 //     three fp16 parts.
 //   O^T[dim][row] = sum_key (n - 8) (p s_v) + sum_key p b'_v
 //     A = nibbles of 16 dims (one group) x 32 keys, B = p s_v as fp16 high part
-//     and remainder (22 bits).  The powers of two in p's reference keep p s_v
-//     below 2^15 (see m_ref below).  The bias term is summed in fp32.
+//     and remainder: 22 bits, down to the fp16 step of 2^-24.  p's reference
+//     holds p s_v to fp16's range (see m_ref below) in tiles whose V scales are
+//     alike; any other tile takes a power of two per row and group of its own,
+//     so that a row's precision does not depend on the V scales of other keys
+//     and groups.  The bias term is summed in fp32.
 // Centred nibbles keep the sums small: the matrix cores' accumulation error
 // grows with the running sum, and with n in place of n - 8 the results were
 // three times as far from 64 bits.
@@ -46,9 +49,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // A running reference moves only when a score passes it by this much (log2).
-constexpr float kPfLazy = 12.0f;
-// log2 of the largest p s_v under the reference (fp16 overflows at 2^16).
-constexpr float kPfHead = 3.0f;
+constexpr float kPfLazy = 8.0f;
+// With 2^e0 above every V scale of a workgroup's first tile: p s_v is below
+// 2^kPfHead for the row's largest weight and a scale of 2^e0, and below 2^15 (fp16
+// overflows at 2^16) for scales up to 2^(e0 + kPfUp).  Scales down to
+// 2^(e0 - kPfDown) leave such a weight 21 bits above fp16's step.
+constexpr int kPfHead = 4, kPfUp = 3, kPfDown = 7;
 
 template <int D, bool F32, int NS, int RS>
 struct PfGeom {
@@ -71,6 +77,7 @@ struct PfGeom {
   static constexpr int NU = (2 * UNITS + NT - 1) / NT;
   static constexpr int SDW = TK * NG * static_cast<int>(sizeof(SB)) / 4;  // dwords of one scale tensor a tile
   static constexpr int NSD = (4 * SDW + NT - 1) / NT;
+  static constexpr int NSW = SDW / 64;   // waves that stage one of them
   static constexpr int OSTR = OW + 2;    // partial output rows (floats): conflict-free 4-byte stores
   struct Stage {
     u32x4 k[2][2 * KH * KU];             // [16-key slice][g][s][c][key]: word 8 g + 2 c + s
@@ -146,9 +153,32 @@ __device__ __forceinline__ uint32_t pf_centre(uint32_t t, uint32_t mask) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2h, b) + v2h{off, off});
 }
 
-// Into LDS buffer b.  vmax: this thread's largest |V scale| so far.
+// Whether this thread's V scales are all within [2^(e0 - kPfDown), 2^(e0 + kPfUp)),
+// per wave that stages some, into ok[NSW].
 template <class Gm>
-__device__ __forceinline__ void pf_store(typename Gm::Stage& S, const PfRaw<Gm>& R, int b, float& vmax) {
+__device__ __forceinline__ void pf_alike(const PfRaw<Gm>& R, int e0, int* ok) {
+  constexpr bool kHalf = sizeof(typename Gm::SB) == 2;
+  // the bounds' bit patterns: magnitudes order as these do
+  const auto bits = [](float x) -> uint32_t {
+    if constexpr (kHalf) return __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
+    else return __float_as_uint(x);
+  };
+  const uint32_t lo = bits(ldexpf(1.0f, e0 - kPfDown)), n = bits(ldexpf(1.0f, e0 + kPfUp)) - lo;
+#pragma unroll
+  for (int i = 0; i < Gm::NSD; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    if (__builtin_amdgcn_readfirstlane(e / Gm::SDW) != 2) continue;
+    const uint32_t a = R.s[i];
+    bool in;
+    if constexpr (kHalf) in = (a & 0x7FFFu) - lo < n && (a >> 16 & 0x7FFFu) - lo < n;
+    else in = (a & 0x7FFFFFFFu) - lo < n;
+    ok[e % Gm::SDW / 64] = __all(in);  // (one value from every lane)
+  }
+}
+
+// Into LDS buffer b.
+template <class Gm>
+__device__ __forceinline__ void pf_store(typename Gm::Stage& S, const PfRaw<Gm>& R, int b) {
   const uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u;
 #pragma unroll
   for (int i = 0; i < Gm::NU; ++i) {
@@ -190,16 +220,25 @@ __device__ __forceinline__ void pf_store(typename Gm::Stage& S, const PfRaw<Gm>&
     const int t = __builtin_amdgcn_readfirstlane(e / Gm::SDW);
     if ((4 * Gm::SDW) % Gm::NT != 0 && t >= 4) continue;
     reinterpret_cast<uint32_t*>(S.sb[b][0])[e] = R.s[i];
-    if (t == 2) {
-      if constexpr (sizeof(typename Gm::SB) == 2) {
-        uint32_t mx = 0;
-        asm("v_max3_f16 %0, %0, abs(%1), abs(%1) op_sel:[0,0,1,0]" : "+v"(mx) : "v"(R.s[i]));
-        vmax = fmaxf(vmax, static_cast<float>(__builtin_bit_cast(v2h, mx)[0]));
-      } else {
-        vmax = fmaxf(vmax, fabsf(__uint_as_float(R.s[i])));
-      }
+  }
+}
+
+// The largest |V scale| of the wave's part of a tile, 0 where it has none.
+template <class Gm>
+__device__ __forceinline__ float pf_vmax(const PfRaw<Gm>& R) {
+  float mx = 0.0f;
+#pragma unroll
+  for (int i = 0; i < Gm::NSD; ++i) {
+    const int e = threadIdx.x + i * Gm::NT;
+    if (__builtin_amdgcn_readfirstlane(e / Gm::SDW) != 2) continue;
+    if constexpr (sizeof(typename Gm::SB) == 2) {
+      const v2h h = __builtin_bit_cast(v2h, R.s[i]);
+      mx = fmaxf(mx, fmaxf(fabsf(static_cast<float>(h[0])), fabsf(static_cast<float>(h[1]))));
+    } else {
+      mx = fmaxf(mx, fabsf(__uint_as_float(R.s[i])));
     }
   }
+  return wave_max_dpp(mx);
 }
 
 // The fp16 remainders x0 - h0, x1 - h1 of a pair whose fp16 high parts are
@@ -220,7 +259,8 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
   using SB = typename Gm::SB;
   constexpr int NG = Gm::NG, NWG = Gm::NW_, TK = Gm::TK, KH = Gm::KH, DH = Gm::DH;
   __shared__ __attribute__((aligned(16))) typename Gm::Lds L;
-  __shared__ uint32_t vmx[2];               // bits of the largest |V scale| up to a buffer's tile
+  __shared__ uint32_t vmx;                  // bits of the first tile's largest |V scale|
+  __shared__ int alike[2][Gm::NSW];         // a buffer's V scales are alike (all of them set)
   __shared__ float ml[Gm::NW][16 * NS], ll[Gm::NW][16 * NS];
 
   const int lane = threadIdx.x & 63;
@@ -320,22 +360,21 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
     }
   }
 
-  if (threadIdx.x < 2) vmx[threadIdx.x] = 0;
+  if (threadIdx.x == 0) vmx = 0;
   __syncthreads();
-  float vmax = 0.0f;
-  auto stage = [&](int b) {
-    pf_store<Gm>(L.st, raw, b, vmax);
-    // each thread's maximum is over all its tiles so far, so the buffer's
-    // value is that of all tiles up to this one, whatever the timing
-    const float wm = wave_max_dpp(vmax);
-    if (lane == 0) atomicMax(&vmx[b], __float_as_uint(wm));
-  };
-  stage(0);
+  const float wm = pf_vmax<Gm>(raw);
+  if (lane == 0) atomicMax(&vmx, __float_as_uint(wm));
+  pf_store<Gm>(L.st, raw, 0);
+  __syncthreads();
+  // (a first tile outside these bounds, like an infinity, is not alike)
+  const int e0 = min(max(__builtin_amdgcn_frexp_expf(__uint_as_float(__builtin_amdgcn_readfirstlane(vmx))), -20), 24);
+  pf_alike<Gm>(raw, e0, alike[0]);
   __syncthreads();
 
-  // p = 2^(x - m_ref).  m_ref >= x + (exponent of the largest |V scale|) -
-  // kPfHead - kPfLazy for every score so far: p s_v stays below 2^15, and the
-  // remainder's absolute step of 2^-24 is 2^-27 of the weight of the largest.
+  // p = 2^(x - m_ref), m_ref = a score of the row + e0 - kPfHead, the largest so
+  // far up to kPfLazy.  A reference that follows the largest V scale staged so far
+  // leaves a row 28 - k bits once a key that it does not attend has 2^k times
+  // the scales of those that it does.
   float m_ref[NS], l_run[NS], bsum[NS][NWG];
   v4f o[NS][4 * NWG];
 #pragma unroll
@@ -446,9 +485,7 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
       }
 
       // ---- online softmax (log2 domain) of rows m ------------------------------
-      const float vm = __uint_as_float(vmx[buf]);
-      const int ve = vm < 0x1p-40f ? -40 : min(__builtin_amdgcn_frexp_expf(vm), 100);
-      const float up = static_cast<float>(ve) - kPfHead;
+      const float up = static_cast<float>(e0 - kPfHead);
       float need[NS];
 #pragma unroll
       for (int n = 0; n < NS; ++n) {
@@ -483,6 +520,59 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
       }
 
       // ---- O^T += V^T P^T ----------------------------------------------------
+      // B operands of eight weights, and O^T's 16 dims x of group g
+      const auto split = [&](const float (&y)[8], v8h& bh, v8h& bl) {
+        u32x4 hi, lw;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          hi[q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(y[2 * q], y[2 * q + 1]));
+          lw[q] = pf_rem_pair(hi[q], y[2 * q], y[2 * q + 1]);
+        }
+        bh = __builtin_bit_cast(v8h, hi);
+        bl = __builtin_bit_cast(v8h, lw);
+      };
+      float pz[NS][8];  // the weights of the common products
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pz[n][j] = pw[n][j];
+      int al = 1;
+#pragma unroll
+      for (int i = 0; i < Gm::NSW; ++i) al &= alike[buf][i];
+      if (!__builtin_amdgcn_readfirstlane(al)) {
+        // V scales apart: the largest weight of every row and group to 2^13 .. 2^14
+        // (an infinity, of exponent 0, stays one), the products on their own, added
+        // in fp32
+#pragma unroll
+        for (int n = 0; n < NS; ++n) {
+#pragma unroll
+          for (int g = 0; g < NWG; ++g) {
+            float y[8], mx = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              y[j] = static_cast<float>(svs[(16 * (j >> 2) + 4 * c + (j & 3)) * NG + g]) * pw[n][j];
+              mx = fmaxf(mx, fabsf(y[j]));
+            }
+            const int k = min(14 - __builtin_amdgcn_frexp_expf(xor32_max(xor16_max(mx))), 120);
+            const float un = ldexpf(1.0f, -k);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) y[j] = ldexpf(y[j], k);
+            v8h bh, bl;
+            split(y, bh, bl);
+#pragma unroll
+            for (int x = 0; x < 4; ++x) {
+              const v8h a = __builtin_bit_cast(v8h, vu[(4 * g + x) * 64 + (m ^ Gm::vswz(g))]);
+              v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, z, 0, 0, 0);
+              t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, t, 0, 0, 0);
+#pragma unroll
+              for (int i = 0; i < 4; ++i) o[n][4 * g + x][i] = fmaf(t[i], un, o[n][4 * g + x][i]);
+            }
+          }
+          // (nothing is left for the products below: a branch around them cost 50 registers)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) pz[n][j] = 0.0f;
+        }
+      }
       SB s[8][NWG], bb[8][NWG];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -496,26 +586,16 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 #pragma unroll
       for (int g = 0; g < NWG; ++g) {
         v8h bh[NS], bl[NS];
-        uint32_t hi[NS][4], lw[NS][4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          // b' = b + 8 s
-          const float b0 = fmaf(static_cast<float>(s[2 * q][g]), 8.0f, static_cast<float>(bb[2 * q][g]));
-          const float b1 = fmaf(static_cast<float>(s[2 * q + 1][g]), 8.0f, static_cast<float>(bb[2 * q + 1][g]));
-#pragma unroll
-          for (int n = 0; n < NS; ++n) {
-            const float x0 = fmaf(static_cast<float>(s[2 * q][g]), pw[n][2 * q], 0.0f);
-            const float x1 = fmaf(static_cast<float>(s[2 * q + 1][g]), pw[n][2 * q + 1], 0.0f);
-            hi[n][q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-            lw[n][q] = pf_rem_pair(hi[n][q], x0, x1);
-            bsum[n][g] = fmaf(b0, pw[n][2 * q], bsum[n][g]);
-            bsum[n][g] = fmaf(b1, pw[n][2 * q + 1], bsum[n][g]);
-          }
-        }
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
-          bh[n] = __builtin_bit_cast(v8h, u32x4{hi[n][0], hi[n][1], hi[n][2], hi[n][3]});
-          bl[n] = __builtin_bit_cast(v8h, u32x4{lw[n][0], lw[n][1], lw[n][2], lw[n][3]});
+          float y[8];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            y[j] = fmaf(static_cast<float>(s[j][g]), pz[n][j], 0.0f);
+            // b' = b + 8 s
+            bsum[n][g] = fmaf(fmaf(static_cast<float>(s[j][g]), 8.0f, static_cast<float>(bb[j][g])), pw[n][j], bsum[n][g]);
+          }
+          split(y, bh[n], bl[n]);
         }
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
@@ -529,7 +609,10 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
         }
       }
     }
-    if (it + 1 < ntile) stage(buf ^ 1);
+    if (it + 1 < ntile) {
+      pf_store<Gm>(L.st, raw, buf ^ 1);
+      pf_alike<Gm>(raw, e0, alike[buf ^ 1]);
+    }
     __syncthreads();
   }
 

@@ -572,6 +572,55 @@ def test_sdpa_prefill_rows_edges(gpu, Hq, Hkv, D, S, prior, W, scale, qmag, vmag
     assert rel < 2e-5, rel
 
 
+def spread_v(rng, Hkv, n, D, low, spread, at):
+    """V whose group 1 is 2^-low of the others everywhere, and one key's V
+    (only its group 0 with at >= n: key at - n) 2^spread times the rest."""
+    v = rng.standard_normal((Hkv, n, D)) * 2.0**-8
+    v[:, :, 64:128] *= 2.0**-low
+    v[:, at % n, :64 if at >= n else D] *= 2.0**spread
+    return v.astype(np.float32)
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,S,prior,W,low,spread,at", [
+    (8, 4, 256, 96, 20, 0, 0, 18, 115),         # the last key: only the last query attends it
+    (8, 4, 256, 96, 20, 0, 10, 12, 80),         # attended by some rows of a workgroup; no tile alike
+    (8, 4, 256, 96, 200, 64, 0, 18, 180),       # outside the window of the later rows
+    (8, 4, 256, 96, 200, 0, 6, -14, 250),       # far smaller than the rest
+    (8, 8, 128, 100, 30, 0, 0, 12, 130 + 60),   # group 0 of one key only
+    (8, 8, 128, 100, 30, 0, 0, 20, 0),          # the first key, attended by all with any weight
+    (16, 2, 512, 80, 50, 0, 0, 18, 129),
+    (16, 2, 512, 80, 50, 40, 10, 16, 70),
+    (16, 2, 512, 80, 90, 0, 0, 16, 170 + 100),
+])
+@pytest.mark.parametrize("sb", ["f16", "f32"])
+def test_sdpa_prefill_v_scales_of_other_keys(gpu, Hq, Hkv, D, S, prior, W, low, spread, at, sb):
+    """A row keeps its precision whatever the V scales of keys and groups that
+    it does not attend (or hardly): every (row, 64-dim group) by itself
+    against float64.  The weights' parts carry 22 bits of the largest term of
+    a (row, group), and scores of magnitude |x| < 80 move an output by x 2^-22
+    of its terms: 2e-5 of their sum."""
+    rng = np.random.default_rng(S + prior + D + at)
+    n = prior + S
+    k = O.rms_norm(rng.standard_normal((Hkv, n, D)).astype(np.float32))
+    c = O.quantize_int4(k, sb) + O.quantize_int4(spread_v(rng, Hkv, n, D, low, spread, at), sb)
+    qd, qv = queries(rng, (S, Hq, D), "bf16")
+    got = host(gpu.sdpa_int4_prefill(qd, *[dev(a) for a in c], prior, Hq // Hkv, 1.0, W)).astype(np.float64)
+    ref = O.sdpa_int4_prefill(qv, *c, prior, Hq // Hkv, 1.0, W)
+    # the sum of the magnitudes of a result's terms: attention over |V|
+    pos, key = prior + np.arange(S)[:, None], np.arange(n)[None]
+    keep = (key <= pos) & ((pos - key < W) if W else True)
+    terms = np.empty_like(got)
+    for h in range(Hq):
+        kv = h // (Hq // Hkv)
+        x = np.where(keep, qv[:, h].astype(np.float64) @ O.dequantize(*(a[kv] for a in c[:3])).T, -np.inf)
+        w = np.exp(x - x.max(axis=1, keepdims=True))
+        terms[:, h] = w @ np.abs(O.dequantize(*(a[kv] for a in c[3:]))) / w.sum(axis=1, keepdims=True)
+    err, den = (np.sqrt((x.reshape(S, Hq, D // 64, 64) ** 2).sum(-1)) for x in (got - ref, terms))
+    assert np.isfinite(got).all()
+    worst = np.unravel_index(np.argmax(err / den), err.shape)
+    assert (err <= 2e-5 * den).all(), (worst, (err / den)[worst])
+
+
 @pytest.mark.parametrize("Hq,Hkv,L,W", [(32, 4, 5000, 0), (32, 4, 3001, 1024), (16, 2, 129, 0)])
 def test_d512_one_wave_and_wave_specialised_kernels_agree(gpu, tq_env, Hq, Hkv, L, W):
     """The two D=512 GQA-8 kernels (TQ_HC_IMPL=1 selects the one-wave one)
