@@ -4,11 +4,10 @@
 // masked scaled_dot_product_attention), for head_dim 128 / 256 / 512.
 //
 // 16-bit queries run the kernels of tq_prefill.hip, which keep the nibbles as
-// they are and are faster for these too (512 queries after 3,584 keys, Hq 32 Hkv 16
-// D 256, window 1,024: 74 against 94 us) and closer to 64 bits (5e-7 against
-// 1.3e-5 of the result).  The results of fp32 queries stay what they were:
-// single elements of the two differ by up to 5e-3 of the result's root mean square,
-// more than a change of speed may move them.
+// they are.  (A form of those with a second product for the remainder of fp32
+// queries took 74 us where this takes 94: 512 queries after 3,584 keys, Hq 32
+// Hkv 16 D 256, window 1,024; it is not built.)  Error against 64 bits there:
+// 2.7e-6 of the result here, 2.5e-5 in the worst row by itself; 5e-7 for that form.
 //
 // A workgroup takes all gqa heads of one kv head for 64 / gqa consecutive
 // queries (16 rows per wave) and streams the union of their key ranges in
@@ -123,6 +122,27 @@ __device__ __forceinline__ uint32_t pf_rem_pair(uint32_t hp, float x0, float x1)
       : "=&v"(r)
       : "v"(hp), "v"(x0), "v"(x1));
   return r;
+}
+
+// Eight scaled query values as fp16 high parts and remainders.  The remainder
+// is formed from the bits of the high part that is stored: two casts of the
+// product x are two roundings to the compiler (it contracts one of them to a
+// mixed-precision fma, rounded once from the exact product), and where x sits
+// halfway between fp16 values they differ -- one element in 2^13 or so was off
+// by 2^-11 of itself, and rows of the result by up to 2.5e-3.
+__device__ __forceinline__ void pf_split_q(const float* q, float scale, v8h& qh, v8h& ql) {
+  typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+  const float4 a = reinterpret_cast<const float4*>(q)[0], b = reinterpret_cast<const float4*>(q)[1];
+  const float x[8] = {a.x * scale, a.y * scale, a.z * scale, a.w * scale,
+                      b.x * scale, b.y * scale, b.z * scale, b.w * scale};
+  u32x4 h, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    h[i] = __builtin_bit_cast(uint32_t, v2h{static_cast<_Float16>(x[2 * i]), static_cast<_Float16>(x[2 * i + 1])});
+    l[i] = pf_rem_pair(h[i], x[2 * i], x[2 * i + 1]);
+  }
+  qh = __builtin_bit_cast(v8h, h);
+  ql = __builtin_bit_cast(v8h, l);
 }
 
 template <int D, bool F32>
@@ -290,18 +310,7 @@ void prefill_int4_kernel(SdpaParams p) {
   v8h qh[CH], ql[CH];
 #pragma unroll
   for (int ch = 0; ch < CH; ++ch) {
-    float f[8];
-    const int64_t e0 = qrow * D + 32 * ch + 8 * c;
-    const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
-    const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
-    f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = f[i] * p.scale_log2;
-      const _Float16 h = static_cast<_Float16>(x);
-      qh[ch][i] = h;
-      ql[ch][i] = static_cast<_Float16>(x - static_cast<float>(h));
-    }
+    pf_split_q(static_cast<const float*>(p.q) + qrow * D + 32 * ch + 8 * c, p.scale_log2, qh[ch], ql[ch]);
   }
 
   // dequant roles: word w of keys kb0 .. kb0 + KPT - 1 of a tile (K), word
@@ -506,18 +515,7 @@ void prefill_int4_ws_kernel(SdpaParams p) {
   v8h qh[CH], ql[CH];
 #pragma unroll
   for (int ch = 0; ch < CH; ++ch) {
-    float f[8];
-    const int64_t e0 = qrow * D + 32 * ch + 8 * c;
-    const float4 a = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0);
-    const float4 b = *reinterpret_cast<const float4*>(static_cast<const float*>(p.q) + e0 + 4);
-    f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w; f[4] = b.x; f[5] = b.y; f[6] = b.z; f[7] = b.w;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = f[i] * p.scale_log2;
-      const _Float16 h = static_cast<_Float16>(x);
-      qh[ch][i] = h;
-      ql[ch][i] = static_cast<_Float16>(x - static_cast<float>(h));
-    }
+    pf_split_q(static_cast<const float*>(p.q) + qrow * D + 32 * ch + 8 * c, p.scale_log2, qh[ch], ql[ch]);
   }
 
   float m_run = -INFINITY, l_run = 0.0f;

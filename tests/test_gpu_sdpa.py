@@ -572,6 +572,22 @@ def test_sdpa_prefill_rows_edges(gpu, Hq, Hkv, D, S, prior, W, scale, qmag, vmag
     assert rel < 2e-5, rel
 
 
+def prefill_terms(q, c, prior, gqa, W):
+    """The sum of the magnitudes of every result's terms: attention over |V|
+    (scale 1), float64."""
+    S, Hq, D = q.shape
+    n = prior + S
+    pos, key = prior + np.arange(S)[:, None], np.arange(n)[None]
+    keep = (key <= pos) & ((pos - key < W) if W else True)
+    terms = np.empty((S, Hq, D))
+    for h in range(Hq):
+        k, v = (O.dequantize(*(a[h // gqa] for a in c[j:j + 3])) for j in (0, 3))
+        x = np.where(keep, q[:, h].astype(np.float64) @ k.T, -np.inf)
+        w = np.exp(x - x.max(axis=1, keepdims=True))
+        terms[:, h] = w @ np.abs(v) / w.sum(axis=1, keepdims=True)
+    return terms
+
+
 def spread_v(rng, Hkv, n, D, low, spread, at):
     """V whose group 1 is 2^-low of the others everywhere, and one key's V
     (only its group 0 with at >= n: key at - n) 2^spread times the rest."""
@@ -606,19 +622,38 @@ def test_sdpa_prefill_v_scales_of_other_keys(gpu, Hq, Hkv, D, S, prior, W, low, 
     qd, qv = queries(rng, (S, Hq, D), "bf16")
     got = host(gpu.sdpa_int4_prefill(qd, *[dev(a) for a in c], prior, Hq // Hkv, 1.0, W)).astype(np.float64)
     ref = O.sdpa_int4_prefill(qv, *c, prior, Hq // Hkv, 1.0, W)
-    # the sum of the magnitudes of a result's terms: attention over |V|
-    pos, key = prior + np.arange(S)[:, None], np.arange(n)[None]
-    keep = (key <= pos) & ((pos - key < W) if W else True)
-    terms = np.empty_like(got)
-    for h in range(Hq):
-        kv = h // (Hq // Hkv)
-        x = np.where(keep, qv[:, h].astype(np.float64) @ O.dequantize(*(a[kv] for a in c[:3])).T, -np.inf)
-        w = np.exp(x - x.max(axis=1, keepdims=True))
-        terms[:, h] = w @ np.abs(O.dequantize(*(a[kv] for a in c[3:]))) / w.sum(axis=1, keepdims=True)
+    terms = prefill_terms(qv, c, prior, Hq // Hkv, W)
     err, den = (np.sqrt((x.reshape(S, Hq, D // 64, 64) ** 2).sum(-1)) for x in (got - ref, terms))
     assert np.isfinite(got).all()
     worst = np.unravel_index(np.argmax(err / den), err.shape)
     assert (err <= 2e-5 * den).all(), (worst, (err / den)[worst])
+
+
+@pytest.mark.parametrize("D,ws", [(128, "1"), (128, "0"), (256, "1"), (256, "0"), (512, "1")])
+@pytest.mark.parametrize("sb", ["f16", "f32"])
+def test_sdpa_prefill_f32_queries_on_half_ties(gpu, tq_env, D, ws, sb):
+    """fp32 queries whose fp32 product with scale * log2(e) lies halfway between
+    two fp16 values, which its exact product does not: the fp16 high part and
+    the remainder still add up.  Every row by itself: the bf16 parts of weights
+    and V leave 3 2^-18 of the terms, the fp16 parts of q and K 3 2^-22 of
+    sum |q k| (about 0.64 D) in a score: 1e-4 at D 256, 2.5e-4 at D 512."""
+    tq_env("TQ_PREFILL_WS", ws)
+    rng = np.random.default_rng(D)
+    x = rng.standard_normal(1 << 24).astype(np.float32)
+    c = np.float32(1.4426950408889634)
+    p32, p64 = x * c, x.astype(np.float64) * np.float64(c)
+    tie = ((p32.view(np.uint32) & 0x1FFF) == 0x1000) & (np.abs(p32) > 2.0**-10)
+    ties = x[tie & (p32.astype(np.float16) != p64.astype(np.float16))]
+    assert ties.size > 200
+    Hq, Hkv, S, prior, W = 4, 2, 80, 50, 100
+    q = rng.choice(ties, (S, Hq, D))
+    k = O.rms_norm(rng.standard_normal((Hkv, prior + S, D)).astype(np.float32))
+    cache = O.quantize_int4(k, sb) + O.quantize_int4(rng.standard_normal(k.shape).astype(np.float32), sb)
+    got = host(gpu.sdpa_int4_prefill(dev(q), *[dev(a) for a in cache], prior, Hq // Hkv, 1.0, W)).astype(np.float64)
+    ref = O.sdpa_int4_prefill(q, *cache, prior, Hq // Hkv, 1.0, W)
+    terms = prefill_terms(q, cache, prior, Hq // Hkv, W)
+    rel = np.linalg.norm(got - ref, axis=-1) / np.linalg.norm(terms, axis=-1)
+    assert rel.max() < (2.5e-4 if D == 512 else 1e-4), rel.max()
 
 
 @pytest.mark.parametrize("Hq,Hkv,L,W", [(32, 4, 5000, 0), (32, 4, 3001, 1024), (16, 2, 129, 0)])
