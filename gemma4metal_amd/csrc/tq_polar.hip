@@ -805,6 +805,11 @@ __global__ __launch_bounds__(kSdpa16Waves * 64) void polar16_sdpa_kernel(SdpaPar
         l_run[g] += s[i][g];
       }
     }
+    if (tb + T > rg.t_end) {  // slots past the end: 0 times the repeated row would make its infinities NaN
+#pragma unroll
+      for (int j = 0; j < NV; ++j)
+        if (tb + j * RPI + vr >= rg.t_end) v[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int src = ((j & 3) * RPI + vr) * LPK;  // a lane of the row's key in batch j / 4

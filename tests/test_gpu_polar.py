@@ -211,6 +211,26 @@ def test_compressed_tiles_and_odd_addresses(pq, D, Hq, Hkv, N):
         assert_close(got, ref_o, f"compressed_sdpa D{D} Hq{Hq} Hkv{Hkv} N{N} offset {off}")
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_compressed_sdpa_infinite_last_value(pq, D):
+    """An infinity in the last key's V row is that row's result only in the
+    dims that hold it, as an infinity, with a partial last tile (whose masked
+    slots have weight 0)."""
+    rng = np.random.default_rng(D)
+    Hkv, N = 2, 1037
+    cbs = rand_codebooks(rng, packed=False)
+    v = rng.standard_normal((Hkv * N, D)).astype(f32)
+    q = rng.standard_normal((Hkv, D)).astype(f32)
+    idx = PQ.polar_quantize(rng.standard_normal((Hkv * N, D)).astype(f32), None, cbs)
+    args = [dev(q), *[dev(a) for a in idx], *[dev(c) for c in cbs]]
+    ref = PQ.compressed_sdpa(q, *idx, cbs, v, 0.05, gqa=1)
+    v[N - 1, 5], v[2 * N - 1, D - 1] = np.inf, -np.inf
+    got = host(pq.compressed_sdpa(*args, dev(v), scale=0.05, num_kv_heads=Hkv))
+    assert got[0, 5] == np.inf and got[1, D - 1] == -np.inf
+    got[0, 5], got[1, D - 1] = ref[0, 5], ref[1, D - 1]
+    assert_close(got, ref, f"D{D}")
+
+
 # --------------------------------------------------------------- polar7 --------
 
 def p7_inputs(seed, n, rot=True):
