@@ -520,12 +520,15 @@ def test_sdpa_prefill_matches_oracle(gpu, Hq, Hkv, D, S, prior, W, qdt):
     (32, 4, 512, 100, 300, 0, "bf16"),     # Gemma global layer: 8 queries x 8 heads
     (8, 1, 512, 70, 40, 64, "f16"),        # D 512 with a window, partial last group
     (16, 8, 512, 64, 10, 0, "f32"),        # D 512 GQA 2: 32 queries x 2 heads
+    (32, 16, 256, 130, 900, 256, "f32"),   # fp32 queries at the main head dim, window
+    (8, 1, 128, 67, 33, 0, "f32"),
 ])
 @pytest.mark.parametrize("sb", ["f16", "f32"])
 def test_sdpa_prefill_tile_kernel(gpu, Hq, Hkv, D, S, prior, W, qdt, sb):
-    """Prefills of >= 64 queries at D 128 / 256 / 512 run the K/V-tile kernel
-    (fp16 / bf16 hi-lo matrix-core products), for fp16 and fp32 (the
-    reference's cache dtype) scale/bias."""
+    """Prefills of >= 64 queries at D 128 / 256 / 512 run the K/V-tile kernels
+    (16-bit queries: products of the centred nibbles; fp32 queries: hi / lo
+    products of the dequantized values), for fp16 and fp32 (the reference's
+    cache dtype) scale/bias.  The plan names the kernel of 16-bit queries."""
     plan = gpu.sdpa_plan(Hq, Hkv, D, prior + S, mode="prefill", batch=S, sliding_window=W,
                          sb_dtype=torch.float32 if sb == "f32" else torch.float16)
     assert plan["kernel"] == ("prefill_int4_kernel" if D == 512 else "prefill_int4_ws_kernel")
@@ -547,12 +550,15 @@ def test_sdpa_prefill_tile_kernel(gpu, Hq, Hkv, D, S, prior, W, qdt, sb):
     (8, 4, 512, 300, 5, 0, 30.0, 1e-3, 1.0),
     (2, 1, 256, 90, 1, 1, 0.0, 1.0, 1.0),            # window 1, scale 0
 ])
-@pytest.mark.parametrize("qdt,sb", [("bf16", "f16"), ("bf16", "f32"), ("f16", "f16"), ("f16", "f32")])
+@pytest.mark.parametrize("qdt,sb", [("bf16", "f16"), ("bf16", "f32"), ("f16", "f16"), ("f16", "f32"), ("f32", "f16"),
+                                    ("f32", "f32")])
 def test_sdpa_prefill_rows_edges(gpu, Hq, Hkv, D, S, prior, W, scale, qmag, vmag, qdt, sb):
     """Edges of the row sets (16), workgroups (32 / 64 rows), tiles (32 / 64
-    keys) and value ranges of the prefill tile kernel.  Its operands carry 22
-    bits and its sums fp32 (16-bit queries are exact): with a score of magnitude x, an output is off by
-    about x 2^-22 of itself, so 2e-5 covers |x| up to 80."""
+    keys) and value ranges of the prefill tile kernels.  The operands for 16-bit
+    queries carry 22 bits and their sums fp32 (the queries are exact): with a
+    score of magnitude x, an output is off by about x 2^-22 of itself, so 2e-5
+    covers |x| up to 80.  Those for fp32 queries leave 3 2^-18 = 1.1e-5 of the
+    terms in P.V (bf16 parts), and as much as above in the scores."""
     rng = np.random.default_rng(S * 3 + prior + Hq + D)
     n = prior + S
     k = O.rms_norm(rng.standard_normal((Hkv, n, D)).astype(np.float32))
@@ -673,11 +679,12 @@ def test_d512_one_wave_and_wave_specialised_kernels_agree(gpu, tq_env, Hq, Hkv, 
 
 @pytest.mark.parametrize("D,gqa", [(256, 2), (128, 8)])
 def test_prefill_tile_kernels_agree(gpu, tq_env, D, gqa):
-    """The wave-specialised and one-role tile kernels (TQ_PREFILL_WS=0)
-    compute the same products in the same order: bit-identical outputs."""
+    """The wave-specialised and one-role tile kernels of fp32 queries
+    (TQ_PREFILL_WS=0) compute the same products in the same order:
+    bit-identical outputs.  (16-bit queries have one tile kernel.)"""
     rng = np.random.default_rng(D + gqa)
     Hkv, S, prior, W = 4, 130, 400, 256
-    qd, qv = queries(rng, (S, Hkv * gqa, D), "bf16")
+    qd, qv = queries(rng, (S, Hkv * gqa, D), "f32")
     c = host_cache(rng, Hkv, prior + S, D, "f16")
     cd = [dev(a) for a in c]
     ws = host(gpu.sdpa_int4_prefill(qd, *cd, prior, gqa, 1.0, W))
