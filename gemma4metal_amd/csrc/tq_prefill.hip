@@ -678,6 +678,9 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 // were centred, which would add 128 instructions), two row sets a wave at one
 // wave per SIMD (97 us), operand reads half a tile ahead (68), the two waves of
 // a SIMD staging at opposite ends of a tile (69).
+//
+// One body under two names, by which the plan and traces tell D 512 from the
+// rest; no wave has a role of its own in either.
 template <int D, bool F32, int NS, int RS>
 __global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
 void prefill_int4_ws_kernel(SdpaParams p) {

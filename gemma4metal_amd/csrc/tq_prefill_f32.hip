@@ -276,7 +276,7 @@ __device__ __forceinline__ void pf_load(PfRaw<D, F32>& R, const SdpaParams& p, i
 template <int D, bool F32>
 __global__ __launch_bounds__(kPfThreads)
 __attribute__((amdgpu_waves_per_eu(D == 512 ? 1 : 2, D == 512 ? 1 : 2)))
-void prefill_int4_kernel(SdpaParams p) {
+void prefill_f32q_kernel(SdpaParams p) {
   pin_args(p);
   using Gm = PfGeom<D>;
   constexpr int W = Gm::W, KSTR = Gm::KSTR, VSTR = Gm::VSTR, CH = Gm::CH, DB = Gm::DB;
@@ -452,7 +452,7 @@ void prefill_int4_kernel(SdpaParams p) {
 // kernel above.
 template <int D, bool F32>
 __global__ __launch_bounds__(2 * kPfThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void prefill_int4_ws_kernel(SdpaParams p) {
+void prefill_f32q_ws_kernel(SdpaParams p) {
   pin_args(p);
   using Gm = PfGeom<D>;
   constexpr int W = Gm::W, KSTR = Gm::KSTR, VSTR = Gm::VSTR, CH = Gm::CH, DB = Gm::DB;
@@ -626,11 +626,11 @@ void prefill_int4_ws_kernel(SdpaParams p) {
 
 template <bool F32>
 void launch_tiles(const SdpaParams& p, int D, bool ws, dim3 grid, hipStream_t s) {
-  if (D == 128 && ws) prefill_int4_ws_kernel<128, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
-  else if (D == 256 && ws) prefill_int4_ws_kernel<256, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
-  else if (D == 128) prefill_int4_kernel<128, F32><<<grid, kPfThreads, 0, s>>>(p);
-  else if (D == 256) prefill_int4_kernel<256, F32><<<grid, kPfThreads, 0, s>>>(p);
-  else prefill_int4_kernel<512, F32><<<grid, kPfThreads, 0, s>>>(p);
+  if (D == 128 && ws) prefill_f32q_ws_kernel<128, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
+  else if (D == 256 && ws) prefill_f32q_ws_kernel<256, F32><<<grid, 2 * kPfThreads, 0, s>>>(p);
+  else if (D == 128) prefill_f32q_kernel<128, F32><<<grid, kPfThreads, 0, s>>>(p);
+  else if (D == 256) prefill_f32q_kernel<256, F32><<<grid, kPfThreads, 0, s>>>(p);
+  else prefill_f32q_kernel<512, F32><<<grid, kPfThreads, 0, s>>>(p);
 }
 
 }  // namespace
@@ -642,7 +642,7 @@ int launch_prefill_tiles_f32(const SdpaParams& p, int D, int sb_dtype, hipStream
   const bool ws = options().prefill_ws;
   if (sb_dtype == TQ_F32) launch_tiles<true>(p, D, ws, grid, s);
   else launch_tiles<false>(p, D, ws, grid, s);
-  TQ_CHECK_LAUNCH("prefill_int4_kernel (fp32 queries)");
+  TQ_CHECK_LAUNCH("prefill_f32q_kernel");
   return TQ_OK;
 }
 

@@ -233,7 +233,7 @@ SdpaPlan plan_sdpa(int mode, int batch, int Hq, int Hkv, int D, int max_len, int
 const char* kernel_name(const SdpaPlan& pl, int D, int sb_dtype) {
   (void)sb_dtype;
   switch (pl.kernel) {
-    case SdpaKernel::prefill_tiles:
+    case SdpaKernel::prefill_tiles:  // of 16-bit queries (fp32 ones: see tq_c_api.h)
       return D != 512 ? "prefill_int4_ws_kernel" : "prefill_int4_kernel";
     case SdpaKernel::hc:
       return options().hc_one ? "sdpa_int4_hc_kernel" : "sdpa_int4_hc2_kernel";

@@ -159,7 +159,8 @@ def sdpa_plan(num_heads: int, num_kv_heads: int, head_dim: int, max_kv_len: int,
               sb_dtype: torch.dtype = torch.float16, mode: str = "decode", batch: int = 1,
               sliding_window: int = 0) -> dict:
     """The kernel a call of this shape launches and its split plan
-    (``tq_sdpa_int4_plan``; no GPU work): ``{"kernel", "splits", "chunk"}``."""
+    (``tq_sdpa_int4_plan``; no GPU work): ``{"kernel", "splits", "chunk"}``.
+    For prefills it names the kernel of 16-bit queries (fp32 ones: tq_c_api.h)."""
     _need(sb_dtype in (torch.float16, torch.float32), "sb_dtype must be float16 or float32")
     splits, chunk = ctypes.c_int(0), ctypes.c_int(0)
     name = ctypes.create_string_buffer(64)

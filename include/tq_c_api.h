@@ -110,7 +110,11 @@ int tq_sdpa_int4_noalloc(const void* q, tq_dtype q_dtype,
  * tq_sdpa_int4 (max_kv_len = kv_len), 1 = tq_sdpa_int4_ragged, 2 =
  * tq_sdpa_int4_prefill (batch = n_new, max_kv_len = n_prior + n_new).
  * *splits = workgroups per sequence along the keys (grid x), *chunk_keys =
- * keys per split; the kernel's name is written to kernel[kernel_bytes].
+ * keys per split; the kernel's name is written to kernel[kernel_bytes].  The
+ * plan does not know the query dtype: "prefill_int4_ws_kernel" (D 128 / 256)
+ * and "prefill_int4_kernel" (D 512) are those of 16-bit queries, in whose
+ * place fp32 queries run "prefill_f32q_ws_kernel" ("prefill_f32q_kernel" with
+ * TQ_PREFILL_WS=0) and "prefill_f32q_kernel"; all else is the same for both.
  * The cache capacity is taken as max_kv_len: caches of fewer than 32 rows
  * run the VALU kernel (the matrix-core kernel reads 32-row blocks). */
 int tq_sdpa_int4_plan(int mode, int batch, int num_heads, int num_kv_heads, int head_dim,
@@ -120,8 +124,8 @@ int tq_sdpa_int4_plan(int mode, int batch, int num_heads, int num_kv_heads, int 
 /* Re-reads the kernel-choice switches from the environment (no counterpart
  * in the reference).  They are read once per process otherwise:
  * TQ_SDPA_IMPL=valu, TQ_SDPA_CHUNK=<keys>, TQ_PREFILL_IMPL=splitk,
- * TQ_PREFILL_WS=0 (fp32 queries), TQ_HC_IMPL=1.  For tests and measurement; calls that run
- * while it executes see the old or the new values. */
+ * TQ_PREFILL_WS=0 (fp32 queries), TQ_HC_IMPL=1.  For tests and measurement;
+ * calls that run while it executes see the old or the new values. */
 int tq_reload_options(void);
 int tq_sdpa_int4(const void* q, tq_dtype q_dtype,
                  const uint32_t* k_quant, const void* k_scales, const void* k_biases,
