@@ -56,7 +56,7 @@ constexpr float kPfLazy = 8.0f;
 // 2^(e0 - kPfDown) leave such a weight 21 bits above fp16's step.
 constexpr int kPfHead = 4, kPfUp = 3, kPfDown = 7;
 
-template <int D, bool F32, int NS, int RS>
+template <int D, bool F32, int RS>
 struct PfGeom {
   using SB = typename std::conditional<F32, float, _Float16>::type;
   static constexpr int W = D / 8;        // packed words per row
@@ -83,11 +83,11 @@ struct PfGeom {
     u32x4 k[2][2 * KH * KU];             // [16-key slice][g][s][c][key]: word 8 g + 2 c + s
     u32x4 v[2][KH * VU];                 // [kh][g][x][c][dim row]: slots 0-7 of lane group c
     SB sb[2][4][TK * NG];                // k scale, k bias, v scale, v bias
-    v4f xch[DH == 2 ? NW : 1][2 * NS][64];  // score parts of a row set's waves
+    v4f xch[DH == 2 ? NW : 1][2][64];    // score parts of a row set's waves
   };
   union Lds {
     Stage st;
-    float o[NW][16 * NS * OSTR];
+    float o[NW][16 * OSTR];
   };
   static_assert(SDW % 64 == 0 && UNITS % 64 == 0, "wave-uniform staging roles");
 };
@@ -253,15 +253,15 @@ __device__ __forceinline__ uint32_t pf_rem_pair(uint32_t hp, float x0, float x1)
   return r;
 }
 
-template <int D, bool F32, int NS, int RS>
+template <int D, bool F32, int RS>
 __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
-  using Gm = PfGeom<D, F32, NS, RS>;
+  using Gm = PfGeom<D, F32, RS>;
   using SB = typename Gm::SB;
   constexpr int NG = Gm::NG, NWG = Gm::NW_, TK = Gm::TK, KH = Gm::KH, DH = Gm::DH;
   __shared__ __attribute__((aligned(16))) typename Gm::Lds L;
   __shared__ uint32_t vmx;                  // bits of the first tile's largest |V scale|
   __shared__ int alike[2][Gm::NSW];         // a buffer's V scales are alike (all of them set)
-  __shared__ float ml[Gm::NW][16 * NS], ll[Gm::NW][16 * NS];
+  __shared__ float ml[Gm::NW][16], ll[Gm::NW][16];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -273,91 +273,86 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
   const int nblk = gridDim.x / p.Hkv;
   const int kvh = blockIdx.x % p.Hkv, blk = nblk - 1 - static_cast<int>(blockIdx.x / p.Hkv);
   const int total = p.nq * p.gqa;           // rows of this kv head
-  const int r0 = blk * 16 * NS * RS;        // first row of this workgroup
+  const int r0 = blk * 16 * RS;             // first row of this workgroup
   const int W_ = p.window;
   const int lo = W_ > 0 ? max(0, p.n + r0 / p.gqa + 1 - W_) : 0;
-  const int last = p.n + (min(r0 + 16 * NS * RS, total) - 1) / p.gqa;  // last key of the last row
+  const int last = p.n + (min(r0 + 16 * RS, total) - 1) / p.gqa;  // last key of the last row
   const int ntile = (last - lo) / TK + 1;
   const int64_t row0 = static_cast<int64_t>(kvh) * p.cap;
 
   PfRaw<Gm> raw;
   pf_load<Gm>(raw, p, row0, lo, last);
 
-  const int rw = r0 + 16 * NS * rs;         // the wave's first row
-  const int pos_lo = p.n + min(rw, total - 1) / p.gqa, pos_hi = p.n + min(rw + 16 * NS - 1, total - 1) / p.gqa;
-  int pos[NS];                              // absolute position of this lane's rows (column m of each set)
+  const int rw = r0 + 16 * rs;              // the wave's first row
+  const int pos_lo = p.n + min(rw, total - 1) / p.gqa, pos_hi = p.n + min(rw + 15, total - 1) / p.gqa;
+  const int R = min(rw + m, total - 1);     // this lane's row (column m)
+  const int qi = R / p.gqa;
+  const int pos = p.n + qi;                 // its absolute position
 
   // ---- q: B operands of k-step s of group g are dims 64 g + 16 c + 8 s + {0, 4,
   // 1, 5, 2, 6, 3, 7}, times 2^(15 - ex) (the row's largest below 2^15), the odd
   // ones over 16.  The sign of a negative scale goes into q.
-  v8h qf[NS][2 * NWG], qb[NS];
-  float rf[NS];                             // score = rf * products
+  v8h qf[2 * NWG], qb;
+  const int64_t qrow = static_cast<int64_t>(qi) * p.Hq + kvh * p.gqa + (R - qi * p.gqa);
+  float f[2 * NWG][8];
+  float mx = 0.0f;
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const int R = min(rw + 16 * n + m, total - 1);
-    const int qi = R / p.gqa;
-    pos[n] = p.n + qi;
-    const int64_t qrow = static_cast<int64_t>(qi) * p.Hq + kvh * p.gqa + (R - qi * p.gqa);
-    float f[2 * NWG][8];
-    float mx = 0.0f;
+  for (int j = 0; j < 2 * NWG; ++j) {
+    const int64_t e0 = qrow * D + Gm::OW * dh + 64 * (j >> 1) + 16 * c + 8 * (j & 1);
+    const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
+    const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-    for (int j = 0; j < 2 * NWG; ++j) {
-      const int64_t e0 = qrow * D + Gm::OW * dh + 64 * (j >> 1) + 16 * c + 8 * (j & 1);
-      const uint4 u = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p.q) + e0);
-      const uint32_t wd[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (p.q_dtype == TQ_F16) {
-          const v2h h = __builtin_bit_cast(v2h, wd[i]);
-          f[j][2 * i] = static_cast<float>(h[0]);
-          f[j][2 * i + 1] = static_cast<float>(h[1]);
-        } else {
-          f[j][2 * i] = __uint_as_float(wd[i] << 16);
-          f[j][2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(f[j][i]));
-    }
-    mx = xor32_max(xor16_max(mx));
-    const int ex = __builtin_amdgcn_frexp_expf(mx);
-    rf[n] = ldexpf(fabsf(p.scale_log2), ex - 15);
-    const bool neg = p.scale_log2 < 0.0f;
-    float qs[NWG];
-#pragma unroll
-    for (int g = 0; g < NWG; ++g) qs[g] = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 2 * NWG; ++j) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        float x = ldexpf(f[j][i], 15 - ex);
-        x = neg ? -x : x;
-        qs[j >> 1] += x;
-        const int slot = (i & 2) ? 4 + 2 * (i & 1) + (i >> 2) : 2 * (i & 1) + (i >> 2);
-        const float y = (i & 1) ? x * 0.0625f : x;
-        qf[n][j][slot] = static_cast<_Float16>(y);
+    for (int i = 0; i < 4; ++i) {
+      if (p.q_dtype == TQ_F16) {
+        const v2h h = __builtin_bit_cast(v2h, wd[i]);
+        f[j][2 * i] = static_cast<float>(h[0]);
+        f[j][2 * i + 1] = static_cast<float>(h[1]);
+      } else {
+        f[j][2 * i] = __uint_as_float(wd[i] << 16);
+        f[j][2 * i + 1] = __uint_as_float(wd[i] & 0xFFFF0000u);
       }
     }
-    // group sums over 512 (|.| < 2^12) in fp16 parts.  fp16 scale/bias: part c
-    // in lane group c (parts 0-2) for the biases, 8 times it for the scales;
-    // fp32: b' = high + low half, high half times parts 0, 1 in lane groups
-    // 0, 1 and low half in 2, 3.
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      _Float16 pt = static_cast<_Float16>(0.0f);
-      if (g < NWG) {
-        float x = xor32_sum(xor16_sum(qs[g < NWG ? g : 0])) * 0x1p-9f;
-        const _Float16 h0 = static_cast<_Float16>(x);
-        x -= static_cast<float>(h0);
-        const _Float16 h1 = static_cast<_Float16>(x);
-        x -= static_cast<float>(h1);
-        const _Float16 h2 = static_cast<_Float16>(x);
-        if constexpr (F32) pt = (c & 1) ? h1 : h0;
-        else pt = c == 0 ? h0 : c == 1 ? h1 : c == 2 ? h2 : pt;
-      }
-      qb[n][g] = pt;
-      qb[n][4 + g] = F32 ? static_cast<_Float16>(0.0f) : pt * static_cast<_Float16>(8.0f);
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(f[j][i]));
+  }
+  mx = xor32_max(xor16_max(mx));
+  const int ex = __builtin_amdgcn_frexp_expf(mx);
+  const float rf = ldexpf(fabsf(p.scale_log2), ex - 15);  // score = rf * products
+  const bool neg = p.scale_log2 < 0.0f;
+  float qs[NWG];
+#pragma unroll
+  for (int g = 0; g < NWG; ++g) qs[g] = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 2 * NWG; ++j) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float x = ldexpf(f[j][i], 15 - ex);
+      x = neg ? -x : x;
+      qs[j >> 1] += x;
+      const int slot = (i & 2) ? 4 + 2 * (i & 1) + (i >> 2) : 2 * (i & 1) + (i >> 2);
+      const float y = (i & 1) ? x * 0.0625f : x;
+      qf[j][slot] = static_cast<_Float16>(y);
     }
+  }
+  // group sums over 512 (|.| < 2^12) in fp16 parts.  fp16 scale/bias: part c
+  // in lane group c (parts 0-2) for the biases, 8 times it for the scales;
+  // fp32: b' = high + low half, high half times parts 0, 1 in lane groups
+  // 0, 1 and low half in 2, 3.
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    _Float16 pt = static_cast<_Float16>(0.0f);
+    if (g < NWG) {
+      float x = xor32_sum(xor16_sum(qs[g < NWG ? g : 0])) * 0x1p-9f;
+      const _Float16 h0 = static_cast<_Float16>(x);
+      x -= static_cast<float>(h0);
+      const _Float16 h1 = static_cast<_Float16>(x);
+      x -= static_cast<float>(h1);
+      const _Float16 h2 = static_cast<_Float16>(x);
+      if constexpr (F32) pt = (c & 1) ? h1 : h0;
+      else pt = c == 0 ? h0 : c == 1 ? h1 : c == 2 ? h2 : pt;
+    }
+    qb[g] = pt;
+    qb[4 + g] = F32 ? static_cast<_Float16>(0.0f) : pt * static_cast<_Float16>(8.0f);
   }
 
   if (threadIdx.x == 0) vmx = 0;
@@ -375,17 +370,12 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
   // far up to kPfLazy.  A reference that follows the largest V scale staged so far
   // leaves a row 28 - k bits once a key that it does not attend has 2^k times
   // the scales of those that it does.
-  float m_ref[NS], l_run[NS], bsum[NS][NWG];
-  v4f o[NS][4 * NWG];
+  float m_ref = -INFINITY, l_run = 0.0f, bsum[NWG];
+  v4f o[4 * NWG];
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    m_ref[n] = -INFINITY;
-    l_run[n] = 0.0f;
+  for (int b = 0; b < 4 * NWG; ++b) o[b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int b = 0; b < 4 * NWG; ++b) o[n][b] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int g = 0; g < NWG; ++g) bsum[n][g] = 0.0f;
-  }
+  for (int g = 0; g < NWG; ++g) bsum[g] = 0.0f;
   const v4f z = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 
 #pragma unroll 1
@@ -402,7 +392,7 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
     const SB* svs = L.st.sb[buf][2] + 32 * kh * NG + NWG * dh;
     const SB* svb = L.st.sb[buf][3] + 32 * kh * NG + NWG * dh;
 
-    float sc[NS][8];
+    float sc[8];
     if (any) {
       // ---- S^T: two 16-key halves ------------------------------------------
 #pragma unroll
@@ -425,98 +415,77 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
             }
           }
         }
-        v4f acc[NS][NWG], bt[NS];
-#pragma unroll
-        for (int n = 0; n < NS; ++n) bt[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qb[n], z, 0, 0, 0);
+        const v4f bt = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb, qb, z, 0, 0, 0);
+        v4f acc[NWG];
 #pragma unroll
         for (int g = 0; g < NWG; ++g) {
           const u32x4* kr = ku + h * Gm::KU + 128 * g + (m ^ Gm::kswz(NWG * dh + g));
           const v8h a0 = __builtin_bit_cast(v8h, kr[0]), a1 = __builtin_bit_cast(v8h, kr[64]);
-#pragma unroll
-          for (int n = 0; n < NS; ++n) {
-            v4f a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[n][2 * g], z, 0, 0, 0);
-            a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[n][2 * g + 1], a, 0, 0, 0);
-            acc[n][g] = a;
-          }
+          v4f a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, qf[2 * g], z, 0, 0, 0);
+          a = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, qf[2 * g + 1], a, 0, 0, 0);
+          acc[g] = a;
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+          float s = bt[i] * 512.0f;
 #pragma unroll
-          for (int n = 0; n < NS; ++n) {
-            float s = bt[n][i] * 512.0f;
-#pragma unroll
-            for (int g = 0; g < NWG; ++g)
-              s = fmaf(static_cast<float>(sks[(16 * h + 4 * c + i) * NG + g]), acc[n][g][i], s);
-            sc[n][4 * h + i] = s * rf[n];
-          }
+          for (int g = 0; g < NWG; ++g)
+            s = fmaf(static_cast<float>(sks[(16 * h + 4 * c + i) * NG + g]), acc[g][i], s);
+          sc[4 * h + i] = s * rf;
+        }
       }
     }
     if constexpr (DH == 2) {
       // the other wave's groups: its parts of the same scores
       if (any) {
 #pragma unroll
-        for (int n = 0; n < NS; ++n)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            L.st.xch[wave][2 * n + h][lane] = v4f{sc[n][4 * h], sc[n][4 * h + 1], sc[n][4 * h + 2], sc[n][4 * h + 3]};
+        for (int h = 0; h < 2; ++h)
+          L.st.xch[wave][h][lane] = v4f{sc[4 * h], sc[4 * h + 1], sc[4 * h + 2], sc[4 * h + 3]};
       }
       __syncthreads();
       if (any) {
 #pragma unroll
-        for (int n = 0; n < NS; ++n)
+        for (int h = 0; h < 2; ++h) {
+          const v4f x = L.st.xch[wave ^ RS][h][lane];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const v4f x = L.st.xch[wave ^ RS][2 * n + h][lane];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sc[n][4 * h + i] += x[i];
-          }
+          for (int i = 0; i < 4; ++i) sc[4 * h + i] += x[i];
+        }
       }
     }
     if (any) {
       const bool inside = t0 + 31 <= pos_lo && (W_ == 0 || pos_hi - t0 < W_);  // wave-uniform
       if (!inside) {
 #pragma unroll
-        for (int n = 0; n < NS; ++n)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            const int t = t0 + 16 * (j >> 2) + 4 * c + (j & 3);
-            sc[n][j] = t <= pos[n] && (W_ == 0 || pos[n] - t < W_) ? sc[n][j] : -INFINITY;
-          }
+        for (int j = 0; j < 8; ++j) {
+          const int t = t0 + 16 * (j >> 2) + 4 * c + (j & 3);
+          sc[j] = t <= pos && (W_ == 0 || pos - t < W_) ? sc[j] : -INFINITY;
+        }
       }
 
       // ---- online softmax (log2 domain) of rows m ------------------------------
       const float up = static_cast<float>(e0 - kPfHead);
-      float need[NS];
+      float mt = sc[0];
 #pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        float mt = sc[n][0];
-#pragma unroll
-        for (int j = 1; j < 8; ++j) mt = fmaxf(mt, sc[n][j]);
-        need[n] = xor32_max(xor16_max(mt)) + up;
-      }
+      for (int j = 1; j < 8; ++j) mt = fmaxf(mt, sc[j]);
+      const float need = xor32_max(xor16_max(mt)) + up;
       // (a row with nothing attended yet and nothing here keeps -inf)
+      if (__any(need > m_ref + kPfLazy)) {
+        const float m_new = need > m_ref ? need : m_ref;
+        const float f = m_new == m_ref ? 1.0f : merge_factor(m_ref, m_new);
+        l_run *= f;
 #pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        if (!__any(need[n] > m_ref[n] + kPfLazy)) continue;
-        const float m_new = need[n] > m_ref[n] ? need[n] : m_ref[n];
-        const float f = m_new == m_ref[n] ? 1.0f : merge_factor(m_ref[n], m_new);
-        l_run[n] *= f;
+        for (int b = 0; b < 4 * NWG; ++b) o[b] *= f;
 #pragma unroll
-        for (int b = 0; b < 4 * NWG; ++b) o[n][b] *= f;
-#pragma unroll
-        for (int g = 0; g < NWG; ++g) bsum[n][g] *= f;
-        m_ref[n] = m_new;
+        for (int g = 0; g < NWG; ++g) bsum[g] *= f;
+        m_ref = m_new;
       }
-      float pw[NS][8];
+      float pw[8];
+      // (with nothing attended so far, -inf - -inf would be NaN)
+      const float ms = m_ref == -INFINITY ? 0.0f : m_ref;
 #pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        // (with nothing attended so far, -inf - -inf would be NaN)
-        const float ms = m_ref[n] == -INFINITY ? 0.0f : m_ref[n];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          pw[n][j] = fast_exp2(sc[n][j] - ms);
-          l_run[n] += pw[n][j];
-        }
+      for (int j = 0; j < 8; ++j) {
+        pw[j] = fast_exp2(sc[j] - ms);
+        l_run += pw[j];
       }
 
       // ---- O^T += V^T P^T ----------------------------------------------------
@@ -531,11 +500,9 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
         bh = __builtin_bit_cast(v8h, hi);
         bl = __builtin_bit_cast(v8h, lw);
       };
-      float pz[NS][8];  // the weights of the common products
+      float pz[8];  // the weights of the common products
 #pragma unroll
-      for (int n = 0; n < NS; ++n)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pz[n][j] = pw[n][j];
+      for (int j = 0; j < 8; ++j) pz[j] = pw[j];
       int al = 1;
 #pragma unroll
       for (int i = 0; i < Gm::NSW; ++i) al &= alike[buf][i];
@@ -544,34 +511,31 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
         // (an infinity, of exponent 0, stays one), the products on their own, added
         // in fp32
 #pragma unroll
-        for (int n = 0; n < NS; ++n) {
+        for (int g = 0; g < NWG; ++g) {
+          float y[8], mx = 0.0f;
 #pragma unroll
-          for (int g = 0; g < NWG; ++g) {
-            float y[8], mx = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-              y[j] = static_cast<float>(svs[(16 * (j >> 2) + 4 * c + (j & 3)) * NG + g]) * pw[n][j];
-              mx = fmaxf(mx, fabsf(y[j]));
-            }
-            const int k = min(14 - __builtin_amdgcn_frexp_expf(xor32_max(xor16_max(mx))), 120);
-            const float un = ldexpf(1.0f, -k);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) y[j] = ldexpf(y[j], k);
-            v8h bh, bl;
-            split(y, bh, bl);
-#pragma unroll
-            for (int x = 0; x < 4; ++x) {
-              const v8h a = __builtin_bit_cast(v8h, vu[(4 * g + x) * 64 + (m ^ Gm::vswz(g))]);
-              v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, z, 0, 0, 0);
-              t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, t, 0, 0, 0);
-#pragma unroll
-              for (int i = 0; i < 4; ++i) o[n][4 * g + x][i] = fmaf(t[i], un, o[n][4 * g + x][i]);
-            }
+          for (int j = 0; j < 8; ++j) {
+            y[j] = static_cast<float>(svs[(16 * (j >> 2) + 4 * c + (j & 3)) * NG + g]) * pw[j];
+            mx = fmaxf(mx, fabsf(y[j]));
           }
-          // (nothing is left for the products below: a branch around them cost 50 registers)
+          const int k = min(14 - __builtin_amdgcn_frexp_expf(xor32_max(xor16_max(mx))), 120);
+          const float un = ldexpf(1.0f, -k);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) pz[n][j] = 0.0f;
+          for (int j = 0; j < 8; ++j) y[j] = ldexpf(y[j], k);
+          v8h bh, bl;
+          split(y, bh, bl);
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const v8h a = __builtin_bit_cast(v8h, vu[(4 * g + x) * 64 + (m ^ Gm::vswz(g))]);
+            v4f t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, z, 0, 0, 0);
+            t = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, t, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[4 * g + x][i] = fmaf(t[i], un, o[4 * g + x][i]);
+          }
         }
+        // (nothing is left for the products below: a branch around them cost 50 registers)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) pz[j] = 0.0f;
       }
       SB s[8][NWG], bb[8][NWG];
 #pragma unroll
@@ -585,27 +549,21 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
       }
 #pragma unroll
       for (int g = 0; g < NWG; ++g) {
-        v8h bh[NS], bl[NS];
+        v8h bh, bl;
+        float y[8];
 #pragma unroll
-        for (int n = 0; n < NS; ++n) {
-          float y[8];
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            y[j] = fmaf(static_cast<float>(s[j][g]), pz[n][j], 0.0f);
-            // b' = b + 8 s
-            bsum[n][g] = fmaf(fmaf(static_cast<float>(s[j][g]), 8.0f, static_cast<float>(bb[j][g])), pw[n][j], bsum[n][g]);
-          }
-          split(y, bh[n], bl[n]);
+        for (int j = 0; j < 8; ++j) {
+          y[j] = fmaf(static_cast<float>(s[j][g]), pz[j], 0.0f);
+          // b' = b + 8 s
+          bsum[g] = fmaf(fmaf(static_cast<float>(s[j][g]), 8.0f, static_cast<float>(bb[j][g])), pw[j], bsum[g]);
         }
+        split(y, bh, bl);
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
           const v8h a = __builtin_bit_cast(v8h, vu[(4 * g + x) * 64 + (m ^ Gm::vswz(g))]);
-#pragma unroll
-          for (int n = 0; n < NS; ++n) {
-            v4f& acc = o[n][4 * g + x];
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh[n], acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl[n], acc, 0, 0, 0);
-          }
+          v4f& acc = o[4 * g + x];
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bh, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bl, acc, 0, 0, 0);
         }
       }
     }
@@ -618,31 +576,28 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 
   // ---- merge of the KH partials of every row, and the output ------------------
   const float un = c < 2 ? 1.0f : 0.0625f;  // odd nibbles (rows 8-15) were 16 times as large
+  const float lt = xor32_sum(xor16_sum(l_run));
+  if (c == 0) {
+    ml[wave][m] = m_ref;
+    ll[wave][m] = lt;
+  }
+  float* orow = L.o[wave] + m * Gm::OSTR;
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const float lt = xor32_sum(xor16_sum(l_run[n]));
-    if (c == 0) {
-      ml[wave][16 * n + m] = m_ref[n];
-      ll[wave][16 * n + m] = lt;
-    }
-    float* orow = L.o[wave] + (16 * n + m) * Gm::OSTR;
+  for (int g = 0; g < NWG; ++g) {
+    const float bg = xor32_sum(xor16_sum(bsum[g]));
 #pragma unroll
-    for (int g = 0; g < NWG; ++g) {
-      const float bg = xor32_sum(xor16_sum(bsum[n][g]));
+    for (int x = 0; x < 4; ++x)
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          orow[64 * g + 8 * (4 * (c & 1) + i) + 2 * x + (c >> 1)] = fmaf(o[n][4 * g + x][i], un, bg);
-    }
+      for (int i = 0; i < 4; ++i)
+        orow[64 * g + 8 * (4 * (c & 1) + i) + 2 * x + (c >> 1)] = fmaf(o[4 * g + x][i], un, bg);
   }
   __syncthreads();
-  for (int u = threadIdx.x; u < 16 * NS * RS * (D / 2); u += Gm::NT) {
+  for (int u = threadIdx.x; u < 16 * RS * (D / 2); u += Gm::NT) {
     // a wave's 64 units lie in one row and in one wave's dims
     const int r = __builtin_amdgcn_readfirstlane(u / (D / 2)), d = 2 * (u % (D / 2));
     const int Ro = r0 + r;
     if (Ro >= total) break;
-    const int rm = r % (16 * NS), w0 = r / (16 * NS) + RS * KH * (d / Gm::OW);
+    const int rm = r % 16, w0 = r / 16 + RS * KH * (d / Gm::OW);
     float M = -INFINITY;
 #pragma unroll
     for (int k = 0; k < KH; ++k) M = fmaxf(M, ml[w0 + RS * k][rm]);
@@ -681,27 +636,25 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 //
 // One body under two names, by which the plan and traces tell D 512 from the
 // rest; no wave has a role of its own in either.
-template <int D, bool F32, int NS, int RS>
+template <int D, bool F32, int RS>
 __global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
 void prefill_int4_ws_kernel(SdpaParams p) {
   pin_args(p);
-  prefill_rows<D, F32, NS, RS>(p);
+  prefill_rows<D, F32, RS>(p);
 }
 
-template <int D, bool F32, int NS, int RS>
+template <int D, bool F32, int RS>
 __global__ __launch_bounds__(128 * RS) __attribute__((amdgpu_waves_per_eu(RS == 4 ? 2 : 1, RS == 4 ? 2 : 1)))
 void prefill_int4_kernel(SdpaParams p) {
   pin_args(p);
-  prefill_rows<D, F32, NS, RS>(p);
+  prefill_rows<D, F32, RS>(p);
 }
 
-template <int D, bool F32, int NS, int RS>
+template <int D, bool F32, int RS>
 void launch_sets(const SdpaParams& p, unsigned grid, hipStream_t s) {
-  if constexpr (D == 512) prefill_int4_kernel<D, F32, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
-  else prefill_int4_ws_kernel<D, F32, NS, RS><<<grid, 128 * RS, 0, s>>>(p);
+  if constexpr (D == 512) prefill_int4_kernel<D, F32, RS><<<grid, 128 * RS, 0, s>>>(p);
+  else prefill_int4_ws_kernel<D, F32, RS><<<grid, 128 * RS, 0, s>>>(p);
 }
-
-constexpr int kPfNS = 1;  // row sets a wave
 
 // 32 rows per workgroup of four waves while that gives every CU at most one
 // (twice the workgroups: 128 queries of Hq 32 Hkv 16 D 256 60 against 65 us, 100 of
@@ -709,11 +662,10 @@ constexpr int kPfNS = 1;  // row sets a wave
 // whole tile, 78 and 29), else 64.
 template <int D, bool F32>
 void launch_rows(const SdpaParams& p, hipStream_t s) {
-  constexpr int NR = 16 * kPfNS, RSM = 4 / kPfNS;
   const int64_t rows = static_cast<int64_t>(p.nq) * p.gqa;
-  const auto grid = [&](int rs) { return static_cast<unsigned>((rows + NR * rs - 1) / (NR * rs) * p.Hkv); };
-  if (grid(2) <= static_cast<unsigned>(target_wgs())) launch_sets<D, F32, kPfNS, 2>(p, grid(2), s);
-  else launch_sets<D, F32, kPfNS, RSM>(p, grid(RSM), s);
+  const auto grid = [&](int rs) { return static_cast<unsigned>((rows + 16 * rs - 1) / (16 * rs) * p.Hkv); };
+  if (grid(2) <= static_cast<unsigned>(target_wgs())) launch_sets<D, F32, 2>(p, grid(2), s);
+  else launch_sets<D, F32, 4>(p, grid(4), s);
 }
 
 template <bool F32>
