@@ -53,8 +53,12 @@ constexpr float kPfLazy = 8.0f;
 // With 2^e0 above every V scale of a workgroup's first tile: p s_v is below
 // 2^kPfHead for the row's largest weight and a scale of 2^e0, and below 2^15 (fp16
 // overflows at 2^16) for scales up to 2^(e0 + kPfUp).  Scales down to
-// 2^(e0 - kPfDown) leave such a weight 21 bits above fp16's step.
-constexpr int kPfHead = 4, kPfUp = 3, kPfDown = 7;
+// 2^(e0 - kPfDown) leave such a weight 19 bits above fp16's step (3 more than bf16
+// parts would).  A tile outside these bounds costs half as much again: with every
+// tile so (one group of 64 dims at 2^-12), 512 queries after 3,584 keys, 85
+// instead of 63 us (Hq 32 Hkv 16 D 256, window 1,024) and 578 instead of 387
+// (Hq 32 Hkv 4 D 512).
+constexpr int kPfHead = 4, kPfUp = 3, kPfDown = 9;
 
 template <int D, bool F32, int RS>
 struct PfGeom {
