@@ -231,6 +231,35 @@ def test_compressed_sdpa_infinite_last_value(pq, D):
     assert_close(got, ref, f"D{D}")
 
 
+def float_aligned(a):
+    """A contiguous device copy whose address is 4 past a multiple of 16."""
+    t = torch.empty(a.size + 1, dtype=torch.float32, device="cuda")[1:].view(a.shape)
+    t.copy_(dev(a))
+    assert t.data_ptr() % 16 == 4
+    return t
+
+
+@pytest.mark.parametrize("D", [48, 64, 128, 256])
+def test_inputs_at_float_alignment(pq, D):
+    """Vectors, matrices, queries and values need the alignment of a float
+    only: the same bits as at aligned addresses."""
+    rng = np.random.default_rng(D + 5)
+    n = 300
+    cbs = [dev(c) for c in rand_codebooks(rng, packed=True)]
+    x, P, v = rng.standard_normal((n, D)).astype(f32), ortho(rng, D), rng.standard_normal((n, D)).astype(f32)
+    q = rng.standard_normal((2, D)).astype(f32)
+    got = [[host(t) for t in pq.polar_quantize_packed(at(x), at(P), *cbs)] for at in (dev, float_aligned)]
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
+    if D != 48:
+        idx = pq.polar_quantize(dev(x), None, *cbs)
+        got = [host(pq.compressed_sdpa(at(q), *idx, *cbs, at(v), scale=0.2, num_kv_heads=1)) for at in (dev, float_aligned)]
+        assert np.array_equal(*got)
+    if D == 128:
+        S = rng.standard_normal((128, 128)).astype(f32)
+        got = [[host(t) for t in pq.Polar7Codec(at(P), at(S)).encode(at(x))] for at in (dev, float_aligned)]
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
 # --------------------------------------------------------------- polar7 --------
 
 def p7_inputs(seed, n, rot=True):

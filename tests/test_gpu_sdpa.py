@@ -578,6 +578,26 @@ def test_sdpa_prefill_rows_edges(gpu, Hq, Hkv, D, S, prior, W, scale, qmag, vmag
     assert rel < 2e-5, rel
 
 
+@pytest.mark.parametrize("D", [128, 256, 512])
+@pytest.mark.parametrize("sb", ["f16", "f32"])
+def test_sdpa_prefill_scales_and_out_at_element_alignment(gpu, D, sb):
+    """Scales, biases and the output need the alignment of one element only
+    (the tile kernel reads fp16 scales in pairs): the same bits."""
+    rng = np.random.default_rng(D)
+    Hq, Hkv, S, prior = 4, 2, 70, 37
+    qd, _ = queries(rng, (S, Hq, D), "bf16")
+    c = [dev(a) for a in host_cache(rng, Hkv, prior + S, D, sb)]
+
+    def odd(t):
+        u = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:].view(t.shape)
+        return u.copy_(t)
+
+    want = gpu.sdpa_int4_prefill(qd, *c, prior, Hq // Hkv, 1.0, 50)
+    out = odd(torch.zeros_like(want))
+    got = gpu.sdpa_int4_prefill(qd, *[t if j % 3 == 0 else odd(t) for j, t in enumerate(c)], prior, Hq // Hkv, 1.0, 50, out=out)
+    assert np.array_equal(host(got), host(want))
+
+
 def prefill_terms(q, c, prior, gqa, W):
     """The sum of the magnitudes of every result's terms: attention over |V|
     (scale 1), float64."""
@@ -609,6 +629,7 @@ def spread_v(rng, Hkv, n, D, low, spread, at):
     (8, 4, 256, 96, 200, 64, 0, 18, 180),       # outside the window of the later rows
     (8, 4, 256, 96, 200, 0, 6, -14, 250),       # far smaller than the rest
     (8, 8, 128, 100, 30, 0, 0, 12, 130 + 60),   # group 0 of one key only
+    (8, 8, 128, 100, 30, 0, 8, 2, 40),          # the edges of what still counts as alike
     (8, 8, 128, 100, 30, 0, 0, 20, 0),          # the first key, attended by all with any weight
     (16, 2, 512, 80, 50, 0, 0, 18, 129),
     (16, 2, 512, 80, 50, 40, 10, 16, 70),
