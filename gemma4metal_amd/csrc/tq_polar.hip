@@ -18,7 +18,8 @@
 // operations (correctly rounded division and square root, FMA contraction
 // off), so every index decision and sketch bit is reproducible.
 //
-// Scores and attention run one key per lane.  The polar7 score uses two
+// Scores and attention of the 16-value blocks give a key D / 16 lanes, a block
+// each; those of polar7 run one key per lane.  The polar7 score uses two
 // per-head LDS tables built in the workgroup prologue: the q'-premultiplied
 // level-1 table t1[j][k] = q'[2j] cos c_k + q'[2j+1] sin c_k (a level-1 angle
 // costs one gather instead of a cos/sin pair and 2 FMAs per head), and the
@@ -149,11 +150,11 @@ constexpr int64_t kEnc16Small = 1 << 20;
 // reads covers every bank once.
 constexpr int kEncColStr = 64 + 4;  // 64 columns of a matrix
 
+typedef float vf4 __attribute__((ext_vector_type(4)));  // (arrays of HIP's float4 stayed in scratch)
+
 // Rows r0 .. r0 + ROWS - 1, columns c0 .. c0 + 63 of a matrix with rows of DIM
 // floats (the 16-byte global loads here need the 4-byte alignment of a float
 // only): into registers, ROWS / 32 float4 a thread, and from there into LDS.
-typedef float vf4 __attribute__((ext_vector_type(4)));  // (arrays of HIP's float4 stayed in scratch)
-
 template <int ROWS, int DIM>
 __device__ __forceinline__ void load_cols(const float* m, int r0, int c0, vf4 (&r)[ROWS / 32]) {
 #pragma unroll
@@ -2092,7 +2093,7 @@ using namespace tq;
 
 namespace {
 
-// 512 blocks per workgroup, or 16 vectors for small inputs (more workgroups).
+// 512 blocks per workgroup, or 16 (D 64: 32) vectors for small inputs (more workgroups).
 template <int D, int V, int TV, int TI, bool kPacked>
 int launch_encode16_tile(const Enc16Params& p, hipStream_t s, const char* fn) {
   const int64_t grid = (p.n + V - 1) / V;

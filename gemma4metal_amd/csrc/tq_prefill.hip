@@ -625,14 +625,16 @@ __device__ __forceinline__ void prefill_rows(const SdpaParams& p) {
 // of 32 keys and two waves a row set, one per half of the dims (D 512; a tile's
 // two buffers fill the LDS): eight waves, two per SIMD.
 //
-// What bounds it: the VALU (about 430 instructions a wave and 32 keys -- weights
+// What bounds it: the VALU (about 420 instructions a wave and 32 keys -- weights
 // times scales and their split 80, exponentials and masks 90, staging 80, bias
 // terms 64, score scales 40 -- against 50 products), busy 60% of the time, the
 // rest being phases of the two waves that do not overlap.  Measured (512 queries
-// after 3,584 keys, whole calls; before: loader waves that dequantized every
-// tile into hi / lo images, whose LDS reads, three products each, bound it):
-//   Hq 32 Hkv 16 D 256, window 1,024: 94.9 -> 67.9 us; without window 275 -> 193
-//   Hq 32 Hkv 4 D 512: 678 -> 404 us;  Hq 16 Hkv 8 D 128: 148 -> 117 us
+// after 3,584 keys; before: loader waves that dequantized every tile into hi / lo
+// images, whose LDS reads, three products each, bound it):
+//   Hq 32 Hkv 16 D 256, window 1,024: 94.9 -> 61 us; without window 275 -> 183
+//   Hq 32 Hkv 4 D 512: 678 -> 386 us;  Hq 16 Hkv 8 D 128: 148 -> 110 us
+// A power of two per row and group for every tile, with a check and a branch per
+// group, in place of the two kinds of tile: 77 us, 229, 464, 122.
 // Slower: nibbles expanded by every wave (no operand images; 70 us before they
 // were centred, which would add 128 instructions), two row sets a wave at one
 // wave per SIMD (97 us), operand reads half a tile ahead (68), the two waves of
